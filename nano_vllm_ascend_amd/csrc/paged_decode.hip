@@ -3,9 +3,10 @@
 //
 // Work decomposition (split-KV, one kernel):
 //   a workgroup of NW waves owns one (sequence b, kv head g, partition p) of
-//   PART = NW * CPW * 64 consecutive context tokens, for all GQA query heads
+//   PART = NW * 64 consecutive context tokens, for all GQA query heads
 //   that read kv head g, so every K/V byte is read from HBM once.  Each wave
-//   owns CPW chunks of 64 tokens.  The grid is 1-D over the items in b, g, p
+//   owns 64 tokens.  Groups of 1 or 2 query heads run on v_dot2 (this kernel), larger ones on
+//   MFMA (the variant below).  The grid is 1-D over the items in b, g, p
 //   order with p fastest, counted over the partitions that exist for the
 //   device-side context lengths: a unit's partitions run side by side, so its
 //   merge overlaps other units' loads, and the slack a loose context bound adds
@@ -57,6 +58,8 @@ constexpr int kPartFloats = 132;  // max, sum, 128 accumulators, 2 pad (16-byte 
 // results where another call expects a zero counter.
 constexpr int kCounterSlots = 16384;
 constexpr size_t kCounterBytes = kCounterSlots * sizeof(int);
+constexpr int kMaxGroups = 4096;  // workgroups of an MFMA launch; each takes every kMaxGroups-th item
+constexpr int kMaxContext = 131072;  // largest context bound of a call
 constexpr int kMinPart = 256;  // smallest partition of a split launch (sizes the workspace)
 
 struct DecodeArgs {
@@ -76,6 +79,7 @@ struct DecodeArgs {
   int num_kv_heads;
   int bs_log2;
   int max_parts;
+  int max_items;  // batch * kv heads * max_parts (MFMA variant)
   int max_ctx;
   int batch;
   float scale_log2e;
@@ -83,6 +87,7 @@ struct DecodeArgs {
   // a whole group (q_group == GQA, q_head0 == 0) unless the ratio needs several launches.
   int q_group;
   int q_head0;
+  int q_sub;  // heads of each group in this launch (MFMA variant)
   // Fused decode step only: q holds the raw projection rows; the kernel applies the per-head
   // RMSNorm and RoPE to q and to the new token's k, and stores that k and the raw v at slots[b].
   const u16 *k_new;
@@ -154,15 +159,14 @@ __device__ __forceinline__ void load_block(__amdgpu_buffer_rsrc_t rsrc, int byte
   }
 }
 
-// GQA 1, and GQA 2 with one chunk per wave, fit 128 VGPRs without spills: four waves
-// per SIMD.
-template <int GQA, int NW, int CPW, int TILES, bool WHOLE, bool FUSED>
+// GQA 1 and 2 fit 128 VGPRs without spills: four waves per SIMD.
+template <int GQA, int NW, bool WHOLE, bool FUSED>
 __global__ void __launch_bounds__(NW * 64)
-__attribute__((amdgpu_waves_per_eu((GQA == 1 || (GQA == 2 && CPW == 1)) ? 4 : 1)))
+__attribute__((amdgpu_waves_per_eu(4)))
 paged_decode_kernel(DecodeArgs a) {
   constexpr int D = kHeadDim;
-  constexpr int CT = 16 * TILES;  // tokens per chunk: TILES tiles of 16 rows
-  constexpr int WT = CPW * CT;    // tokens per wave
+  constexpr int TILES = 4;        // tiles of 16 rows per wave
+  constexpr int WT = 16 * TILES;  // tokens per wave
   constexpr int PART = NW * WT;
 
   const int hkv = a.num_kv_heads;
@@ -346,126 +350,120 @@ paged_decode_kernel(DecodeArgs a) {
       }
       __builtin_amdgcn_s_waitcnt(0);  // vmcnt counts stores on gfx9: they are acknowledged
     }
-    if constexpr (CPW > 1) {  // several chunks per wave: normalise once, before the loop
-      if (t_begin < t_end) norm_queries();
-    }
   }
 
   if (t_begin < t_end) {
     const int last_tile = (t_end - 1) & ~15;
-#pragma unroll 1
-    for (int tc = t_begin; tc < t_end; tc += CT) {
-      KVTile T[TILES];
-      // the chunk's block-table entries first, so their scalar loads share one wait
-      int blk_t[TILES];
+    KVTile T[TILES];
+    // the chunk's block-table entries first, so their scalar loads share one wait
+    int blk_t[TILES];
 #pragma unroll
-      for (int i = 0; i < TILES; ++i)
-        blk_t[i] = (FUSED && CPW == 1) ? first_blk[i] : bt_row[min(tc + 16 * i, last_tile) >> a.bs_log2];
+    for (int i = 0; i < TILES; ++i)
+      blk_t[i] = FUSED ? first_blk[i] : bt_row[min(t_begin + 16 * i, last_tile) >> a.bs_log2];
 #pragma unroll
-      for (int i = 0; i < TILES; ++i) {
-        const int t0 = min(tc + 16 * i, last_tile);
-        int blk = blk_t[i];
-        if ((unsigned)blk >= (unsigned)a.num_blocks) err_bits |= NVAMD_ERR_BLOCK;
-        blk = min(max(blk, 0), a.num_blocks - 1);               // never leave the pool
-        const int64_t slot = ((int64_t)blk << a.bs_log2) + (t0 & bs_mask) + r;
-        const int64_t off = slot * row_elems + (int64_t)g * D + 8 * c;
-        const u16 *kp = a.k_cache + off;
-        const u16 *vp = a.v_cache + off;
-        // K/V are read once per step.  Bandwidth-bound (split) launches use nontemporal loads,
-        // which keep them from displacing other lines in the L2 (1.08x faster over a
-        // 32 x U[256, 2304] step); latency-bound whole-unit launches use plain loads, whose
-        // round trip is shorter (1.16x faster over a 4 x U[1, 512] step).
-        auto ld = [](const u16 *ptr) { return WHOLE ? ld16(ptr) : ld16_stream(ptr); };
-        T[i].ka0 = ld(kp);
-        T[i].ka1 = ld(kp + 64);
-        T[i].kb0 = ld(kp + step8);
-        T[i].kb1 = ld(kp + step8 + 64);
-        T[i].va0 = ld(vp);
-        T[i].va1 = ld(vp + 64);
-        T[i].vb0 = ld(vp + step8);
-        T[i].vb1 = ld(vp + step8 + 64);
-      }
-      if constexpr (FUSED && CPW == 1) norm_queries();  // the wave's only chunk
-      // QK for the chunk: s[tile][row a/b][head]
-      float s[TILES][2][GQA];
+    for (int i = 0; i < TILES; ++i) {
+      const int t0 = min(t_begin + 16 * i, last_tile);
+      int blk = blk_t[i];
+      if ((unsigned)blk >= (unsigned)a.num_blocks) err_bits |= NVAMD_ERR_BLOCK;
+      blk = min(max(blk, 0), a.num_blocks - 1);               // never leave the pool
+      const int64_t slot = ((int64_t)blk << a.bs_log2) + (t0 & bs_mask) + r;
+      const int64_t off = slot * row_elems + (int64_t)g * D + 8 * c;
+      const u16 *kp = a.k_cache + off;
+      const u16 *vp = a.v_cache + off;
+      // K/V are read once per step.  Bandwidth-bound (split) launches use nontemporal loads,
+      // which keep them from displacing other lines in the L2 (1.08x faster over a
+      // 32 x U[256, 2304] step); latency-bound whole-unit launches use plain loads, whose
+      // round trip is shorter (1.16x faster over a 4 x U[1, 512] step).
+      auto ld = [](const u16 *ptr) { return WHOLE ? ld16(ptr) : ld16_stream(ptr); };
+      T[i].ka0 = ld(kp);
+      T[i].ka1 = ld(kp + 64);
+      T[i].kb0 = ld(kp + step8);
+      T[i].kb1 = ld(kp + step8 + 64);
+      T[i].va0 = ld(vp);
+      T[i].va1 = ld(vp + 64);
+      T[i].vb0 = ld(vp + step8);
+      T[i].vb1 = ld(vp + step8 + 64);
+    }
+    if constexpr (FUSED) norm_queries();
+    // QK for the chunk: s[tile][row a/b][head]
+    float s[TILES][2][GQA];
 #pragma unroll
-      for (int i = 0; i < TILES; ++i) {
-#pragma unroll
-        for (int j = 0; j < GQA; ++j) {
-          float sa = 0.f, sb = 0.f;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            sa = dot2_bf16(qr[j][0][e], T[i].ka0[e], sa);
-            sb = dot2_bf16(qr[j][0][e], T[i].kb0[e], sb);
-          }
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            sa = dot2_bf16(qr[j][1][e], T[i].ka1[e], sa);
-            sb = dot2_bf16(qr[j][1][e], T[i].kb1[e], sb);
-          }
-          s[i][0][j] = sa;
-          s[i][1][j] = sb;
-        }
-      }
-      bool ok[TILES][2];
-#pragma unroll
-      for (int i = 0; i < TILES; ++i) {
-        ok[i][0] = (tc + 16 * i + r) < t_end;
-        ok[i][1] = (tc + 16 * i + 8 + r) < t_end;
-#pragma unroll
-        for (int j = 0; j < GQA; ++j) {
-          const float sa = sum8(s[i][0][j]) * a.scale_log2e;
-          const float sb = sum8(s[i][1][j]) * a.scale_log2e;
-          s[i][0][j] = ok[i][0] ? sa : -INFINITY;
-          s[i][1][j] = ok[i][1] ? sb : -INFINITY;
-        }
-      }
-
-      // Online softmax, one step per chunk, per 8-lane row group.
-      u32 pp[TILES][GQA];
+    for (int i = 0; i < TILES; ++i) {
 #pragma unroll
       for (int j = 0; j < GQA; ++j) {
-        float cm = m[j];
-#pragma unroll
-        for (int i = 0; i < TILES; ++i) cm = fmaxf(cm, fmaxf(s[i][0][j], s[i][1][j]));
-        const float ref = cm == -INFINITY ? 0.f : cm;  // a group with no valid row yet
-        const float alpha = fast_exp2(m[j] - ref);
-        m[j] = cm;
-        float add = 0.f;
-#pragma unroll
-        for (int i = 0; i < TILES; ++i) {
-          pp[i][j] = pack_bf16x2(fast_exp2(s[i][0][j] - ref), fast_exp2(s[i][1][j] - ref));
-          add += bf16_lo(pp[i][j]) + bf16_hi(pp[i][j]);
-        }
-        l[j] = l[j] * alpha + add;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) o[j][e] *= alpha;
-      }
-
-      // Rows past the context may hold stale bits (NaN * 0 = NaN): zero their V.
-      if (tc + CT > t_end) {
-        const u32x4 z = {0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int i = 0; i < TILES; ++i) {
-          if (!ok[i][0]) { T[i].va0 = z; T[i].va1 = z; }
-          if (!ok[i][1]) { T[i].vb0 = z; T[i].vb1 = z; }
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < TILES; ++i) {
+        float sa = 0.f, sb = 0.f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const u32 lo0 = pair_lo(T[i].va0[e], T[i].vb0[e]);
-          const u32 hi0 = pair_hi(T[i].va0[e], T[i].vb0[e]);
-          const u32 lo1 = pair_lo(T[i].va1[e], T[i].vb1[e]);
-          const u32 hi1 = pair_hi(T[i].va1[e], T[i].vb1[e]);
+          sa = dot2_bf16(qr[j][0][e], T[i].ka0[e], sa);
+          sb = dot2_bf16(qr[j][0][e], T[i].kb0[e], sb);
+        }
 #pragma unroll
-          for (int j = 0; j < GQA; ++j) {
-            o[j][2 * e] = dot2_bf16(pp[i][j], lo0, o[j][2 * e]);
-            o[j][2 * e + 1] = dot2_bf16(pp[i][j], hi0, o[j][2 * e + 1]);
-            o[j][8 + 2 * e] = dot2_bf16(pp[i][j], lo1, o[j][8 + 2 * e]);
-            o[j][8 + 2 * e + 1] = dot2_bf16(pp[i][j], hi1, o[j][8 + 2 * e + 1]);
-          }
+        for (int e = 0; e < 4; ++e) {
+          sa = dot2_bf16(qr[j][1][e], T[i].ka1[e], sa);
+          sb = dot2_bf16(qr[j][1][e], T[i].kb1[e], sb);
+        }
+        s[i][0][j] = sa;
+        s[i][1][j] = sb;
+      }
+    }
+    bool ok[TILES][2];
+#pragma unroll
+    for (int i = 0; i < TILES; ++i) {
+      ok[i][0] = (t_begin + 16 * i + r) < t_end;
+      ok[i][1] = (t_begin + 16 * i + 8 + r) < t_end;
+#pragma unroll
+      for (int j = 0; j < GQA; ++j) {
+        const float sa = sum8(s[i][0][j]) * a.scale_log2e;
+        const float sb = sum8(s[i][1][j]) * a.scale_log2e;
+        s[i][0][j] = ok[i][0] ? sa : -INFINITY;
+        s[i][1][j] = ok[i][1] ? sb : -INFINITY;
+      }
+    }
+
+    // Online softmax, one step per chunk, per 8-lane row group.
+    u32 pp[TILES][GQA];
+#pragma unroll
+    for (int j = 0; j < GQA; ++j) {
+      float cm = m[j];
+#pragma unroll
+      for (int i = 0; i < TILES; ++i) cm = fmaxf(cm, fmaxf(s[i][0][j], s[i][1][j]));
+      const float ref = cm == -INFINITY ? 0.f : cm;  // a group with no valid row yet
+      const float alpha = fast_exp2(m[j] - ref);
+      m[j] = cm;
+      float add = 0.f;
+#pragma unroll
+      for (int i = 0; i < TILES; ++i) {
+        pp[i][j] = pack_bf16x2(fast_exp2(s[i][0][j] - ref), fast_exp2(s[i][1][j] - ref));
+        add += bf16_lo(pp[i][j]) + bf16_hi(pp[i][j]);
+      }
+      l[j] = l[j] * alpha + add;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) o[j][e] *= alpha;
+    }
+
+    // Rows past the context may hold stale bits (NaN * 0 = NaN): zero their V.
+    if (t_begin + WT > t_end) {
+      const u32x4 z = {0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int i = 0; i < TILES; ++i) {
+        if (!ok[i][0]) { T[i].va0 = z; T[i].va1 = z; }
+        if (!ok[i][1]) { T[i].vb0 = z; T[i].vb1 = z; }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < TILES; ++i) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const u32 lo0 = pair_lo(T[i].va0[e], T[i].vb0[e]);
+        const u32 hi0 = pair_hi(T[i].va0[e], T[i].vb0[e]);
+        const u32 lo1 = pair_lo(T[i].va1[e], T[i].vb1[e]);
+        const u32 hi1 = pair_hi(T[i].va1[e], T[i].vb1[e]);
+#pragma unroll
+        for (int j = 0; j < GQA; ++j) {
+          o[j][2 * e] = dot2_bf16(pp[i][j], lo0, o[j][2 * e]);
+          o[j][2 * e + 1] = dot2_bf16(pp[i][j], hi0, o[j][2 * e + 1]);
+          o[j][8 + 2 * e] = dot2_bf16(pp[i][j], lo1, o[j][8 + 2 * e]);
+          o[j][8 + 2 * e + 1] = dot2_bf16(pp[i][j], hi1, o[j][8 + 2 * e + 1]);
         }
       }
     }
@@ -644,16 +642,580 @@ paged_decode_kernel(DecodeArgs a) {
   }
 }
 
-template <int GQA, int NW, int CPW, int TILES = 4, bool WHOLE = false, bool FUSED = false>
+template <int GQA, int NW, bool WHOLE, bool FUSED>
 int launch(DecodeArgs a, int batch, hipStream_t stream) {
-  constexpr int PART = NW * CPW * 16 * TILES;
+  constexpr int PART = NW * 64;
   a.max_parts = ceil_div(a.max_ctx, PART);
   if (a.max_parts > 64) return NVAMD_EUNSUPPORTED;  // merge stage holds <= 64 partitions
   if (WHOLE && a.max_parts != 1) return NVAMD_EINVAL;
   a.batch = batch;
   // One workgroup per possible (b, g, p); the ones past the last existing item exit at once.
   dim3 grid((unsigned)((int64_t)batch * a.num_kv_heads * a.max_parts));
-  hipLaunchKernelGGL((paged_decode_kernel<GQA, NW, CPW, TILES, WHOLE, FUSED>), grid, dim3(NW * 64), 0, stream, a);
+  hipLaunchKernelGGL((paged_decode_kernel<GQA, NW, WHOLE, FUSED>), grid, dim3(NW * 64), 0, stream, a);
+  return launch_status();
+}
+
+// ------------------------------------------------------------------------------------------
+// MFMA variant, for groups of 3 to 16 query heads.
+//
+// The same split-KV items, scan, records and arrival counting as above, for up to GP query heads of
+// a kv head in one launch, so K and V are read once whatever the ratio.  A wave's 64 tokens:
+//   S^T = K . Q^T by v_mfma_f32_16x16x32_bf16 with A = rows of K as read from the cache.  The operand's
+//        16 rows x 32 dims give a load only 64 consecutive bytes of a cache row, and K read that way
+//        took 1.07-1.15x the launch's time.  So 8 row slots take dims 0..31 of a 64-dim half and the other 8 (z = 1)
+//        dims 32..63 of the same 8 tokens: a load covers 128 bytes of 8 rows.  The columns hold up to
+//        8 heads' matching dims twice over (column (z, h): dims 32z.. of head h); of the
+//        accumulators only the slots and columns of equal z count, and a token's score is the sum of
+//        its two: one v_permlane32_swap and one DPP add per accumulator register gather both parts
+//        of token 4gq + i of a 16-token tile in lane (h, z = 0, gq);
+//   O^T[128 dims x 16 heads] += V^T . P^T: lane n + 16 gq reads dims 8n .. 8n+7 of tokens 4gq + t of
+//        two 16-token tiles (t = 0..3 each), whole 256-byte rows per load instruction, and pairs the
+//        tokens per dim with v_perm: product e takes dims 8c + e as its 16 rows.  P^T needs no lane
+//        movement: its k-slots are taken in the order the S^T accumulators hold the tokens.
+// Tiles and rows past the wave's range lie past the tile's buffer range: they read zeros without a
+// memory access.  Bound by the K/V stream, as the kernel above: a group of 8 over 16 x U[512, 4096] takes 28.8 us
+// (4.4 TB/s) where two launches over 4 heads took 63.5 us, and 100 x U[2048, 4096] 232 us (5.3 TB/s) against
+// 458; what is left over the dot-product kernel's 5.8 TB/s at 2 heads is the records' traffic.
+__device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8v, a), __builtin_bit_cast(bf16x8v, b), c, 0,
+                                                 0, 0);
+}
+// v of lanes l and l ^ 16 combined in every lane: v_permlane16_swap of a register with itself
+// leaves rows (0, 0, 2, 2) and (1, 1, 3, 3) of 16 lanes in its two results.
+__device__ __forceinline__ float sum_xor16(float v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float max_xor16(float v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+// Maximum and sum over each half-wave of 32 lanes.
+__device__ __forceinline__ float half_max(float v) {
+  v = fmaxf(v, dpp<kDppQuadXor1>(v));
+  v = fmaxf(v, dpp<kDppQuadXor2>(v));
+  v = fmaxf(v, dpp<kDppHalfMirror>(v));
+  v = fmaxf(v, dpp<kDppMirror>(v));
+  return max_xor16(v);
+}
+__device__ __forceinline__ float half_sum(float v) { return sum_xor16(sum16(v)); }
+
+constexpr int kCachePolicyStream = 2;  // nt
+template <int GP, int NW, bool WHOLE, bool FUSED, bool MANY>
+__device__ __forceinline__ bool mfma_item(const DecodeArgs &a, const int tid, const int item, float (&s_o)[NW][GP * kPartFloats],
+                                          float (&s_m)[NW][GP], float (&s_l)[NW][GP], int &s_last) {
+  constexpr int D = kHeadDim;
+  constexpr int PART = NW * 64;
+  constexpr int HS = kPartFloats;   // floats per head in LDS (4 of padding: rows spread over the banks)
+  const int hkv = a.num_kv_heads;
+  const int G = a.q_sub;
+  const int lane = tid & 63;
+
+  // Nothing writes these during the launch: read through the constant address space they stay
+  // scalar loads behind the stores of an earlier item.
+  typedef const __attribute__((address_space(4))) int32_t const_i32;
+  typedef const __attribute__((address_space(4))) int64_t const_i64;
+  const_i32 *lens = (const_i32 *)a.context_lens;
+  const_i64 *pos = (const_i64 *)a.positions;
+  const int ctx_cap = min(a.max_ctx, a.bt_width << a.bs_log2);
+  int b = -1, n_parts = 0, first = 0, ctx = 0;
+  int64_t nr = -1;
+  u32 err_bits = 0;
+  if constexpr (WHOLE) {
+    b = item / hkv;
+    n_parts = 1;
+    first = b;
+    const int raw = lens[b];
+    if (raw < 0 || raw > ctx_cap) err_bits |= NVAMD_ERR_CONTEXT;
+    ctx = max(min(raw, ctx_cap), 0);
+    if constexpr (FUSED) nr = pos[b];
+  } else {
+    for (int b0 = 0, base = 0; b0 < a.batch; b0 += 64) {
+      const int bi = b0 + lane;
+      int ci = 0, np = 0;
+      int64_t pi = 0;
+      bool bad = false;
+      if (bi < a.batch) {
+        const int raw = a.context_lens[bi];
+        bad = raw < 0 || raw > ctx_cap;
+        ci = max(min(raw, ctx_cap), 0);
+        np = max(ceil_div(ci, PART), 1);
+        if constexpr (FUSED) pi = a.positions[bi];
+      }
+      if (__ballot(bad)) err_bits |= NVAMD_ERR_CONTEXT;
+      const int incl = wave_incl_scan(np, lane);
+      const int total = __builtin_amdgcn_readlane(incl, 63);
+      if (item < (base + total) * hkv) {
+        const uint64_t past = __ballot((base + incl) * hkv > item);
+        const int sel = __ffsll((unsigned long long)past) - 1;
+        b = b0 + sel;
+        n_parts = __builtin_amdgcn_readlane(np, sel);
+        first = base + __builtin_amdgcn_readlane(incl, sel) - n_parts;
+        ctx = __builtin_amdgcn_readlane(ci, sel);
+        if constexpr (FUSED) {
+          const int lo = __builtin_amdgcn_readlane((int)(uint32_t)pi, sel);
+          const int hi = __builtin_amdgcn_readlane((int)(pi >> 32), sel);
+          nr = (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+        }
+        break;
+      }
+      base += total;
+    }
+  }
+  if (b < 0) return false;  // past the last item
+  b = __builtin_amdgcn_readfirstlane(b);
+  n_parts = __builtin_amdgcn_readfirstlane(n_parts);
+  if constexpr (!WHOLE) {
+    ctx = __builtin_amdgcn_readfirstlane(ctx);
+    if constexpr (FUSED) {
+      const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)nr);
+      const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)nr >> 32));
+      nr = (int64_t)(((uint64_t)hi << 32) | lo);
+    }
+  }
+  const int rem = item - __builtin_amdgcn_readfirstlane(first) * hkv;
+  const int g = rem / n_parts;
+  const int p = rem - g * n_parts;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15;
+  const int h8 = lane & 7;
+  const int z = (lane >> 3) & 1;
+  const int gq = lane >> 4;
+
+  const_i32 *bt_row = (const_i32 *)(a.block_tables + (int64_t)b * a.bt_stride);
+  const int t_begin = p * PART + 64 * w;
+  const int t_end = min(t_begin + 64, ctx);
+  const int bs_mask = (1 << a.bs_log2) - 1;
+  const int64_t row_elems = (int64_t)hkv * D;
+  const int head0 = g * a.q_group + a.q_head0;
+
+  int blk_t[4] = {};
+  if (t_begin < t_end) {
+    const int last = (t_end - 1) & ~15;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) blk_t[i] = bt_row[min(t_begin + 16 * i, last) >> a.bs_log2];
+  }
+
+  // Query operand: lane (z, h, gq) holds dims 64k + 32z + 8gq .. +7 of head h (lanes past the group's
+  // last head repeat it; their columns are never read).
+  u32x4 qf[2];
+  f32x4 rc0 = {}, rc1 = {}, rs0 = {}, rs1 = {};
+  u32x4 qr[2], qw0 = {}, qw1 = {};
+  const int r = lane >> 3, c = lane & 7;
+  if constexpr (!FUSED) {
+    const u16 *qp = a.q + (int64_t)b * a.q_stride + (int64_t)(head0 + min(h8, G - 1)) * D + 32 * z + 8 * gq;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) qf[k] = ld16(qp + 64 * k);
+  } else {
+    // An aligned group of 8 lanes normalises one raw query row.
+    auto rope_row = [&](float (&cs)[8], float (&sn)[8]) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        cs[e] = round_bf16(rc0[e]);
+        cs[4 + e] = round_bf16(rc1[e]);
+        sn[e] = round_bf16(rs0[e]);
+        sn[4 + e] = round_bf16(rs1[e]);
+      }
+    };
+    const bool nr_in = nr >= 0 && nr < ctx;
+    const bool owner = a.store_new && (nr_in ? (nr >= t_begin && nr < t_end) : (p == n_parts - 1 && w == 0));
+    const u16 *qp = a.q + (int64_t)b * a.q_stride + (int64_t)(head0 + min(r, G - 1)) * D + 8 * c;
+    qr[0] = ld16(qp);
+    qr[1] = ld16(qp + 64);
+    if (owner && (nr < 0 || nr >= a.max_positions)) err_bits |= NVAMD_ERR_POSITION;
+    const int64_t pc = nr < 0 ? 0 : (nr >= a.max_positions ? a.max_positions - 1 : nr);
+    const float *row = a.cos_sin + pc * D + 8 * c;
+    rc0 = *reinterpret_cast<const f32x4 *>(row);
+    rc1 = *reinterpret_cast<const f32x4 *>(row + 4);
+    rs0 = *reinterpret_cast<const f32x4 *>(row + 64);
+    rs1 = *reinterpret_cast<const f32x4 *>(row + 68);
+    qw0 = ld16(a.q_w + 8 * c);
+    qw1 = ld16(a.q_w + 64 + 8 * c);
+    if (owner) {
+      const u16 *kp = a.k_new + (int64_t)b * a.k_new_stride + g * D + 8 * c;
+      const u16 *vp = a.v_new + (int64_t)b * a.v_new_stride + g * D + 8 * c;
+      u32x4 k0 = ld16(kp), k1 = ld16(kp + 64);
+      const u32x4 v0 = ld16(vp), v1 = ld16(vp + 64);
+      const u32x4 kw0 = ld16(a.k_w + 8 * c), kw1 = ld16(a.k_w + 64 + 8 * c);
+      const int64_t slot = a.slots[b];
+      __builtin_amdgcn_sched_barrier(0);
+      float cs[8], sn[8];
+      rope_row(cs, sn);
+      head_norm_rope(k0, k1, kw0, kw1, cs, sn, a.eps);
+      if (slot >= a.num_slots || slot < -1) err_bits |= NVAMD_ERR_SLOT;
+      if (r == 0 && slot >= 0 && slot < a.num_slots) {
+        const int64_t dst = slot * row_elems + (int64_t)g * D + 8 * c;
+        u16 *kc = const_cast<u16 *>(a.k_cache);
+        u16 *vc = const_cast<u16 *>(a.v_cache);
+        st16(kc + dst, k0);
+        st16(kc + dst + 64, k1);
+        st16(vc + dst, v0);
+        st16(vc + dst + 64, v1);
+      }
+      __builtin_amdgcn_s_waitcnt(0);  // vmcnt counts stores on gfx9: they are acknowledged
+    }
+  }
+
+  float m = -INFINITY, l = 0.f;
+  f32x4 o[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) o[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int row_bytes = (int)(row_elems * 2);
+  const int k_off = h8 * row_bytes + g * (2 * D) + 64 * z + 16 * gq;
+  const int v_off = 4 * gq * row_bytes + g * (2 * D) + 16 * n;
+  constexpr int kAux = WHOLE ? 0 : kCachePolicyStream;
+
+  // The raw query rows, normalised, reach the operand layout through this wave's own share of s_o.
+  auto norm_queries = [&]() {
+    float cs[8], sn[8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      cs[e] = round_bf16(rc0[e]);
+      cs[4 + e] = round_bf16(rc1[e]);
+      sn[e] = round_bf16(rs0[e]);
+      sn[4 + e] = round_bf16(rs1[e]);
+    }
+    head_norm_rope(qr[0], qr[1], qw0, qw1, cs, sn, a.eps);
+    if (r < GP) {
+      u32x4 *dst = reinterpret_cast<u32x4 *>(&s_o[w][r * HS]);
+      dst[c] = qr[0];
+      dst[8 + c] = qr[1];
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+      qf[k] = reinterpret_cast<const u32x4 *>(&s_o[w][min(h8, GP - 1) * HS])[8 * k + 4 * z + gq];
+  };
+  // Four 16-token tiles: K/V rows and the buffer range of each tile's valid rows.
+  const u16 *kb[4], *vb[4];
+  int bytes[4];
+  u32x4 kt[4][4], vt[2][8];
+  f32x4 s[4];
+  auto tiles = [&]() {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int t0 = t_begin + 16 * i;
+      int blk = blk_t[i];
+      if ((unsigned)blk >= (unsigned)a.num_blocks) err_bits |= NVAMD_ERR_BLOCK;
+      blk = min(max(blk, 0), a.num_blocks - 1);  // never leave the pool
+      const int64_t off = (((int64_t)blk << a.bs_log2) + (t0 & bs_mask)) * row_elems;
+      kb[i] = a.k_cache + off;
+      vb[i] = a.v_cache + off;
+      bytes[i] = min(max(t_end - t0, 0), 16) * row_bytes;
+    }
+  };
+  auto load_k = [&](const int i) {
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16 *>(kb[i]), 0, bytes[i],
+                                                                       kBufferRsrcWord3);
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+        kt[i][2 * x + k] = __builtin_amdgcn_raw_buffer_load_b128(rk, k_off + 128 * k, 8 * x * row_bytes, kAux);
+  };
+  auto load_v = [&](const int h) {
+#pragma unroll
+    for (int i = 2 * h; i < 2 * h + 2; ++i) {
+      const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<u16 *>(vb[i]), 0, bytes[i],
+                                                                         kBufferRsrcWord3);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        vt[h][4 * (i & 1) + t] = __builtin_amdgcn_raw_buffer_load_b128(rv, v_off, t * row_bytes, kAux);
+    }
+  };
+  auto score = [&](const int i) {
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    const f32x4 c0 = mfma16(kt[i][1], qf[1], mfma16(kt[i][0], qf[0], zero));
+    const f32x4 c1 = mfma16(kt[i][3], qf[1], mfma16(kt[i][2], qf[0], zero));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(c0[e]), __float_as_uint(c1[e]), false, false);
+      s[i][e] = __uint_as_float(sw[0]) + dpp<kDppRowRor8>(__uint_as_float(sw[1]));
+    }
+  };
+  u32x4 pf[2], pr[2];
+  auto softmax = [&]() {
+    float cm = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float v = s[i][e] * a.scale_log2e;
+        s[i][e] = t_begin + 16 * i + 4 * gq + e < t_end ? v : -INFINITY;
+        cm = fmaxf(cm, s[i][e]);
+      }
+    cm = max_xor32(max_xor16(cm));
+    const float ref = cm == -INFINITY ? 0.f : cm;  // no visible score yet
+    m = cm;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      // P as a bf16 value and the bf16 of its remainder: a wave's reference is one maximum over 64 tokens, so
+      // P rounded once would put more error on the large weights than the kernel above does, whose 8
+      // references per wave each leave the largest weight of 8 tokens exact (relative error against 64 bits over 4 x
+      // U[8192, 40960]: 2.1e-3 rounded once, 1.7e-3 with the remainder, 1.9e-3 there; no difference in time).
+      // An infinity in V gives NaN.
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 2 * h + (e >> 1), x = 2 * (e & 1);
+        const float p0 = fast_exp2(s[i][x] - ref), p1 = fast_exp2(s[i][x + 1] - ref);
+        pf[h][e] = pack_bf16x2(p0, p1);
+        pr[h][e] = pack_bf16x2(p0 - bf16_lo(pf[h][e]), p1 - bf16_hi(pf[h][e]));
+        l += p0 + p1;
+      }
+    }
+  };
+  auto pv = [&]() {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        u32x4 lo, hi;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          lo[q] = pair_lo(vt[h][2 * q][d], vt[h][2 * q + 1][d]);
+          hi[q] = pair_hi(vt[h][2 * q][d], vt[h][2 * q + 1][d]);
+        }
+        o[2 * d] = mfma16(lo, pr[h], mfma16(lo, pf[h], o[2 * d]));
+        o[2 * d + 1] = mfma16(hi, pr[h], mfma16(hi, pf[h], o[2 * d + 1]));
+      }
+    }
+  };
+  // K first, V in halves as the scores free K's registers: 128 VGPRs (four waves per SIMD) hold no more.
+  // Every load up front at 147-183 VGPRs measured the same or slower, at small batches too.
+  if (t_begin < t_end) {
+    tiles();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) load_k(i);
+    if constexpr (FUSED) norm_queries();  // while K is in flight
+    __builtin_amdgcn_sched_barrier(0);
+    score(0);
+    score(1);
+    __builtin_amdgcn_sched_barrier(0);
+    load_v(0);
+    score(2);
+    score(3);
+    softmax();
+    __builtin_amdgcn_sched_barrier(0);
+    load_v(1);
+    __builtin_amdgcn_sched_barrier(0);
+    pv();
+  }
+
+  err_bits = __builtin_amdgcn_readfirstlane(err_bits);
+  if (err_bits != 0 && lane == 0) flag_index_error(a.err, err_bits);
+
+  // The wave's tile to LDS: register i of o[e] is dim 8(4gq + i) + e of head n.
+  l = sum_xor32(sum_xor16(l));
+  if (n < G) {
+    float *dst = &s_o[w][n * HS + 32 * gq];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      *reinterpret_cast<f32x4 *>(dst + 8 * i) = f32x4{o[0][i], o[1][i], o[2][i], o[3][i]};
+      *reinterpret_cast<f32x4 *>(dst + 8 * i + 4) = f32x4{o[4][i], o[5][i], o[6][i], o[7][i]};
+    }
+    if (gq == 0) {
+      s_m[w][n] = m;
+      s_l[w][n] = l;
+    }
+  }
+  __syncthreads();
+
+  // Workgroup merge: a half-wave takes a head, its lane dims 4dl .. 4dl+3.
+  constexpr int kHalves = 2 * NW;
+  static_assert(WHOLE || (GP <= kHalves && kHalves <= NW * GP), "one head per half-wave; the shares of a merge fit s_o");
+  constexpr int HP = (GP + kHalves - 1) / kHalves;  // heads per half-wave
+  const int hw = tid >> 5;
+  constexpr int MP = 8;  // partitions whose records a half-wave loads at a time
+  // The merge's head slots (2, 4 or 8) and the half-waves that share a head's merge.
+  const int slots_log2 = G <= 2 ? 1 : (G <= 4 ? 2 : 3);
+  const int split = kHalves >> slots_log2;
+  const bool shared = !WHOLE && split > 1 && n_parts > 2 * MP;
+  // Waves without a head are done, unless they share the merge (or the workgroup's next item, whose
+  // barriers all of its waves meet).
+  const bool idle = 2 * w >= G && !shared;
+  if (!MANY && idle) return true;
+  const int dl = lane & 31;
+  f32x4 acc[HP];
+  float mx[HP], ls[HP];
+#pragma unroll
+  for (int k = 0; k < HP; ++k) {
+    const int h = min(hw + k * kHalves, G - 1);
+    float M = -INFINITY;
+#pragma unroll
+    for (int x = 0; x < NW; ++x) M = fmaxf(M, s_m[x][h]);
+    acc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    ls[k] = 0.f;
+#pragma unroll
+    for (int x = 0; x < NW; ++x) {
+      const float mv = s_m[x][h];
+      const float f = mv == -INFINITY ? 0.f : fast_exp2(mv - M);
+      acc[k] += f * *reinterpret_cast<const f32x4 *>(&s_o[x][h * HS + 4 * dl]);
+      ls[k] += f * s_l[x][h];
+    }
+    mx[k] = M;
+  }
+  u16 *out_base = a.out + (int64_t)b * a.out_stride + (int64_t)head0 * D + 4 * dl;
+  auto write_out = [&](int h, f32x4 v, float den) {
+    const float inv = den > 0.f ? 1.f / den : 0.f;
+    *reinterpret_cast<u32x2 *>(out_base + h * D) =
+        u32x2{pack_bf16x2(v[0] * inv, v[1] * inv), pack_bf16x2(v[2] * inv, v[3] * inv)};
+  };
+  if (WHOLE || n_parts <= 1) {
+#pragma unroll
+    for (int k = 0; k < HP; ++k)
+      if (hw + k * kHalves < G) write_out(hw + k * kHalves, acc[k], ls[k]);
+    return true;
+  }
+  if constexpr (!WHOLE) {
+    // A partition's record: per head (max, sum, 2 unused, 128 accumulators).
+    float *part_base = a.partials + (((int64_t)b * hkv + g) * a.max_parts) * (G * HS);
+    const int rec_bytes = G * HS * (int)sizeof(float);
+    const __amdgpu_buffer_rsrc_t rsrc =
+        __builtin_amdgcn_make_buffer_rsrc(part_base, 0, n_parts * rec_bytes, kBufferRsrcWord3);
+    if (hw < G) {
+      const int off = p * rec_bytes + hw * (HS * (int)sizeof(float));
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, acc[0]), rsrc, off + 16 + 16 * dl, 0,
+                                             kCachePolicyAgent);
+      if (dl == 0)
+        __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(mx[0]), __float_as_uint(ls[0])}, rsrc, off, 0,
+                                              kCachePolicyAgent);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // keep the stores above the wait
+    __builtin_amdgcn_s_waitcnt(0);
+    unsigned *counter = reinterpret_cast<unsigned *>(a.counters + (int64_t)b * hkv + g);
+    int prev = 0;
+    if (G <= 2 && !shared) {  // wave 0 holds every head
+      if (w != 0) return true;
+      if (lane == 0)
+        prev = (int)__builtin_amdgcn_atomic_inc32(counter, (unsigned)(n_parts - 1), __ATOMIC_RELAXED, "agent");
+      prev = __builtin_amdgcn_readfirstlane(prev);
+    } else {
+      __syncthreads();  // every publishing wave's stores are acknowledged
+      if (tid == 0)
+        s_last = (int)__builtin_amdgcn_atomic_inc32(counter, (unsigned)(n_parts - 1), __ATOMIC_RELAXED, "agent");
+      __syncthreads();
+      prev = s_last;
+    }
+    if (prev != n_parts - 1 || idle) return true;
+
+    // The last arriver merges.  Half-wave sp of the `split` that share a head takes every split-th run of MP
+    // partitions, 64 of its own at a time: two (max, sum) pairs per lane, the running numerator and
+    // denominator rescaled to the maximum so far.
+    const int h = hw & ((1 << slots_log2) - 1), sp = hw >> slots_log2;
+    const int hoff = min(h, G - 1) * (HS * (int)sizeof(float));
+    const int stride = shared ? split : 1;
+    auto part = [&](int y) { return ((y / MP) * stride + (shared ? sp : 0)) * MP + y % MP; };  // its y-th partition
+    const int mine = ceil_div(n_parts, stride * MP) * MP;
+    f32x4 num = {0.f, 0.f, 0.f, 0.f};
+    float M = -INFINITY, den = 0.f;
+#pragma unroll 1
+    for (int y0 = 0; y0 < mine; y0 += 64) {
+      float pm[2], pl[2], fx[2];
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const int pi = part(y0 + dl + 32 * x);
+        const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rsrc, pi * rec_bytes + hoff, 0, kCachePolicyAgent);
+        pm[x] = pi < n_parts ? __uint_as_float(v[0]) : -INFINITY;
+        pl[x] = __uint_as_float(v[1]);
+      }
+#pragma unroll 1
+      for (int y = 0; y < min(mine - y0, 64); y += MP) {
+        u32x4 v[MP];
+        const int base = part(y0 + y) * rec_bytes + hoff + 16 + 16 * dl;
+#pragma unroll
+        for (int k = 0; k < MP; ++k)  // past n_parts: zeros, no memory access
+          v[k] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, base + k * rec_bytes, 0, kCachePolicyAgent);
+        if (y == 0) {
+          const float m_new = fmaxf(M, half_max(fmaxf(pm[0], pm[1])));
+#pragma unroll
+          for (int x = 0; x < 2; ++x) fx[x] = pm[x] == -INFINITY ? 0.f : fast_exp2(pm[x] - m_new);
+          const float alpha = M == -INFINITY ? 0.f : fast_exp2(M - m_new);
+          den = den * alpha + half_sum(fx[0] * pl[0] + fx[1] * pl[1]);
+          num *= alpha;
+          M = m_new;
+        }
+        const float fr = y < 32 ? fx[0] : fx[1];
+#pragma unroll
+        for (int k = 0; k < MP; ++k)
+          num += __shfl(fr, (lane & 32) + ((y + k) & 31)) * __builtin_bit_cast(f32x4, v[k]);
+      }
+    }
+    if (shared) {
+      // s_o, s_m and s_l are free: every wave has passed two barriers since it read them.  The shares of
+      // a head meet in share order.
+      float *so = &s_o[0][0], *sm = &s_m[0][0], *sl = &s_l[0][0];
+      *reinterpret_cast<f32x4 *>(so + hw * HS + 4 * dl) = num;
+      if (dl == 0) {
+        sm[hw] = M;
+        sl[hw] = den;
+      }
+      __syncthreads();
+      if (sp == 0) {
+        float mm = M;
+        for (int x = 1; x < split; ++x) mm = fmaxf(mm, sm[(x << slots_log2) + h]);
+        const float f0 = M == -INFINITY ? 0.f : fast_exp2(M - mm);
+        num *= f0;
+        den *= f0;
+        for (int x = 1; x < split; ++x) {
+          const int y = (x << slots_log2) + h;
+          const float f = sm[y] == -INFINITY ? 0.f : fast_exp2(sm[y] - mm);
+          num += f * *reinterpret_cast<const f32x4 *>(so + y * HS + 4 * dl);
+          den += f * sl[y];
+        }
+      }
+    }
+    if (sp == 0 && h < G) write_out(h, num, den);
+  }
+  return true;
+}
+
+// MANY: a workgroup takes items blockIdx.x, + gridDim.x, ... of a launch of kMaxGroups workgroups, so a
+// context bound far above the contexts (a model's longest) costs no dispatch of empty ones (8,192 more empty
+// workgroups: 4-8 us).  Each
+// item reads its arguments and thread index anew: values kept over the loop would not fit the
+// registers.
+template <int GP, int NW, bool WHOLE, bool FUSED, bool MANY>
+__global__ void __launch_bounds__(NW * 64)
+__attribute__((amdgpu_waves_per_eu(4)))
+paged_decode_mfma_kernel(DecodeArgs a) {
+  __shared__ __attribute__((aligned(16))) float s_o[NW][GP * kPartFloats];
+  __shared__ float s_m[NW][GP];
+  __shared__ float s_l[NW][GP];
+  __shared__ int s_last;
+  if constexpr (!MANY) {
+    mfma_item<GP, NW, WHOLE, FUSED, MANY>(a, threadIdx.x, blockIdx.x, s_o, s_m, s_l, s_last);
+  } else {
+    const int items = a.max_items;
+#pragma unroll 1
+    for (int item = blockIdx.x;;) {
+      typedef const __attribute__((address_space(4))) DecodeArgs const_args;
+      const_args *p = (const_args *)__builtin_amdgcn_kernarg_segment_ptr();
+      int tid = threadIdx.x;
+      asm volatile("" : "+s"(p), "+v"(tid));
+      const DecodeArgs args = *(const DecodeArgs *)p;
+      if (!mfma_item<GP, NW, WHOLE, FUSED, MANY>(args, tid, item, s_o, s_m, s_l, s_last)) break;
+      item += gridDim.x;
+      if (item >= items) break;
+      __syncthreads();  // every wave has read this item's LDS
+    }
+  }
+}
+
+template <int GP, int NW, bool WHOLE, bool FUSED>
+int launch_mfma(DecodeArgs a, int batch, hipStream_t stream) {
+  a.max_parts = ceil_div(a.max_ctx, NW * 64);
+  if (WHOLE && a.max_parts != 1) return NVAMD_EINVAL;
+  a.batch = batch;
+  const int64_t items = (int64_t)batch * a.num_kv_heads * a.max_parts;
+  a.max_items = (int)items;  // <= kCounterSlots units of <= 512 partitions
+  if constexpr (!WHOLE) {
+    if (items > kMaxGroups) {
+      hipLaunchKernelGGL((paged_decode_mfma_kernel<GP, NW, WHOLE, FUSED, true>), dim3(kMaxGroups), dim3(NW * 64),
+                         0, stream, a);
+      return launch_status();
+    }
+  }
+  hipLaunchKernelGGL((paged_decode_mfma_kernel<GP, NW, WHOLE, FUSED, false>), dim3((unsigned)items),
+                     dim3(NW * 64), 0, stream, a);
   return launch_status();
 }
 
@@ -670,33 +1232,53 @@ int num_cus() {
   return cus;
 }
 
+// 256-token partitions of 4 waves (measured best on MI355X for 32 x ~1.3k contexts).  A launch
+// whose context bound gives fewer than two such items per CU is latency-bound: with a bound of
+// <= 512 tokens one workgroup of bound/64 waves takes a whole (sequence, kv head), so there is
+// no cross-workgroup merge.  Beyond that one CU would stream a whole unit, and a CU alone reads
+// at most ~41-57 GB/s: bounds of 513-1024 tokens split into 256-token partitions too (whole
+// units of 16 waves measured 1.2-1.7x slower for 1-16 sequences).  The 256-token partitions
+// stay at any batch: 128- or 64-token partitions of 2 or 1 waves (more workgroups, more partials
+// to merge) measured 1.1-1.7x slower for 1-8 sequences of 2-4k tokens and for one kv head.
+// Waves of a whole-unit workgroup, or 0 for a split launch.
+int whole_waves(const DecodeArgs &a, int batch) {
+  const int64_t units = (int64_t)batch * a.num_kv_heads;
+  if (units * ceil_div(a.max_ctx, 256) >= 2LL * num_cus() || a.max_ctx > 512) return 0;
+  const int nw = ceil_div(a.max_ctx, 64);
+  return nw <= 2 ? 2 : (nw <= 4 ? 4 : 8);
+}
+
 template <int GQA, bool FUSED>
 int dispatch(const DecodeArgs &a, int batch, hipStream_t stream) {
-  // 256-token partitions of 4 waves (measured best on MI355X for 32 x ~1.3k contexts).  A launch
-  // whose context bound gives fewer than two such items per CU is latency-bound: with a bound of
-  // <= 512 tokens one workgroup of bound/64 waves takes a whole (sequence, kv head), so there is
-  // no cross-workgroup merge.  Beyond that one CU would stream a whole unit, and a CU alone reads
-  // at most ~41-57 GB/s: bounds of 513-1024 tokens split into 256-token partitions too (whole
-  // units of 16 waves measured 1.2-1.7x slower for 1-16 sequences).  The 256-token partitions
-  // stay at any batch: 128- or 64-token partitions of 2 or 1 waves (more workgroups, more partials
-  // to merge) measured 1.1-1.7x slower for 1-8 sequences of 2-4k tokens and for one kv head.
+  switch (whole_waves(a, batch)) {
+    case 2: return launch<GQA, 2, true, FUSED>(a, batch, stream);
+    case 4: return launch<GQA, 4, true, FUSED>(a, batch, stream);
+    case 8: return launch<GQA, 8, true, FUSED>(a, batch, stream);
+    default: return launch<GQA, 4, false, FUSED>(a, batch, stream);
+  }
+}
+
+// Partitions of the MFMA variant: 256 tokens, or 512 tokens of 8 waves (half the partial records) in two cases.
+// Groups of 5 to 8 heads publish 4 KB per partition, 3% of what a 256-token partition reads: launches of
+// more than 8,192 items, which are bandwidth-bound over many rounds, take 512 (100 x U[2048, 4096] at 8
+// heads: 235 against 245 us; fewer items prefer 256: 28.7 against 30.5 us at 16 x U[512, 4096]).  Bounds past
+// 16,384 tokens over fewer than 64 (sequence, kv head) units take 512 for the sake of the last merges,
+// 80 records instead of 160 at 40,960 tokens (4 x U[8192, 40960]: 59.2 / 55.2 / 53.1 against 67.2 / 59.4 / 54.6 us at 8 /
+// 4 / 2 heads); over more units contexts tend to be far shorter than such a bound: 256 (32 x U[256, 2304]
+// at a bound of 40,960: 36.7 against 38.9 us at 2 heads, 40.5 against 42.5 us at 8).
+template <int GP, bool FUSED>
+int dispatch_mfma(const DecodeArgs &a, int batch, hipStream_t stream) {
+  if (a.max_ctx > kMaxContext) return NVAMD_EUNSUPPORTED;
   const int64_t units = (int64_t)batch * a.num_kv_heads;
-  const int64_t want = 2LL * num_cus();
-  if (units * ceil_div(a.max_ctx, 256) < want) {
-    const int nw_whole = ceil_div(a.max_ctx, 64);
-    if (nw_whole <= 2) return launch<GQA, 2, 1, 4, true, FUSED>(a, batch, stream);
-    if (nw_whole <= 4) return launch<GQA, 4, 1, 4, true, FUSED>(a, batch, stream);
-    if (nw_whole <= 8) return launch<GQA, 8, 1, 4, true, FUSED>(a, batch, stream);
+  switch (whole_waves(a, batch)) {
+    case 2: return launch_mfma<GP, 2, true, FUSED>(a, batch, stream);
+    case 4: return launch_mfma<GP, 4, true, FUSED>(a, batch, stream);
+    case 8: return launch_mfma<GP, 8, true, FUSED>(a, batch, stream);
+    default: break;
   }
-  int cpw = 1;
-  while (ceil_div(a.max_ctx, 256 * cpw) > 64) cpw *= 2;
-  switch (cpw) {
-    case 1: return launch<GQA, 4, 1, 4, false, FUSED>(a, batch, stream);
-    case 2: return launch<GQA, 4, 2, 4, false, FUSED>(a, batch, stream);
-    case 4: return launch<GQA, 4, 4, 4, false, FUSED>(a, batch, stream);
-    case 8: return launch<GQA, 4, 8, 4, false, FUSED>(a, batch, stream);
-    default: return NVAMD_EUNSUPPORTED;
-  }
+  if ((GP == 8 && units * ceil_div(a.max_ctx, 256) > 8192) || (a.max_ctx > 16384 && units < 64))
+    return launch_mfma<GP, 8, false, FUSED>(a, batch, stream);
+  return launch_mfma<GP, 4, false, FUSED>(a, batch, stream);
 }
 
 }  // namespace
@@ -760,22 +1342,25 @@ int fill_decode_args(DecodeArgs &a, void *out, int64_t out_stride, const void *q
   return NVAMD_OK;
 }
 
-// The kernel holds 1, 2 or 4 query heads per kv head in registers.  Other ratios (Qwen3-14B's 5,
-// Qwen3-32B's 8) run as consecutive launches over 4, then 2, then 1 heads of every group; each
-// re-reads the group's K/V, and only the first stores the fused step's new k / v.
+// Groups of 3 to 8 query heads take the MFMA variant, larger ones consecutive launches over 8 heads and
+// the rest; each launch re-reads the group's K/V, and only the first stores the fused step's new k / v.
+// Groups of 1 and 2 heads keep the dot-product kernel, which is as fast over large batches and faster
+// where latency counts (at 2 heads 33.6 against 33.9 us over 32 x U[256, 2304], 6.6 against 7.1 us over 4 x U[1, 512]; at 4
+// heads the MFMA variant leads: 35.7 against 36.5 us and 7.2 against 9.6 us), up to the 64 partitions of 256
+// tokens that its merge holds.
 template <bool FUSED>
 int dispatch_gqa(DecodeArgs a, int gqa, int batch, hipStream_t stream) {
   a.q_group = gqa;
   for (int head0 = 0; head0 < gqa;) {
-    const int rest = gqa - head0;
-    const int sub = rest >= 4 ? 4 : (rest >= 2 ? 2 : 1);
     a.q_head0 = head0;
+    a.q_sub = min(gqa - head0, 8);
     a.store_new = head0 == 0;
-    const int st = sub == 4 ? dispatch<4, FUSED>(a, batch, stream)
-                 : sub == 2 ? dispatch<2, FUSED>(a, batch, stream)
-                            : dispatch<1, FUSED>(a, batch, stream);
+    const bool dots = a.q_sub <= 2 && a.max_ctx <= 16384;
+    const int st = dots ? (a.q_sub == 2 ? dispatch<2, FUSED>(a, batch, stream) : dispatch<1, FUSED>(a, batch, stream))
+                 : a.q_sub <= 4 ? dispatch_mfma<4, FUSED>(a, batch, stream)
+                                : dispatch_mfma<8, FUSED>(a, batch, stream);
     if (st != NVAMD_OK) return st;
-    head0 += sub;
+    head0 += a.q_sub;
   }
   return NVAMD_OK;
 }

@@ -172,3 +172,13 @@ def test_fused_step_graph_replays(device):
         ref_out, ref_kc, ref_vc = case.unfused(max_ctx)
         torch.cuda.synchronize()
         assert torch.equal(out, ref_out) and torch.equal(kc, ref_kc) and torch.equal(vc, ref_vc)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,bound", [((24, 8), 0), ((32, 8), 4096), ((40, 8), 0), ((64, 8), 4096), ((9, 1), 0),
+                                         ((2, 1), 40960), ((16, 2), 40960), ((64, 8), 40960)])
+def test_fused_step_mfma_groups(device, heads, bound):
+    """The MFMA variant's fused step: the new token in every wave of a partition, at its ends, in a partition
+    of its own, and outside the pool's order; bounds that share merges and loop over items."""
+    ctx = [1, 64, 65, 129, 200, 256, 257, 300, 777, 1023, 1025, 2100]
+    check(Case(device, len(ctx), 0, 0, 128, seed=11, heads=heads, context_lens=ctx), max_ctx=bound or None)

@@ -274,3 +274,44 @@ def test_range_checks_raise_before_launching(device):
     finally:
         _C.set_range_checks(prev)
     torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads", [(3, 1), (8, 2), (5, 1), (8, 1), (9, 1), (16, 1), (19, 1)])
+def test_decode_mfma_groups(device, heads):
+    """Groups past 2 query heads: one MFMA launch per 8 heads (9, 16 and 19 take a second and third), whole units
+    and split launches, contexts at the edges of a 16-token tile, a wave, a partition and its merge."""
+    hq, hkv = heads
+    ctx = [1, 15, 16, 17, 63, 64, 65, 0, 255, 256, 257, 511, 512]
+    check(W.make_decode(len(ctx), 0, 0, 64, seed=hq, device=device, num_heads=hq, num_kv_heads=hkv, context_lens=ctx))
+    ctx += [513, 2048, 2049, 4095, 4097, 6000]  # 8 partitions, 9, 16, 17 (merges of one and more loads)
+    work = W.make_decode(len(ctx), 0, 0, 220, seed=hq, device=device, num_heads=hq, num_kv_heads=hkv, context_lens=ctx)
+    check(work)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,batch", [((1, 1), 3), ((2, 1), 70), ((8, 2), 5), ((8, 1), 70), ((40, 8), 9)])
+def test_decode_mfma_shared_merges_and_item_loops(device, heads, batch):
+    """Bounds past 16,384 tokens: merges of many partitions shared by the half-waves (512-token partitions below
+    64 units, 256-token ones above), and workgroups that take several items (more than 4,096 of them)."""
+    hq, hkv = heads
+    ctx = [20000, 1, 4200] + [(37 * i) % 900 for i in range(batch - 3)]
+    work = W.make_decode(batch, 0, 0, 600, seed=batch, device=device, num_heads=hq, num_kv_heads=hkv, context_lens=ctx)
+    check(work, max_ctx=40960)
+    check(work, max_ctx=131072)
+
+
+@pytest.mark.gpu
+def test_decode_many_items_per_workgroup(device):
+    """More items than workgroups with real contexts behind them: 120 sequences x 8 kv heads of 8 heads."""
+    ctx = [1200 + 13 * (i % 60) for i in range(120)]
+    work = W.make_decode(120, 0, 0, 120 * 16, seed=9, device=device, num_heads=64, num_kv_heads=8, context_lens=ctx)
+    check(work, max_ctx=4096)
+    check(work, max_ctx=2560)
+
+
+@pytest.mark.gpu
+def test_decode_refuses_bounds_past_the_largest(device):
+    work = W.make_decode(1, 0, 0, 8, seed=1, device=device, num_heads=8, num_kv_heads=1, context_lens=[40])
+    with pytest.raises(ValueError, match="unsupported"):
+        run_decode(work.q, work.key_cache[0], work.value_cache[0], work.block_tables, work.context_lens, 131073)
