@@ -86,3 +86,25 @@ def test_argmax_rows_ragged_vocab_and_ties_within_a_thread(device):
     out = _C.argmax_rows(logits)
     torch.cuda.synchronize()
     assert out.tolist() == [8, 24, vocab - 1, 5, logits[4].float().argmax().item(), 0]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,hidden", [(1, 8), (3, 504), (5, 520), (2, 2040), (9, 2560), (4, 4088), (7, 5120), (3, 8192),
+                                         (5, 8200), (4100, 4096)])
+def test_add_rms_norm_row_widths(device, rows, hidden):
+    """Widths that leave lanes without a vector, each register count's ends, the two-pass kernel (past 8192) and
+    the streaming form (16M elements and more); within one bf16 rounding of the fp32 reference."""
+    g = torch.Generator(device=device).manual_seed(hidden)
+    delta, res, w = (torch.randn(n, generator=g, device=device).bfloat16()
+                     for n in (rows * hidden, rows * hidden, hidden))
+    delta, res = delta.view(rows, hidden), res.view(rows, hidden)
+    total = (res.float() + delta.float()).bfloat16()
+    for d, x in ((delta, total), (None, res.clone())):
+        got_res, out = res.clone(), torch.full_like(res, float("nan"))
+        _C.add_rms_norm(d, got_res, w, out, 1e-6)
+        torch.cuda.synchronize()
+        assert torch.equal(got_res, x)
+        f = x.float()
+        ref = f * torch.rsqrt(f.pow(2).mean(-1, keepdim=True) + 1e-6) * w.float()
+        # one bf16 rounding (2^-9) of the value, and fp32 sums in another order
+        assert ((out.float() - ref).abs() <= ref.abs() * (2.0 ** -8) + 1e-6).all()
