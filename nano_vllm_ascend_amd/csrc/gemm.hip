@@ -358,35 +358,57 @@ struct Plan {
   int nw, nt, ks, kb;
 };
 
-// Measured on MI355X at M = 32: the decode step's projection sequence over 28 layers' own
-// weights (882 MB, streamed from HBM as in the model), replayed as one graph:
-//   * vocabulary-sized N (LM head): 128 columns per 4-wave workgroup, no split;
+// Measured on MI355X with weights streamed from HBM (rotating copies, one graph), us per launch:
+//   * vocabulary-sized N (LM head), no split: 32 columns per 8-wave workgroup up to 16 rows (N = 151,936, K = 1,024 / 4,096 at M = 4:
+//     51.8 / 211 against 56.3 / 226 for 128 columns of 4 waves), 64 up to 32 rows (58.5 / 236.7 against
+//     61.6 / 242), where X is read again per column group; 64 of 4 waves for 64-row slabs (128
+//     would need 128 accumulator registers at 4 M tiles);
 //   * residual epilogue (N = hidden: o_proj, down_proj): 32 columns (the epilogue's sums of
 //     squares cover whole 32-column groups) per 8-wave workgroup, K split over >= 128
-//     workgroups (o 6.5 us, down 6.6 us; 4-wave workgroups over >= 256: 6.7 / 7.4 us;
-//     unsplit 16-wave workgroups: 8.2 us, faster only while the weights sit in the
-//     Infinity Cache);
-//   * otherwise (qkv, gate_up): 16 columns per 8-wave workgroup, no split.
-// 64-row slabs (wide): the vocabulary-sized projection takes 64 columns per workgroup (128
-// would need 128 accumulator registers at 4 M tiles); with two slabs (M > 64) the other
-// projections take 32 columns per workgroup, halving the X reads per weight byte (a projection
-// chain at M = 100: 35.2-35.8 against 41.4-42.1 us per layer; at M = 64, one slab, the halved
-// workgroup count makes it slower).
+//     workgroups (at N = 1,024, K = 2,048 / 3,072 o 6.5, down 6.6; unsplit 16-wave workgroups 8.2).  A long K
+//     (down_proj, K >= 1.5 N) is split further, to >= 512 workgroups of >= 1,152 K each, where a workgroup's
+//     stream would otherwise last many rounds of 128 workgroups: at M = 32, N x K = 4,096 x 12,288 22.6 against 32.7,
+//     5,120 x 17,408 37.4 against 47.2, 2,560 x 9,728 14.6 against 16.7, 2,048 x 6,144 9.3 against 11.6; where that gives 512
+//     workgroups four waves lead eight (37.4 / 42, 14.6 / 15.9).  Above 64 rows the merges of two slabs cost what the split gains
+//     (4,096 x 12,288 at M = 100: 39.4 unsplit, 42.4 in two);
+//   * gate_up: 16 columns per 8-wave workgroup; from N = 4,096 on 32, from N = 8,192 on and up to 32 rows 16 per 4-wave workgroup (M = 32:
+//     6,144 x 2,048 normed 14.1 against 17.3, 12,288 x 4,096 37.3 against 39.6, 9,728 x 2,560 21.2 against 23.5; above 64 rows
+//     32 per 4-wave workgroup, 62.3 against 67.2);
+//   * otherwise (qkv): 16 columns per 8-wave workgroup, 32 from N = 6,144 on (6,144 x 4,096 at M = 8 / 32: 11.4 / 13.5
+//     against 13.6 / 17.5) and above 64 rows, halving the X reads per weight byte (normed, K = 2,048 at
+//     M = 100: 13.6 against 20.3).
 Plan make_plan(int n, int k, int epi, int m, bool wide) {
   Plan p{8, 1, 1, k % 512 == 0 ? 2 : 1};
   if (epi == kEpiStore && n % 128 == 0 && n / 128 >= 512) {
-    p = wide ? Plan{4, 4, 1, 2} : Plan{4, 8, 1, 2};
-  } else if (wide && m > 64 && epi != kEpiResid) {
-    p.nt = 2;
-  } else if (epi == kEpiResid) {
+    if (wide) return Plan{4, 4, 1, 2};
+    return m <= 16 ? Plan{8, 2, 1, 2} : Plan{8, 4, 1, 1};
+  }
+  if (epi == kEpiResid) {
     p = Plan{8, 2, 1, 2};
     const int groups = n / 32;
     static const int kSlices[] = {1, 2, 3, 4, 6, 8, 12, 16};
+    auto whole = [&](int ks) { return k % ks == 0 && (k / ks) % 64 == 0; };  // 64-wide wave blocks
     for (int ks : kSlices) {
-      if (k % ks != 0 || (k / ks) % 64 != 0) continue;  // whole 64-wide wave blocks per slice
+      if (!whole(ks)) continue;
       p.ks = ks;
       if (groups * ks >= 128) break;
     }
+    if (m > 64 || 2 * k < 3 * n) return p;
+    for (int ks : kSlices) {
+      if (groups * p.ks >= 512 || k / ks < 1152) break;
+      if (ks > p.ks && whole(ks)) p.ks = ks;
+    }
+    if (groups * p.ks >= 512) p = Plan{4, 2, p.ks, 1};
+    return p;
+  }
+  if (m > 64) {
+    p.nt = 2;
+    if (epi == kEpiSilu ? n >= 4096 : !wide && n < 6144) p.nw = 4;
+  } else if (epi == kEpiSilu) {
+    if (n >= 8192 && m <= 32) return Plan{4, 1, 1, k <= 4096 ? 1 : 2};
+    if (n >= 4096 && n < 8192) return Plan{8, 2, 1, 1};
+  } else if (n >= 6144) {
+    p.nt = 2;
   }
   return p;
 }
@@ -407,13 +429,13 @@ bool wide_rows(int m, int k, bool norm, int epi) {
   return m > 32 && (!norm || (k <= kMaxWideNormK && epi != kEpiResid));
 }
 // Configurations 64-row slabs are built for (at most 64 columns per workgroup).
-template <int NT, int EPI, bool NORM>
-constexpr bool kWideBuilt = NT <= 4 && !(NORM && EPI == kEpiResid);
+template <int NW, int NT, int EPI, bool NORM>
+constexpr bool kWideBuilt = (NT <= 2 || NW == 4) && !(NORM && EPI == kEpiResid);
 
 template <int NW, int KB, int NT, int EPI, bool NORM>
 int launch(const GemmArgs &a, int grid, bool wide, hipStream_t stream) {
   if (wide) {
-    if constexpr (kWideBuilt<NT, EPI, NORM>) {
+    if constexpr (kWideBuilt<NW, NT, EPI, NORM>) {
       if (a.m <= 64)
         hipLaunchKernelGGL((skinny_gemm_kernel<NW, KB, NT, 4, EPI, NORM, false>), dim3(grid), dim3(NW * 64), 0,
                            stream, a);
@@ -444,15 +466,16 @@ int launch_kb(const GemmArgs &a, const Plan &p, int grid, bool wide, hipStream_t
 template <int EPI, bool NORM>
 int dispatch(const GemmArgs &a, const Plan &p, int grid, bool wide, hipStream_t stream) {
   if constexpr (EPI == kEpiStore) {
-    if (p.nw == 4 && p.nt == 8) return launch_kb<4, 8, EPI, NORM>(a, p, grid, wide, stream);
     if (p.nw == 4 && p.nt == 4) return launch_kb<4, 4, EPI, NORM>(a, p, grid, wide, stream);
+    if (p.nw == 8 && p.nt == 4) return launch_kb<8, 4, EPI, NORM>(a, p, grid, wide, stream);
+  } else if constexpr (EPI == kEpiSilu) {
+    if (p.nw == 4 && p.nt == 1) return launch_kb<4, 1, EPI, NORM>(a, p, grid, wide, stream);
   }
-  if constexpr (EPI == kEpiResid) {
-    if (p.nw == 8 && p.nt == 2) return launch_kb<8, 2, EPI, NORM>(a, p, grid, wide, stream);
-  } else {
+  if constexpr (EPI != kEpiResid) {
     if (p.nw == 8 && p.nt == 1) return launch_kb<8, 1, EPI, NORM>(a, p, grid, wide, stream);
-    if (p.nw == 8 && p.nt == 2) return launch_kb<8, 2, EPI, NORM>(a, p, grid, wide, stream);
   }
+  if (p.nw == 4 && p.nt == 2) return launch_kb<4, 2, EPI, NORM>(a, p, grid, wide, stream);
+  if (p.nw == 8 && p.nt == 2) return launch_kb<8, 2, EPI, NORM>(a, p, grid, wide, stream);
   return NVAMD_EUNSUPPORTED;
 }
 

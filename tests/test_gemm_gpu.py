@@ -362,3 +362,56 @@ def test_random_rows_and_epilogues(device, seed):
             torch.cuda.synchronize()
             assert torch.equal(y[sl], y1), (f"epilogue {epi} norm {norm} m {m} n {n} k {k} row {row}: "
                                             f"max diff {(y[sl].float() - y1.float()).abs().max().item():.3g}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 16, 17, 32, 33, 64, 65, 128])
+@pytest.mark.parametrize("nk", [(6144, 512), (4096, 2048), (65536, 256)], ids=["n6144", "k2048", "vocab"])
+def test_linear_column_plans(device, m, nk):
+    """The store plans by width and rows: 16 and 32 columns per workgroup, and the vocabulary-sized ones."""
+    n, k = nk
+    x, w = _operands(m, n, k, device, seed=m + n)
+    y = _C.linear(x, _C.tile(w))
+    torch.cuda.synchronize()
+    _assert_close_bf16(y, x.float() @ w.float().t())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [3, 32, 48, 100])
+@pytest.mark.parametrize("inter,k", [(4096, 512), (8192, 256), (8192, 4352)])
+def test_silu_column_plans(device, m, inter, k):
+    """The gate/up plans by width, depth and rows against the projection and SiLU launches: the same rounding
+    points, so an element differs only where a sum in another order rounds to the neighbouring value."""
+    x, w = _operands(m, 2 * inter, k, device, seed=m + k)
+    y = _C.linear_silu_mul(x, _C.tile(w)).float()
+    full = (x.float() @ w.float().t()).to(torch.bfloat16)
+    ref = _C.silu_mul(full).float()
+    torch.cuda.synchronize()
+    # one step of gate or up (2^-7 of it, the SiLU's slope is at most 1.1) and of the two later roundings
+    bound = 2.0 ** -6 * ref.abs() + 2.0 ** -7 * 1.1 * full[:, :inter].abs().float() * full[:, inter:].abs().float() + 3e-5
+    assert ((y - ref).abs() <= bound).all()
+    assert ((y - ref).abs() <= 4 * ULP * ref.abs() + 1e-3).float().mean().item() > 0.999
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 16, 32, 64, 65, 128])
+@pytest.mark.parametrize("nk", [(2048, 6144), (2560, 9728), (4096, 6144), (256, 2304)])
+def test_residual_long_k_plans(device, m, nk):
+    """K split further than 128 workgroups need (4, 8 and 4 slices, of 8 or 4 waves), and a K that keeps its split."""
+    n, k = nk
+    x, w = _operands(m, n, k, device, seed=k + m)
+    gen = torch.Generator(device=device).manual_seed(6)
+    r0 = torch.randn((m, n), generator=gen, device=device).to(torch.bfloat16)
+    r, wt = r0.clone(), _C.tile(w)
+    ssq = torch.full((m, n // 32), -1.0, device=device)
+    ws = torch.zeros(_C.skinny_linear_workspace_size(n, k, _C.EPI_RESID), dtype=torch.uint8, device=device)
+    _C.skinny_linear(x, wt, r, epilogue=_C.EPI_RESID, y_ssq=ssq, workspace=ws)
+    torch.cuda.synchronize()
+    d = (x.float() @ w.float().t()).to(torch.bfloat16).float()
+    ref = r0.float() + d
+    assert ((r.float() - ref).abs() <= 2 * ULP * (d.abs() + ref.abs()) + 1e-5).all()
+    assert torch.allclose(ssq, _tile_ssq(r), rtol=1e-5, atol=1e-6)
+    again = r0.clone()  # the workspace is ready for the next call, and the sums' order is fixed
+    _C.skinny_linear(x, wt, again, epilogue=_C.EPI_RESID, y_ssq=ssq, workspace=ws)
+    torch.cuda.synchronize()
+    assert torch.equal(again, r)
