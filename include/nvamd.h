@@ -344,6 +344,14 @@ int nvamd_embed_rows(const int64_t *ids, const void *table,
                      int64_t out_stride, int out_tiled, float *ssq, int rows,
                      int hidden, hipStream_t stream);
 
+/* rms_norm_tiled: out (tiled [16 * ceil(rows/16), hidden], the layout above;  */
+/*   rows past `rows` untouched) = bf16((x * rsqrt(mean(x^2) + eps)) * weight)  */
+/*   of row-major x, in fp32: a normed operand for nvamd_skinny_linear where    */
+/*   k exceeds its own prologue.  hidden % 32 == 0, hidden <= 8192.             */
+int nvamd_rms_norm_tiled(const void *x, int64_t x_stride, const void *weight,
+                         void *out, int rows, int hidden, float eps,
+                         hipStream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -71,6 +71,7 @@ _SIGNATURES = {
          _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_ptr],
     ),
     "nvamd_add_rms_norm": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_float, _c_ptr]),
+    "nvamd_rms_norm_tiled": (_c_int, [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_int, _c_int, _c_float, _c_ptr]),
     "nvamd_silu_mul": (_c_int, [_c_ptr, _c_i64, _c_ptr, _c_i64, _c_int, _c_int, _c_ptr]),
     "nvamd_argmax_rows": (_c_int, [_c_ptr, _c_i64, _c_int, _c_int, _c_ptr, _c_ptr]),
     "nvamd_skinny_linear_workspace_size": (_c_size, [_c_int, _c_int, _c_int]),
@@ -673,6 +674,24 @@ def skinny_linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = N
         out.data_ptr(), 0 if y_tiled else out.stride(0), _ptr(y_ssq), int(epilogue), flags, m, n, k,
         _ptr(workspace), workspace.numel() if workspace is not None else 0, _stream())
     _check(status, "nvamd_skinny_linear")
+    return out
+
+
+def rms_norm_tiled(x: torch.Tensor, weight: torch.Tensor, eps: float, out: torch.Tensor | None = None) -> torch.Tensor:
+    """RMSNorm of row-major [M, H] (H % 32 == 0, H <= 8192), written tiled: the operand of ``skinny_linear`` where
+    H is no width of its norm prologue.  Rounds like ``add_rms_norm``."""
+    lib = load()
+    _bf16_cuda("x", x)
+    _bf16_cuda("weight", weight)
+    _require(x.dim() == 2 and x.stride(1) == 1, "x must be [M, H] with dense rows")
+    rows, hidden = x.shape
+    _require(weight.numel() == hidden and weight.is_contiguous(), "weight must be [H]")
+    out = tiled_empty(max(rows, 1), hidden, x.device) if out is None else out
+    _require(is_tiled(out) and out.dtype == torch.bfloat16 and out.is_contiguous() and out.shape[1] * 32 == hidden
+             and 16 * out.shape[0] >= rows, "out must be tiled bf16 [M, H]")
+    status = lib.nvamd_rms_norm_tiled(x.data_ptr(), x.stride(0), weight.data_ptr(), out.data_ptr(), rows, hidden,
+                                      float(eps), _stream())
+    _check(status, "nvamd_rms_norm_tiled")
     return out
 
 

@@ -112,6 +112,47 @@ add_rms_norm_any_kernel(const u16 *__restrict__ delta, u16 *__restrict__ residua
   }
 }
 
+// RMSNorm of row-major rows, written in the skinny GEMM's tiled operand order (rows past `rows` of the last row tile
+// untouched): the norm of a decode batch whose width the GEMM's own prologue does not take.  One workgroup per row
+// of up to V * 256 vectors, for latency: at most 128 rows, each a few KB (8 x 4,096: 3.3 us).  Rounding as above.
+template <int V>
+__global__ void __launch_bounds__(256)
+rms_norm_tiled_kernel(const u16 *__restrict__ x, int64_t x_stride, const u16 *__restrict__ weight, u16 *__restrict__ out,
+                      int hidden, float eps) {
+  const int row = blockIdx.x;
+  const int tid = threadIdx.x;
+  const int vecs = hidden / 8 - tid;  // this thread's vectors: k with 256k < vecs
+  const u32x4 zero = {0u, 0u, 0u, 0u};
+  const u16 *src = x + row * x_stride + 8 * tid;
+  u32x4 v[V], w[V];
+#pragma unroll
+  for (int k = 0; k < V; ++k) v[k] = 256 * k < vecs ? ld16(src + 2048 * k) : zero;
+#pragma unroll
+  for (int k = 0; k < V; ++k) w[k] = 256 * k < vecs ? ld16(weight + 8 * tid + 2048 * k) : zero;
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < V; ++k)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float a = bf16_lo(v[k][e]), b = bf16_hi(v[k][e]);
+      ss += a * a + b * b;
+    }
+  __shared__ float s_ss[4];
+  ss = wave_sum(ss);
+  if ((tid & 63) == 0) s_ss[tid >> 6] = ss;
+  __syncthreads();
+  ss = (s_ss[0] + s_ss[1]) + (s_ss[2] + s_ss[3]);
+  const float rstd = rsqrtf(ss / (float)hidden + eps);
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    u32x4 y;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      y[e] = pack_bf16x2(bf16_lo(v[k][e]) * rstd * bf16_lo(w[k][e]), bf16_hi(v[k][e]) * rstd * bf16_hi(w[k][e]));
+    if (256 * k < vecs) st16(out + tiled_index(row, 8 * tid + 2048 * k, hidden), y);
+  }
+}
+
 // Rows too many for the caches until their next use (32 MB a tensor, half of the 256 MB Infinity Cache for
 // all four streams): nontemporal loads, and stores of the residual, whose next reader comes a
 // whole block of launches later; the normalised rows stay plain for the projection that reads them next.
@@ -281,6 +322,19 @@ extern "C" int nvamd_add_rms_norm(const void *delta, void *residual, const void 
   else
     hipLaunchKernelGGL((add_rms_norm_any_kernel<false>), grid, dim3(256), 0, stream, nullptr, r, w, o, rows, hidden,
                        eps);
+  return launch_status();
+}
+
+extern "C" int nvamd_rms_norm_tiled(const void *x, int64_t x_stride, const void *weight, void *out, int rows, int hidden,
+                                    float eps, hipStream_t stream) {
+  if (rows == 0) return NVAMD_OK;
+  if (!x || !weight || !out || rows < 0) return NVAMD_EINVAL;
+  if (hidden <= 0 || hidden % 32 != 0 || hidden > 8192) return NVAMD_EUNSUPPORTED;
+  if (!aligned16(x) || !aligned16(weight) || !aligned16(out) || x_stride < hidden || x_stride % 8) return NVAMD_EINVAL;
+  const auto kernel = hidden <= 2048 ? rms_norm_tiled_kernel<1> : hidden <= 4096 ? rms_norm_tiled_kernel<2>
+                                                                                 : rms_norm_tiled_kernel<4>;
+  hipLaunchKernelGGL(kernel, dim3(rows), dim3(256), 0, stream, static_cast<const u16 *>(x), x_stride,
+                     static_cast<const u16 *>(weight), static_cast<u16 *>(out), hidden, eps);
   return launch_status();
 }
 

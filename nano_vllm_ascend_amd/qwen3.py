@@ -13,6 +13,8 @@ skinny-M HIP GEMM runs every projection, each RMSNorm in the prologue of the GEM
 that consumes it, and each residual add in the epilogue of the GEMM that produces
 it (with the per-32-column sums of squares the next norm needs), and SiLU*mul in
 the gate/up epilogue -- 5 launches per layer instead of 9, same rounding points.
+Hidden sizes that are no multiple of 1024, or past 2048, keep the norms in launches of
+their own (``forward_decode_wide``): 7 per layer.
 That path reads tiled copies of the projection weights (the GEMM's operand order,
 built once by ``build_decode_weights``) and keeps the residual stream and the SiLU
 output tiled as well; the qkv output, the attention output and the logits stay
@@ -39,6 +41,14 @@ class CausalLMOutput:
     logits: torch.Tensor
 
 
+def _retile(tiled, weight):
+    """The weight's tiled copy, written over an earlier one of the same shape: captured graphs read that storage."""
+    new = _C.tile(weight.detach())
+    if tiled is None or tiled.shape != new.shape or tiled.device != new.device or tiled.dtype != new.dtype:
+        return new
+    return tiled.copy_(new)
+
+
 class Qwen3Attention(nn.Module):
     def __init__(self, config: Qwen3Config, layer_idx: int, block_size: int, max_model_len: int):
         super().__init__()
@@ -59,8 +69,8 @@ class Qwen3Attention(nn.Module):
         self.o_tiled = None
 
     def build_tiled(self) -> None:
-        self.qkv_tiled = _C.tile(self.qkv_weight.detach())
-        self.o_tiled = _C.tile(self.o_weight.detach())
+        self.qkv_tiled = _retile(self.qkv_tiled, self.qkv_weight)
+        self.o_tiled = _retile(self.o_tiled, self.o_weight)
 
     def forward(self, hidden_states, rotary: RotaryEmbedding, positions, kv_cache, attn_metadata, is_prefill: bool):
         t = hidden_states.shape[0]
@@ -85,6 +95,16 @@ class Qwen3Attention(nn.Module):
                                            attn_metadata.context_lens,
                                            max_context_len=getattr(attn_metadata, "max_context_bound", None),
                                            workspace=getattr(attn_metadata, "decode_workspace", None))
+
+    def decode_wide(self, x, residual, ssq, t: int, rotary, positions, kv_cache, attn_metadata, workspace):
+        """residual += o_proj(attention(qkv_proj(x))) in place for t rows: x normed and tiled, residual row-major."""
+        qkv = _C.skinny_linear(x, self.qkv_tiled, workspace=workspace, m=t)
+        q = qkv[:, : self.q_size].view(t, self.num_heads, self.head_dim)
+        k = qkv[:, self.q_size : self.q_size + self.kv_size].view(t, self.num_kv_heads, self.head_dim)
+        v = qkv[:, self.q_size + self.kv_size :].view(t, self.num_kv_heads, self.head_dim)
+        attn = self.decode_attention(q, k, v, rotary, positions, kv_cache, attn_metadata)
+        _C.skinny_linear(attn.reshape(t, self.q_size), self.o_tiled, residual, epilogue=_C.EPI_RESID, y_ssq=ssq,
+                         workspace=workspace)
 
     def decode_fused(self, residual, ssq, t: int, norm: RMSNorm, rotary, positions, kv_cache, attn_metadata,
                      workspace):
@@ -111,11 +131,16 @@ class Qwen3MLP(nn.Module):
         self.down_tiled = None
 
     def build_tiled(self) -> None:
-        self.gate_up_tiled = _C.tile(self.gate_up_weight.detach())
-        self.down_tiled = _C.tile(self.down_weight.detach())
+        self.gate_up_tiled = _retile(self.gate_up_tiled, self.gate_up_weight)
+        self.down_tiled = _retile(self.down_tiled, self.down_weight)
 
     def forward(self, x):
         return linear(gate_up_silu(x, self.gate_up_weight, self.gate_up_tiled), self.down_weight, skinny=False)
+
+    def decode_wide(self, x, residual, ssq, t: int, workspace):
+        """residual += mlp(x) in place for t rows: x normed and tiled, residual row-major."""
+        act = _C.skinny_linear(x, self.gate_up_tiled, epilogue=_C.EPI_SILU, workspace=workspace, m=t, y_tiled=True)
+        _C.skinny_linear(act, self.down_tiled, residual, epilogue=_C.EPI_RESID, y_ssq=ssq, workspace=workspace, m=t)
 
     def decode_fused(self, residual, ssq, t: int, norm: RMSNorm, workspace):
         """residual += down(silu(gate(norm(residual))) * up(norm(residual))) in place (t <= 128 rows,
@@ -179,6 +204,23 @@ class Qwen3Model(nn.Module):
             layer.mlp.decode_fused(residual, ssq, t, layer.post_attention_layernorm, workspace)
         return residual, ssq
 
+    def forward_decode_wide(self, input_ids_flat, position_ids_flat, kv_cache, attn_metadata, workspace):
+        """Decode forward for <= 128 rows at the hidden sizes that the projections' norm prologue does not take:
+        as forward_decode_fused, with each RMSNorm in a launch that writes the next projection's tiled
+        operand -- 7 launches per layer.  Returns the final residual stream, row-major."""
+        t = input_ids_flat.shape[0]
+        residual = F.embedding(input_ids_flat, self.embed_tokens)
+        ssq = torch.empty((t, residual.shape[1] // 32), dtype=torch.float32, device=residual.device)
+        for layer in self.layers:
+            norm = layer.input_layernorm
+            x = _C.rms_norm_tiled(residual, norm.weight, norm.variance_epsilon)
+            layer.self_attn.decode_wide(x, residual, ssq, t, self.rotary_emb, position_ids_flat, kv_cache,
+                                        attn_metadata, workspace)
+            norm = layer.post_attention_layernorm
+            x = _C.rms_norm_tiled(residual, norm.weight, norm.variance_epsilon)
+            layer.mlp.decode_wide(x, residual, ssq, t, workspace)
+        return residual
+
 
 class Qwen3ForCausalLM(nn.Module):
     def __init__(self, config: Qwen3Config, block_size: int = 128, max_model_len: int = 2048):
@@ -201,24 +243,46 @@ class Qwen3ForCausalLM(nn.Module):
         for layer in self.model.layers:
             layer.self_attn.build_tiled()
             layer.mlp.build_tiled()
-        self.lm_head_tiled = _C.tile(self.lm_head.detach())
+        self.lm_head_tiled = _retile(self.lm_head_tiled, self.lm_head)
         self._tiled_ready = True
-
-    def _drop_decode_weights(self) -> None:
-        """Forget the tiled copies (the weights are about to change)."""
-        for layer in self.model.layers:
-            layer.self_attn.qkv_tiled = layer.self_attn.o_tiled = None
-            layer.mlp.gate_up_tiled = layer.mlp.down_tiled = None
-        self.lm_head_tiled = None
-        self._tiled_ready = False
 
     def decode_fusable(self, rows: int) -> bool:
         """Whether a decode batch of `rows` runs on the fused skinny-GEMM path."""
         c = self.config
-        dev = self.model.embed_tokens.device
-        return (dev.type == "cuda" and 0 < rows <= _C.SKINNY_MAX_ROWS and c.hidden_size % 1024 == 0
-                and c.hidden_size <= 2048 and c.intermediate_size % 256 == 0
-                and (c.num_attention_heads * c.head_dim) % 256 == 0 and c.vocab_size % 32 == 0)
+        return self._skinny_shapes(rows) and c.hidden_size % 1024 == 0 and c.hidden_size <= 2048
+
+    def decode_wide(self, rows: int) -> bool:
+        """Whether a decode batch of `rows` runs on the skinny GEMMs with the norms in launches of their own."""
+        c = self.config
+        return (self._skinny_shapes(rows) and c.hidden_size % 256 == 0 and c.hidden_size <= 8192
+                and not (c.hidden_size % 1024 == 0 and c.hidden_size <= 2048)
+                and self.model.embed_tokens.dtype == torch.bfloat16)
+
+    def _skinny_shapes(self, rows: int) -> bool:
+        c = self.config
+        return (self.model.embed_tokens.device.type == "cuda" and 0 < rows <= _C.SKINNY_MAX_ROWS
+                and c.intermediate_size % 256 == 0 and (c.num_attention_heads * c.head_dim) % 256 == 0
+                and c.vocab_size % 32 == 0)
+
+    def _tiled_current(self) -> bool:
+        return self._tiled_ready and self.lm_head_tiled.device == self.lm_head.device
+
+    def _wide_weights_ready(self) -> bool:
+        """Build the tiled weights of a wide model if they are missing and can be: not under capture, nor when
+        the copies would leave less than a 32nd of the device's memory free (a KV pool sized to the rest of
+        it).  Without them its decode stays on the library GEMMs."""
+        if self._tiled_current():
+            return True
+        if torch.cuda.is_current_stream_capturing():
+            return False
+        dev = self.lm_head.device
+        need = sum(p.numel() for p in self.parameters()) * 2
+        free, total = torch.cuda.mem_get_info(dev)
+        free += torch.cuda.memory_reserved(dev) - torch.cuda.memory_allocated(dev)
+        if free < need + total // 32:
+            return False
+        self.build_decode_weights()
+        return True
 
     def gemm_workspace(self) -> torch.Tensor:
         """Zero-filled workspace shared by the decode projections (calls run in stream order)."""
@@ -233,8 +297,9 @@ class Qwen3ForCausalLM(nn.Module):
 
     def forward(self, input_ids_flat, position_ids_flat, kv_cache, attn_metadata, is_prefill: bool,
                 logits_indices=None) -> CausalLMOutput:
-        if not is_prefill and logits_indices is None and self.decode_fusable(input_ids_flat.shape[0]):
-            if not self._tiled_ready or self.lm_head_tiled.device != self.lm_head.device:
+        rows = input_ids_flat.shape[0]
+        if not is_prefill and logits_indices is None and self.decode_fusable(rows):
+            if not self._tiled_current():
                 self.build_decode_weights()
             ws = self.gemm_workspace()
             residual, ssq = self.model.forward_decode_fused(input_ids_flat, position_ids_flat, kv_cache,
@@ -242,18 +307,27 @@ class Qwen3ForCausalLM(nn.Module):
             norm = self.model.norm
             return CausalLMOutput(logits=_C.skinny_linear(residual, self.lm_head_tiled, x_ssq=ssq,
                                                           norm_weight=norm.weight, eps=norm.variance_epsilon,
-                                                          workspace=ws, m=input_ids_flat.shape[0]))
+                                                          workspace=ws, m=rows))
+        if not is_prefill and logits_indices is None and self.decode_wide(rows) and self._wide_weights_ready():
+            ws = self.gemm_workspace()
+            residual = self.model.forward_decode_wide(input_ids_flat, position_ids_flat, kv_cache, attn_metadata, ws)
+            norm = self.model.norm
+            if rows > 64:  # two slabs read the head's weight twice: 363 against 282 us at 128 rows x 4096
+                return CausalLMOutput(logits=linear(norm(residual), self.lm_head, skinny=False))
+            x = _C.rms_norm_tiled(residual, norm.weight, norm.variance_epsilon)
+            return CausalLMOutput(logits=_C.skinny_linear(x, self.lm_head_tiled, workspace=ws, m=rows))
         h = self.model(input_ids_flat, position_ids_flat, kv_cache, attn_metadata, is_prefill)
         if logits_indices is not None:
             h = h.index_select(0, logits_indices)
-        return CausalLMOutput(logits=linear(h, self.lm_head, tiled=self.lm_head_tiled))
+        skinny = h.shape[0] <= 64 or not self.decode_wide(h.shape[0])
+        return CausalLMOutput(logits=linear(h, self.lm_head, skinny, tiled=self.lm_head_tiled))
 
     # ---------------------------------------------------------------- weights
     @torch.no_grad()
     def init_random(self, seed: int = 0, std: float | None = None) -> None:
         """Seeded N(0, std) for every projection and the embedding, ones for every norm weight."""
         std = self.config.initializer_range if std is None else std
-        self._drop_decode_weights()
+        tiled, self._tiled_ready = self._tiled_ready, False  # the tiled copies are rewritten below
         dev = self.model.embed_tokens.device
         gen = torch.Generator(device=dev)
         gen.manual_seed(seed)
@@ -264,12 +338,14 @@ class Qwen3ForCausalLM(nn.Module):
                 tmp = torch.empty(p.shape, dtype=torch.float32, device=dev)
                 tmp.normal_(0.0, std, generator=gen)
                 p.copy_(tmp)
+        if tiled:
+            self.build_decode_weights()
 
     @torch.no_grad()
     def load_hf_state_dict(self, sd: dict) -> list[str]:
         """Copy HF Qwen3ForCausalLM weights (q/k/v and gate/up are concatenated); returns missing names."""
         missing = []
-        self._drop_decode_weights()
+        tiled, self._tiled_ready = self._tiled_ready, False  # the tiled copies are rewritten below
         m = self.model
 
         def put(dst, name):
@@ -301,6 +377,8 @@ class Qwen3ForCausalLM(nn.Module):
             put(layer.post_attention_layernorm.weight, p + "post_attention_layernorm.weight")
         if not self.config.tie_word_embeddings:
             put(self.lm_head, "lm_head.weight")
+        if tiled:
+            self.build_decode_weights()
         return missing
 
 

@@ -1,0 +1,127 @@
+"""Decode path of hidden sizes that the projections' norm prologue does not take (2560, 4096, 5120, ...)."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from nano_vllm_ascend_amd import _C
+from nano_vllm_ascend_amd.block_manager import PagedKVCacheMetadata
+from nano_vllm_ascend_amd.config import Qwen3Config
+from nano_vllm_ascend_amd.layers import RotaryEmbedding
+from nano_vllm_ascend_amd.paged_kv_cache import PagedKVCache
+from nano_vllm_ascend_amd.qwen3 import Qwen3ForCausalLM
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,hidden", [(1, 32), (5, 2016), (16, 2048), (17, 2560), (40, 4096), (33, 5120), (2, 8192)])
+def test_rms_norm_tiled_equals_row_major(device, rows, hidden):
+    """The tiled norm against add_rms_norm: the sums of squares are added in another order, so an element may round
+    to the neighbouring bf16 value (relative 2^-7)."""
+    gen = torch.Generator(device=device).manual_seed(hidden)
+    buf = torch.randn((rows, hidden + 8), generator=gen, device=device).bfloat16()
+    x, w = buf[:, :hidden], torch.randn(hidden, generator=gen, device=device).bfloat16()
+    out = _C.tiled_empty(rows, hidden, device).fill_(7.0)
+    _C.rms_norm_tiled(x, w, 1e-6, out)
+    ref = torch.empty((rows, hidden), dtype=torch.bfloat16, device=device)
+    _C.add_rms_norm(None, x.contiguous(), w, ref, 1e-6)
+    torch.cuda.synchronize()
+    full = _C.untile(out).float()
+    assert bool((full[rows:] == 7.0).all())  # padding rows untouched
+    diff = (full[:rows] - ref.float()).abs()
+    assert bool((diff <= 2.0 ** -7 * ref.float().abs()).all()) and (diff == 0).float().mean().item() > 0.99
+
+
+def _model(device, hidden, inter, heads, batch):
+    config = Qwen3Config(vocab_size=2048, hidden_size=hidden, intermediate_size=inter, num_hidden_layers=2,
+                         num_attention_heads=heads, num_key_value_heads=8)
+    with torch.device(device):
+        model = Qwen3ForCausalLM(config, 16, 512).to(torch.bfloat16)
+    model.model.rotary_emb = RotaryEmbedding(128, 512, 1e6).to(device)  # the table stays in fp32
+    model.init_random(3)
+    model.eval()
+    cache = PagedKVCache(2, batch * 4, 16, 8, 128, torch.bfloat16, device)
+    gen = torch.Generator(device=device).manual_seed(5)
+    cache.key_cache.normal_(generator=gen)
+    cache.value_cache.normal_(generator=gen)
+    lens = torch.tensor([1 + (13 * i) % 60 for i in range(batch)])
+    tables = torch.arange(batch * 4, dtype=torch.int32).view(batch, 4)
+    pos = lens - 1
+    slots = tables[torch.arange(batch), pos // 16].long() * 16 + pos % 16
+    md = PagedKVCacheMetadata(block_tables=tables.to(device), context_lens=lens.int().to(device),
+                              slot_mapping=slots.to(device), positions=pos.to(device), max_context_bound=512,
+                              decode_workspace=_C.alloc_paged_decode_workspace(batch, heads, 8, 512, device))
+    ids = torch.randint(0, 2048, (batch,), generator=gen, device=device)
+    return model, cache, md, ids
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hidden,inter,heads,batch", [(2560, 3072, 32, 7), (4096, 8192, 32, 33), (5120, 2560, 40, 16),
+                                                      (4096, 4096, 64, 70), (256, 512, 8, 1)])
+@torch.inference_mode()
+def test_wide_decode_matches_the_library_path(device, hidden, inter, heads, batch):
+    model, cache, md, ids = _model(device, hidden, inter, heads, batch)
+
+    def step():
+        return model(input_ids_flat=ids, position_ids_flat=md.positions, kv_cache=cache, attn_metadata=md,
+                     is_prefill=False).logits.float()
+
+    assert model.decode_wide(batch) and not model.decode_fusable(batch)
+    wide = step()
+    assert model.lm_head_tiled is not None
+    model.decode_wide = lambda rows: False
+    plain = step()
+    torch.cuda.synchronize()
+    # each of the 2 layers rounds its projections to bf16 six times (1.7e-3 rms each) on either path
+    assert ((wide - plain).norm() / plain.norm()).item() < 2e-2
+
+
+@pytest.mark.gpu
+@torch.inference_mode()
+def test_wide_decode_keeps_the_library_path_under_a_first_capture_and_without_room(device, monkeypatch):
+    """A capture cannot build the tiled weights, and neither can a device whose memory the KV pool fills."""
+    model, cache, md, ids = _model(device, 2560, 3072, 32, 4)
+
+    def step():
+        return model(input_ids_flat=ids, position_ids_flat=md.positions, kv_cache=cache, attn_metadata=md,
+                     is_prefill=False).logits
+
+    with monkeypatch.context() as m:
+        m.setattr(torch.cuda, "mem_get_info", lambda d=None: (0, 1 << 40))
+        eager = step().float()
+        assert model.lm_head_tiled is None
+        torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    assert model.lm_head_tiled is None
+    for _ in range(2):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.float(), eager)
+    step()
+    assert model.lm_head_tiled is not None
+
+
+@pytest.mark.gpu
+@torch.inference_mode()
+def test_new_weights_reach_captured_graphs(device):
+    """Loading weights rewrites the tiled copies in place: a graph captured before replays with the new ones."""
+    model, cache, md, ids = _model(device, 2560, 3072, 32, 4)
+
+    def step():
+        return model(input_ids_flat=ids, position_ids_flat=md.positions, kv_cache=cache, attn_metadata=md,
+                     is_prefill=False).logits
+
+    first = step().float()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    model.init_random(4)
+    for _ in range(2):
+        graph.replay()
+        torch.cuda.synchronize()
+        got = out.float()
+        eager = step().float()
+        torch.cuda.synchronize()
+        assert torch.equal(got, eager) and not torch.equal(got, first)
