@@ -214,3 +214,21 @@ def test_paged_prefill_full_prompt_equals_dense(device):
     out, qs, q, k, v, kc, vc, tables, cu_q, cu_full, sel = _paged_case(device, prompt_lens, [0, 0], seed=3)
     ref = varlen_prefill_ref(q, k, v, cu_full, SCALE)
     assert (out.float().cpu() - ref).abs().max().item() <= TOL
+
+
+@pytest.mark.gpu
+def test_dense_prefill_strided_output_writes_its_rows_only(device):
+    """Whole rows are stored from the turned-around tile: into a strided view, at lengths that end inside a wave's
+    32 rows, nothing past a prompt's last row or beside its heads is written."""
+    lens = [1, 31, 33, 70]
+    t = sum(lens)
+    gen = torch.Generator(device=device).manual_seed(4)
+    q, k, v = (rand((t, h, 128), gen, device) for h in (4, 2, 2))
+    cu = W.cu_seqlens(lens)
+    buf = torch.full((t + 2, 6 * 128), 3.0, dtype=torch.bfloat16, device=device)
+    out = buf[1 : t + 1, 128 : 5 * 128].view(t, 4, 128)
+    _C.varlen_prefill(out, q, k, v, torch.tensor(cu, dtype=torch.int32, device=device), max(lens), SCALE)
+    torch.cuda.synchronize()
+    assert (out.float().cpu() - varlen_prefill_ref(q, k, v, cu, SCALE)).abs().max().item() <= TOL
+    out.fill_(3.0)
+    assert bool((buf == 3.0).all())
