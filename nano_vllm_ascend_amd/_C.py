@@ -319,28 +319,39 @@ def paged_decode_noalloc(out: torch.Tensor, q: torch.Tensor, key_cache: torch.Te
 
 
 def _decode_args(out, q, key_cache, value_cache, block_tables, context_lens, scale, max_context_len) -> tuple:
-    """Checked arguments of the decode entry points, up to the workspace."""
-    _bf16_cuda("q", q)
-    _bf16_cuda("out", out)
-    _bf16_cuda("key_cache", key_cache)
-    _bf16_cuda("value_cache", value_cache)
-    _require(q.dim() == 3 and out.shape == q.shape,
-             lambda: f"q/out shape mismatch: {tuple(q.shape)} vs {tuple(out.shape)}")
-    _require(key_cache.dim() == 4 and key_cache.shape == value_cache.shape, "key/value cache shape mismatch")
-    _require(key_cache.is_contiguous() and value_cache.is_contiguous(), "caches must be contiguous")
-    nb, bs, hkv, d = key_cache.shape
-    b, hq, dq = q.shape
-    _require(dq == d, lambda: f"head_dim mismatch {dq} vs {d}")
-    _require(block_tables.dtype == torch.int32 and block_tables.dim() == 2 and block_tables.shape[0] == b,
-             "block_tables must be int32 [B, W]")
-    _require(block_tables.stride(1) == 1, "block_tables rows must be dense")
-    _require(context_lens.dtype == torch.int32 and context_lens.numel() == b and context_lens.is_cuda,
-             "context_lens must be int32 [B] on the device")
-    _require(context_lens.is_contiguous(), "context_lens must be contiguous")
-    if _checking():
+    """Checked arguments of the decode entry points, up to the workspace.  The checks are written out (a small
+    batch's eager decode is bound by the host: 4.7 us of a 15 us call went to them as helper calls)."""
+    for name, t in (("q", q), ("out", out), ("key_cache", key_cache), ("value_cache", value_cache)):
+        if t.dtype is not torch.bfloat16 or not t.is_cuda:
+            _bf16_cuda(name, t)  # raises
+    q_shape, kv_shape = q.shape, key_cache.shape
+    if len(q_shape) != 3 or out.shape != q_shape:
+        raise ValueError(f"q/out shape mismatch: {tuple(q_shape)} vs {tuple(out.shape)}")
+    if len(kv_shape) != 4 or value_cache.shape != kv_shape:
+        raise ValueError("key/value cache shape mismatch")
+    if not (key_cache.is_contiguous() and value_cache.is_contiguous()):
+        raise ValueError("caches must be contiguous")
+    nb, bs, hkv, d = kv_shape
+    b, hq, dq = q_shape
+    if dq != d:
+        raise ValueError(f"head_dim mismatch {dq} vs {d}")
+    bt_shape, bt_stride = block_tables.shape, block_tables.stride()
+    if block_tables.dtype is not torch.int32 or len(bt_shape) != 2 or bt_shape[0] != b:
+        raise ValueError("block_tables must be int32 [B, W]")
+    if bt_stride[1] != 1:
+        raise ValueError("block_tables rows must be dense")
+    if context_lens.dtype is not torch.int32 or context_lens.numel() != b or not context_lens.is_cuda:
+        raise ValueError("context_lens must be int32 [B] on the device")
+    if not context_lens.is_contiguous():
+        raise ValueError("context_lens must be contiguous")
+    q_stride, out_stride = q.stride(), out.stride()
+    for t, st in ((q, q_stride), (out, out_stride)):
+        if st[2] != 1 or st[1] != d:
+            raise ValueError(f"rows of {tuple(t.shape)} are not dense")
+    if _range_checks and _checking():
         check_paged_context(block_tables, context_lens, nb, bs, int(max_context_len))
-    return (out.data_ptr(), _row_stride(out), q.data_ptr(), _row_stride(q), key_cache.data_ptr(),
-            value_cache.data_ptr(), nb, bs, block_tables.data_ptr(), block_tables.stride(0), block_tables.shape[1],
+    return (out.data_ptr(), out_stride[0], q.data_ptr(), q_stride[0], key_cache.data_ptr(),
+            value_cache.data_ptr(), nb, bs, block_tables.data_ptr(), bt_stride[0], bt_shape[1],
             context_lens.data_ptr(), b, hq, hkv, d, float(scale), int(max_context_len))
 
 
@@ -356,44 +367,35 @@ def paged_decode_fused(out: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: t
     slot_mapping[i] must be the cache slot of row positions[i] of sequence i (decode metadata).
     """
     lib = load()
-    for name, t in (("q", q), ("k", k), ("v", v), ("out", out), ("key_cache", key_cache),
-                    ("value_cache", value_cache)):
-        _bf16_cuda(name, t)
-    _require(q.dim() == 3 and out.shape == q.shape,
-             lambda: f"q/out shape mismatch: {tuple(q.shape)} vs {tuple(out.shape)}")
-    _require(k.dim() == 3 and k.shape == v.shape and k.shape[0] == q.shape[0], "k/v must be [B, Hkv, D]")
-    _require(key_cache.dim() == 4 and key_cache.shape == value_cache.shape, "key/value cache shape mismatch")
-    _require(key_cache.is_contiguous() and value_cache.is_contiguous(), "caches must be contiguous")
-    nb, bs, hkv, d = key_cache.shape
-    b, hq, dq = q.shape
-    _require(dq == d and k.shape[1:] == (hkv, d),
-             lambda: f"head shape mismatch: q {tuple(q.shape)}, k {tuple(k.shape)}")
-    _require(q_weight.dtype == torch.bfloat16 and k_weight.dtype == torch.bfloat16, "norm weights must be bf16")
-    _require(q_weight.numel() == d and k_weight.numel() == d, "norm weights must have head_dim elements")
-    _require(q_weight.is_contiguous() and k_weight.is_contiguous(), "norm weights must be contiguous")
-    _require(positions.dtype == torch.int64 and positions.numel() == b and positions.is_cuda,
-             "positions must be int64 [B] on the device")
-    _require(cos_sin.dtype == torch.float32 and cos_sin.dim() == 2 and cos_sin.shape[1] == d and cos_sin.is_cuda
-             and cos_sin.is_contiguous(), "cos_sin must be contiguous fp32 [max_positions, head_dim]")
-    _require(slot_mapping.dtype == torch.int64 and slot_mapping.numel() == b and slot_mapping.is_cuda,
-             "slot_mapping must be int64 [B] on the device")
-    _require(block_tables.dtype == torch.int32 and block_tables.dim() == 2 and block_tables.shape[0] == b,
-             "block_tables must be int32 [B, W]")
-    _require(block_tables.stride(1) == 1, "block_tables rows must be dense")
-    _require(context_lens.dtype == torch.int32 and context_lens.numel() == b and context_lens.is_cuda
-             and context_lens.is_contiguous(), "context_lens must be int32 [B] on the device")
-    if _checking():
-        check_paged_context(block_tables, context_lens, nb, bs, int(max_context_len))
-        check_positions(positions, cos_sin.shape[0])
-        check_slots(slot_mapping, nb * bs)
+    args = _decode_args(out, q, key_cache, value_cache, block_tables, context_lens, scale, max_context_len)
+    for name, t in (("k", k), ("v", v)):
+        if t.dtype is not torch.bfloat16 or not t.is_cuda:
+            _bf16_cuda(name, t)  # raises
+    b, hkv, d = q.shape[0], key_cache.shape[2], key_cache.shape[3]
+    if k.shape != v.shape or k.shape != (b, hkv, d):
+        raise ValueError(f"k/v must be [B, Hkv, D] = {(b, hkv, d)}, got {tuple(k.shape)} and {tuple(v.shape)}")
+    if q_weight.dtype is not torch.bfloat16 or k_weight.dtype is not torch.bfloat16:
+        raise ValueError("norm weights must be bf16")
+    if q_weight.numel() != d or k_weight.numel() != d:
+        raise ValueError("norm weights must have head_dim elements")
+    if not (q_weight.is_contiguous() and k_weight.is_contiguous()):
+        raise ValueError("norm weights must be contiguous")
+    if positions.dtype is not torch.int64 or positions.numel() != b or not positions.is_cuda:
+        raise ValueError("positions must be int64 [B] on the device")
+    table = cos_sin.shape
+    if (cos_sin.dtype is not torch.float32 or len(table) != 2 or table[1] != d or not cos_sin.is_cuda
+            or not cos_sin.is_contiguous()):
+        raise ValueError("cos_sin must be contiguous fp32 [max_positions, head_dim]")
+    if slot_mapping.dtype is not torch.int64 or slot_mapping.numel() != b or not slot_mapping.is_cuda:
+        raise ValueError("slot_mapping must be int64 [B] on the device")
+    if _range_checks and _checking():
+        check_positions(positions, table[0])
+        check_slots(slot_mapping, key_cache.shape[0] * key_cache.shape[1])
     status = lib.nvamd_paged_decode_fused(
-        out.data_ptr(), _row_stride(out), q.data_ptr(), _row_stride(q), k.data_ptr(), _row_stride(k),
-        v.data_ptr(), _row_stride(v), q_weight.data_ptr(), k_weight.data_ptr(), positions.contiguous().data_ptr(),
-        cos_sin.data_ptr(), cos_sin.shape[0], float(eps), key_cache.data_ptr(), value_cache.data_ptr(), nb, bs,
-        slot_mapping.contiguous().data_ptr(), block_tables.data_ptr(), block_tables.stride(0),
-        block_tables.shape[1], context_lens.data_ptr(), b, hq, hkv, d, float(scale), int(max_context_len),
-        workspace.data_ptr(), workspace.numel() * workspace.element_size(), _stream(),
-    )
+        *args[:4], k.data_ptr(), _row_stride(k), v.data_ptr(), _row_stride(v), q_weight.data_ptr(),
+        k_weight.data_ptr(), positions.contiguous().data_ptr(), cos_sin.data_ptr(), table[0], float(eps), *args[4:8],
+        slot_mapping.contiguous().data_ptr(), *args[8:], workspace.data_ptr(),
+        workspace.numel() * workspace.element_size(), _stream())
     _check(status, "nvamd_paged_decode_fused")
     return out
 

@@ -101,9 +101,10 @@ class HipPagedAttention(nn.Module):
         if workspace is None:
             workspace = self.workspace(total_tokens, max_context_len, q.device)
         out = torch.empty_like(q) if out is None else out
-        return _C.paged_decode(out, q, key_cache, value_cache, block_tables, context_lens.to(torch.int32),
-                               self.scale, max_context_len, workspace)
-
+        if context_lens.dtype is not torch.int32:
+            context_lens = context_lens.to(torch.int32)
+        return _C.paged_decode(out, q, key_cache, value_cache, block_tables, context_lens, self.scale,
+                               max_context_len, workspace)
 
     def decode_step(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_norm: RMSNorm, k_norm: RMSNorm,
                     rotary: RotaryEmbedding, positions: torch.Tensor, key_cache: torch.Tensor,
@@ -123,9 +124,11 @@ class HipPagedAttention(nn.Module):
         if workspace is None:
             workspace = self.workspace(total_tokens, max_context_len, q.device)
         out = torch.empty_like(q) if out is None else out
+        if context_lens.dtype is not torch.int32:
+            context_lens = context_lens.to(torch.int32)
         return _C.paged_decode_fused(out, q, k, v, q_norm.weight, k_norm.weight, positions, rotary.cos_sin,
                                      q_norm.variance_epsilon, key_cache, value_cache, slot_mapping, block_tables,
-                                     context_lens.to(torch.int32), self.scale, max_context_len, workspace)
+                                     context_lens, self.scale, max_context_len, workspace)
 
 
 class HipBatchPrefillAttention(nn.Module):
