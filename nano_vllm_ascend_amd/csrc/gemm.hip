@@ -22,8 +22,7 @@
 //     tiles (32-row slabs where a NORM prologue's k exceeds 1024 or it feeds a residual
 //     epilogue), the slab index fastest in the grid, so the slabs reading one weight tile
 //     run side by side and its repeat reads come from the Infinity Cache; its waves split
-//     the slice again, and a wave's NT column tiles share each A fragment (64-row slabs of
-//     the vocabulary-sized projection: 64 columns per workgroup instead of 128);
+//     the slice again, and a wave's NT column tiles share each A fragment;
 //   * the waves' partial tiles meet in LDS; with KS > 1 the workgroups publish fp32
 //     partials with agent-scope write-through stores, count arrivals per column group,
 //     and the last to arrive adds the KS partials in slice order.  Every sum has a
