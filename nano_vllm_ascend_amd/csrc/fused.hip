@@ -114,7 +114,8 @@ add_rms_norm_any_kernel(const u16 *__restrict__ delta, u16 *__restrict__ residua
 
 // RMSNorm of row-major rows, written in the skinny GEMM's tiled operand order (rows past `rows` of the last row tile
 // untouched): the norm of a decode batch whose width the GEMM's own prologue does not take.  One workgroup per row
-// of up to V * 256 vectors, for latency: at most 128 rows, each a few KB (8 x 4,096: 3.3 us).  Rounding as above.
+// of up to V * 256 vectors, for latency: at most 128 rows, each a few KB (8 x 4,096 inside a decode step: 4.7 us, most of
+// it the round trip for inputs that the weight streams have pushed out of the caches).  Rounding as above.
 template <int V>
 __global__ void __launch_bounds__(256)
 rms_norm_tiled_kernel(const u16 *__restrict__ x, int64_t x_stride, const u16 *__restrict__ weight, u16 *__restrict__ out,
@@ -198,8 +199,11 @@ silu_mul_kernel(const u16 *__restrict__ gu, u16 *__restrict__ out, int rows, int
 __device__ __forceinline__ bool better(float v, int i, float bv, int bi) { return v > bv || (v == bv && i < bi); }
 
 // One 1024-thread workgroup per row.  A thread scans 16-byte vectors in increasing index
-// order, four loads in flight per step, keeping the first index of its maximum; waves then
-// reduce with shuffles and the 16 wave results meet in LDS.
+// order, four loads in flight per step, keeping the first vector that holds its maximum, and
+// looks up the element at the end; waves then reduce with shuffles and the 16 wave results meet
+// in LDS.  One CU takes a row, and half of its time is the scan's arithmetic, so an element costs
+// its unpacking and half a three-way maximum, no compare and selects: 32 rows of 151,936 8.8 us
+// against 10.1, one row 7.6 against 8.6 (7, 10 or 19 loads in flight: no change).
 constexpr int kArgmaxThreads = 1024;
 __global__ void __launch_bounds__(kArgmaxThreads)
 argmax_rows_kernel(const u16 *__restrict__ logits, int64_t row_stride, int vocab, int64_t *__restrict__ out) {
@@ -219,14 +223,22 @@ argmax_rows_kernel(const u16 *__restrict__ logits, int64_t row_stride, int vocab
       x[u] = c < vec_end ? ld16(p + c) : u32x4{0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};  // -inf
     }
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int u = 0; u < U; ++u) {
+      float m = fmaxf(bf16_lo(x[u][0]), bf16_hi(x[u][0]));
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int c = c0 + u * kStep + 2 * e;
-        const float a = bf16_lo(x[u][e]), b = bf16_hi(x[u][e]);
-        if (a > best) { best = a; best_i = c; }
-        if (b > best) { best = b; best_i = c + 1; }
-      }
+      for (int e = 1; e < 4; ++e) m = fmaxf(m, fmaxf(bf16_lo(x[u][e]), bf16_hi(x[u][e])));
+      if (m > best) { best = m; best_i = c0 + u * kStep; }
+    }
+  }
+  if (best_i != 0x7fffffff) {  // the first element of the vector that holds its maximum
+    const u32x4 x = ld16(p + best_i);
+    int at = 7;
+#pragma unroll
+    for (int e = 3; e >= 0; --e) {
+      if (bf16_hi(x[e]) == best) at = 2 * e + 1;
+      if (bf16_lo(x[e]) == best) at = 2 * e;
+    }
+    best_i += at;
   }
   for (int c = vec_end + tid; c < vocab; c += kArgmaxThreads) {
     const float a = bf16_to_f32(p[c]);
