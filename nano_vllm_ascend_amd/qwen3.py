@@ -23,6 +23,7 @@ add_rms_norm over the row-major weights.
 """
 from __future__ import annotations
 
+from contextlib import contextmanager
 from dataclasses import dataclass
 from pathlib import Path
 
@@ -41,12 +42,31 @@ class CausalLMOutput:
     logits: torch.Tensor
 
 
-def _retile(tiled, weight):
-    """The weight's tiled copy, written over an earlier one of the same shape: captured graphs read that storage."""
-    new = _C.tile(weight.detach())
-    if tiled is None or tiled.shape != new.shape or tiled.device != new.device or tiled.dtype != new.dtype:
-        return new
-    return tiled.copy_(new)
+class _TiledCopy:
+    """A weight's copy in the skinny GEMM's operand order, handed out only while it holds the weight's values."""
+
+    def __init__(self):
+        self.storage = None
+        self.current = False
+
+    def of(self, weight: torch.Tensor):
+        """The copy, or None if it is missing, dropped or on another device than the weight."""
+        return self.storage if self.current and self.storage.device == weight.device else None
+
+    def drop(self) -> None:
+        """The weight is about to change.  The storage stays: captured graphs read it, and ``build`` rewrites it."""
+        self.current = False
+
+    def build(self, weight: torch.Tensor) -> None:
+        self.current = False
+        with torch.inference_mode():  # also where the storage was made in inference mode and this call is outside it
+            new = _C.tile(weight)
+            t = self.storage
+            if t is not None and t.shape == new.shape and t.device == new.device and t.dtype == new.dtype:
+                t.copy_(new)
+            else:
+                self.storage = new
+        self.current = True
 
 
 class Qwen3Attention(nn.Module):
@@ -65,16 +85,16 @@ class Qwen3Attention(nn.Module):
         self.prefill_attn = HipBatchPrefillAttention(self.num_heads, self.num_kv_heads, self.head_dim, block_size,
                                                      max_model_len)
         self.paged_attn = HipPagedAttention(self.num_heads, self.num_kv_heads, self.head_dim)
-        self.qkv_tiled = None  # tiled copies for the fused decode path (build_tiled)
-        self.o_tiled = None
+        self.qkv_tiled = _TiledCopy()  # for the fused decode path (build_tiled)
+        self.o_tiled = _TiledCopy()
 
     def build_tiled(self) -> None:
-        self.qkv_tiled = _retile(self.qkv_tiled, self.qkv_weight)
-        self.o_tiled = _retile(self.o_tiled, self.o_weight)
+        self.qkv_tiled.build(self.qkv_weight)
+        self.o_tiled.build(self.o_weight)
 
     def forward(self, hidden_states, rotary: RotaryEmbedding, positions, kv_cache, attn_metadata, is_prefill: bool):
         t = hidden_states.shape[0]
-        qkv = linear(hidden_states, self.qkv_weight, tiled=self.qkv_tiled)
+        qkv = linear(hidden_states, self.qkv_weight, tiled=self.qkv_tiled.of(self.qkv_weight))
         q = qkv[:, : self.q_size].view(t, self.num_heads, self.head_dim)
         k = qkv[:, self.q_size : self.q_size + self.kv_size].view(t, self.num_kv_heads, self.head_dim)
         v = qkv[:, self.q_size + self.kv_size :].view(t, self.num_kv_heads, self.head_dim)
@@ -98,27 +118,27 @@ class Qwen3Attention(nn.Module):
 
     def decode_wide(self, x, residual, ssq, t: int, rotary, positions, kv_cache, attn_metadata, workspace):
         """residual += o_proj(attention(qkv_proj(x))) in place for t rows: x normed and tiled, residual row-major."""
-        qkv = _C.skinny_linear(x, self.qkv_tiled, workspace=workspace, m=t)
+        qkv = _C.skinny_linear(x, self.qkv_tiled.storage, workspace=workspace, m=t)
         q = qkv[:, : self.q_size].view(t, self.num_heads, self.head_dim)
         k = qkv[:, self.q_size : self.q_size + self.kv_size].view(t, self.num_kv_heads, self.head_dim)
         v = qkv[:, self.q_size + self.kv_size :].view(t, self.num_kv_heads, self.head_dim)
         attn = self.decode_attention(q, k, v, rotary, positions, kv_cache, attn_metadata)
-        _C.skinny_linear(attn.reshape(t, self.q_size), self.o_tiled, residual, epilogue=_C.EPI_RESID, y_ssq=ssq,
-                         workspace=workspace)
+        _C.skinny_linear(attn.reshape(t, self.q_size), self.o_tiled.storage, residual, epilogue=_C.EPI_RESID,
+                         y_ssq=ssq, workspace=workspace)
 
     def decode_fused(self, residual, ssq, t: int, norm: RMSNorm, rotary, positions, kv_cache, attn_metadata,
                      workspace):
         """residual += o_proj(attention(qkv_proj(norm(residual)))) in place, for a decode batch of
         t <= 128 rows held tiled in `residual`: the input RMSNorm runs in the qkv GEMM's prologue and
         the residual add (with the sums of squares the next norm needs) in the o_proj GEMM's epilogue."""
-        qkv = _C.skinny_linear(residual, self.qkv_tiled, x_ssq=ssq, norm_weight=norm.weight,
+        qkv = _C.skinny_linear(residual, self.qkv_tiled.storage, x_ssq=ssq, norm_weight=norm.weight,
                                eps=norm.variance_epsilon, workspace=workspace, m=t)
         q = qkv[:, : self.q_size].view(t, self.num_heads, self.head_dim)
         k = qkv[:, self.q_size : self.q_size + self.kv_size].view(t, self.num_kv_heads, self.head_dim)
         v = qkv[:, self.q_size + self.kv_size :].view(t, self.num_kv_heads, self.head_dim)
         attn = self.decode_attention(q, k, v, rotary, positions, kv_cache, attn_metadata)
-        _C.skinny_linear(attn.reshape(t, self.q_size), self.o_tiled, residual, epilogue=_C.EPI_RESID, y_ssq=ssq,
-                         workspace=workspace, y_tiled=True)
+        _C.skinny_linear(attn.reshape(t, self.q_size), self.o_tiled.storage, residual, epilogue=_C.EPI_RESID,
+                         y_ssq=ssq, workspace=workspace, y_tiled=True)
 
 
 class Qwen3MLP(nn.Module):
@@ -127,30 +147,33 @@ class Qwen3MLP(nn.Module):
         self.intermediate = config.intermediate_size
         self.gate_up_weight = nn.Parameter(torch.empty(2 * config.intermediate_size, config.hidden_size))
         self.down_weight = nn.Parameter(torch.empty(config.hidden_size, config.intermediate_size))
-        self.gate_up_tiled = None  # tiled copies for the fused decode path (build_tiled)
-        self.down_tiled = None
+        self.gate_up_tiled = _TiledCopy()  # for the fused decode path (build_tiled)
+        self.down_tiled = _TiledCopy()
 
     def build_tiled(self) -> None:
-        self.gate_up_tiled = _retile(self.gate_up_tiled, self.gate_up_weight)
-        self.down_tiled = _retile(self.down_tiled, self.down_weight)
+        self.gate_up_tiled.build(self.gate_up_weight)
+        self.down_tiled.build(self.down_weight)
 
     def forward(self, x):
-        return linear(gate_up_silu(x, self.gate_up_weight, self.gate_up_tiled), self.down_weight, skinny=False)
+        act = gate_up_silu(x, self.gate_up_weight, self.gate_up_tiled.of(self.gate_up_weight))
+        return linear(act, self.down_weight, skinny=False)
 
     def decode_wide(self, x, residual, ssq, t: int, workspace):
         """residual += mlp(x) in place for t rows: x normed and tiled, residual row-major."""
-        act = _C.skinny_linear(x, self.gate_up_tiled, epilogue=_C.EPI_SILU, workspace=workspace, m=t, y_tiled=True)
-        _C.skinny_linear(act, self.down_tiled, residual, epilogue=_C.EPI_RESID, y_ssq=ssq, workspace=workspace, m=t)
+        act = _C.skinny_linear(x, self.gate_up_tiled.storage, epilogue=_C.EPI_SILU, workspace=workspace, m=t,
+                               y_tiled=True)
+        _C.skinny_linear(act, self.down_tiled.storage, residual, epilogue=_C.EPI_RESID, y_ssq=ssq,
+                         workspace=workspace, m=t)
 
     def decode_fused(self, residual, ssq, t: int, norm: RMSNorm, workspace):
         """residual += down(silu(gate(norm(residual))) * up(norm(residual))) in place (t <= 128 rows,
         tiled): norm in the gate/up GEMM's prologue, SiLU*mul in its epilogue (written tiled), the
         residual add in the down GEMM's epilogue."""
-        act = _C.skinny_linear(residual, self.gate_up_tiled, epilogue=_C.EPI_SILU, x_ssq=ssq,
+        act = _C.skinny_linear(residual, self.gate_up_tiled.storage, epilogue=_C.EPI_SILU, x_ssq=ssq,
                                norm_weight=norm.weight, eps=norm.variance_epsilon, workspace=workspace, m=t,
                                y_tiled=True)
-        _C.skinny_linear(act, self.down_tiled, residual, epilogue=_C.EPI_RESID, y_ssq=ssq, workspace=workspace, m=t,
-                         y_tiled=True)
+        _C.skinny_linear(act, self.down_tiled.storage, residual, epilogue=_C.EPI_RESID, y_ssq=ssq,
+                         workspace=workspace, m=t, y_tiled=True)
 
 
 class Qwen3DecoderLayer(nn.Module):
@@ -231,20 +254,40 @@ class Qwen3ForCausalLM(nn.Module):
             torch.empty(config.vocab_size, config.hidden_size))
 
         self._gemm_workspace = None
-        self.lm_head_tiled = None
-        self._tiled_ready = False
+        self.lm_head_tiled = _TiledCopy()
+
+    def _drop_decode_weights(self) -> None:
+        """Use no tiled copy until the next build (the weights are about to change)."""
+        for layer in self.model.layers:
+            for copy in (layer.self_attn.qkv_tiled, layer.self_attn.o_tiled, layer.mlp.gate_up_tiled,
+                         layer.mlp.down_tiled):
+                copy.drop()
+        self.lm_head_tiled.drop()
 
     def build_decode_weights(self) -> None:
         """Tiled copies of the projection and LM head weights for the fused decode path (about the
         size of the weights again).  Built on the first fused decode; call it again after changing
         weights in place."""
-        if torch.cuda.is_current_stream_capturing():
+        if self.lm_head.is_cuda and torch.cuda.is_current_stream_capturing():
             raise RuntimeError("the tiled decode weights must be built before graph capture")
+        self._drop_decode_weights()
         for layer in self.model.layers:
             layer.self_attn.build_tiled()
             layer.mlp.build_tiled()
-        self.lm_head_tiled = _retile(self.lm_head_tiled, self.lm_head)
-        self._tiled_ready = True
+        self.lm_head_tiled.build(self.lm_head)  # last: its copy is current only if every copy is
+
+    @contextmanager
+    def _changing_weights(self):
+        """Around code that writes the weights: no tiled copy is used meanwhile, and those that were built are
+        rewritten at the end, whether or not the code raised, so that they and the captured graphs that read
+        them follow the weights."""
+        built = self.lm_head_tiled.storage
+        self._drop_decode_weights()
+        try:
+            yield
+        finally:
+            if built is not None and built.device == self.lm_head.device:
+                self.build_decode_weights()
 
     def decode_fusable(self, rows: int) -> bool:
         """Whether a decode batch of `rows` runs on the fused skinny-GEMM path."""
@@ -265,7 +308,7 @@ class Qwen3ForCausalLM(nn.Module):
                 and c.vocab_size % 32 == 0)
 
     def _tiled_current(self) -> bool:
-        return self._tiled_ready and self.lm_head_tiled.device == self.lm_head.device
+        return self.lm_head_tiled.of(self.lm_head) is not None
 
     def _wide_weights_ready(self) -> bool:
         """Build the tiled weights of a wide model if they are missing and can be: not under capture, nor when
@@ -305,7 +348,7 @@ class Qwen3ForCausalLM(nn.Module):
             residual, ssq = self.model.forward_decode_fused(input_ids_flat, position_ids_flat, kv_cache,
                                                             attn_metadata, ws)
             norm = self.model.norm
-            return CausalLMOutput(logits=_C.skinny_linear(residual, self.lm_head_tiled, x_ssq=ssq,
+            return CausalLMOutput(logits=_C.skinny_linear(residual, self.lm_head_tiled.storage, x_ssq=ssq,
                                                           norm_weight=norm.weight, eps=norm.variance_epsilon,
                                                           workspace=ws, m=rows))
         if not is_prefill and logits_indices is None and self.decode_wide(rows) and self._wide_weights_ready():
@@ -315,70 +358,66 @@ class Qwen3ForCausalLM(nn.Module):
             if rows > 64:  # two slabs read the head's weight twice: 363 against 282 us at 128 rows x 4096
                 return CausalLMOutput(logits=linear(norm(residual), self.lm_head, skinny=False))
             x = _C.rms_norm_tiled(residual, norm.weight, norm.variance_epsilon)
-            return CausalLMOutput(logits=_C.skinny_linear(x, self.lm_head_tiled, workspace=ws, m=rows))
+            return CausalLMOutput(logits=_C.skinny_linear(x, self.lm_head_tiled.storage, workspace=ws, m=rows))
         h = self.model(input_ids_flat, position_ids_flat, kv_cache, attn_metadata, is_prefill)
         if logits_indices is not None:
             h = h.index_select(0, logits_indices)
         skinny = h.shape[0] <= 64 or not self.decode_wide(h.shape[0])
-        return CausalLMOutput(logits=linear(h, self.lm_head, skinny, tiled=self.lm_head_tiled))
+        return CausalLMOutput(logits=linear(h, self.lm_head, skinny, tiled=self.lm_head_tiled.of(self.lm_head)))
 
     # ---------------------------------------------------------------- weights
     @torch.no_grad()
     def init_random(self, seed: int = 0, std: float | None = None) -> None:
         """Seeded N(0, std) for every projection and the embedding, ones for every norm weight."""
         std = self.config.initializer_range if std is None else std
-        tiled, self._tiled_ready = self._tiled_ready, False  # the tiled copies are rewritten below
-        dev = self.model.embed_tokens.device
-        gen = torch.Generator(device=dev)
-        gen.manual_seed(seed)
-        for name, p in self.named_parameters():
-            if name.endswith("norm.weight") or "layernorm" in name:
-                p.fill_(1.0)
-            else:
-                tmp = torch.empty(p.shape, dtype=torch.float32, device=dev)
-                tmp.normal_(0.0, std, generator=gen)
-                p.copy_(tmp)
-        if tiled:
-            self.build_decode_weights()
+        with self._changing_weights():
+            dev = self.model.embed_tokens.device
+            gen = torch.Generator(device=dev)
+            gen.manual_seed(seed)
+            for name, p in self.named_parameters():
+                if name.endswith("norm.weight") or "layernorm" in name:
+                    p.fill_(1.0)
+                else:
+                    tmp = torch.empty(p.shape, dtype=torch.float32, device=dev)
+                    tmp.normal_(0.0, std, generator=gen)
+                    p.copy_(tmp)
 
     @torch.no_grad()
     def load_hf_state_dict(self, sd: dict) -> list[str]:
         """Copy HF Qwen3ForCausalLM weights (q/k/v and gate/up are concatenated); returns missing names."""
         missing = []
-        tiled, self._tiled_ready = self._tiled_ready, False  # the tiled copies are rewritten below
-        m = self.model
+        with self._changing_weights():
+            m = self.model
 
-        def put(dst, name):
-            if name in sd:
-                dst.copy_(sd[name])
-            else:
-                missing.append(name)
+            def put(dst, name):
+                if name in sd:
+                    dst.copy_(sd[name])
+                else:
+                    missing.append(name)
 
-        put(m.embed_tokens, "model.embed_tokens.weight")
-        put(m.norm.weight, "model.norm.weight")
-        for i, layer in enumerate(m.layers):
-            p = f"model.layers.{i}."
-            a = layer.self_attn
-            names = [p + "self_attn.q_proj.weight", p + "self_attn.k_proj.weight", p + "self_attn.v_proj.weight"]
-            if all(n in sd for n in names):
-                a.qkv_weight.copy_(torch.cat([sd[n] for n in names], 0))
-            else:
-                missing += [n for n in names if n not in sd]
-            put(a.o_weight, p + "self_attn.o_proj.weight")
-            put(a.q_norm.weight, p + "self_attn.q_norm.weight")
-            put(a.k_norm.weight, p + "self_attn.k_norm.weight")
-            names = [p + "mlp.gate_proj.weight", p + "mlp.up_proj.weight"]
-            if all(n in sd for n in names):
-                layer.mlp.gate_up_weight.copy_(torch.cat([sd[n] for n in names], 0))
-            else:
-                missing += [n for n in names if n not in sd]
-            put(layer.mlp.down_weight, p + "mlp.down_proj.weight")
-            put(layer.input_layernorm.weight, p + "input_layernorm.weight")
-            put(layer.post_attention_layernorm.weight, p + "post_attention_layernorm.weight")
-        if not self.config.tie_word_embeddings:
-            put(self.lm_head, "lm_head.weight")
-        if tiled:
-            self.build_decode_weights()
+            put(m.embed_tokens, "model.embed_tokens.weight")
+            put(m.norm.weight, "model.norm.weight")
+            for i, layer in enumerate(m.layers):
+                p = f"model.layers.{i}."
+                a = layer.self_attn
+                names = [p + "self_attn.q_proj.weight", p + "self_attn.k_proj.weight", p + "self_attn.v_proj.weight"]
+                if all(n in sd for n in names):
+                    a.qkv_weight.copy_(torch.cat([sd[n] for n in names], 0))
+                else:
+                    missing += [n for n in names if n not in sd]
+                put(a.o_weight, p + "self_attn.o_proj.weight")
+                put(a.q_norm.weight, p + "self_attn.q_norm.weight")
+                put(a.k_norm.weight, p + "self_attn.k_norm.weight")
+                names = [p + "mlp.gate_proj.weight", p + "mlp.up_proj.weight"]
+                if all(n in sd for n in names):
+                    layer.mlp.gate_up_weight.copy_(torch.cat([sd[n] for n in names], 0))
+                else:
+                    missing += [n for n in names if n not in sd]
+                put(layer.mlp.down_weight, p + "mlp.down_proj.weight")
+                put(layer.input_layernorm.weight, p + "input_layernorm.weight")
+                put(layer.post_attention_layernorm.weight, p + "post_attention_layernorm.weight")
+            if not self.config.tie_word_embeddings:
+                put(self.lm_head, "lm_head.weight")
         return missing
 
 

@@ -67,7 +67,7 @@ def test_wide_decode_matches_the_library_path(device, hidden, inter, heads, batc
 
     assert model.decode_wide(batch) and not model.decode_fusable(batch)
     wide = step()
-    assert model.lm_head_tiled is not None
+    assert model.lm_head_tiled.of(model.lm_head) is not None
     model.decode_wide = lambda rows: False
     plain = step()
     torch.cuda.synchronize()
@@ -88,18 +88,18 @@ def test_wide_decode_keeps_the_library_path_under_a_first_capture_and_without_ro
     with monkeypatch.context() as m:
         m.setattr(torch.cuda, "mem_get_info", lambda d=None: (0, 1 << 40))
         eager = step().float()
-        assert model.lm_head_tiled is None
+        assert model.lm_head_tiled.of(model.lm_head) is None
         torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         out = step()
-    assert model.lm_head_tiled is None
+    assert model.lm_head_tiled.of(model.lm_head) is None
     for _ in range(2):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out.float(), eager)
     step()
-    assert model.lm_head_tiled is not None
+    assert model.lm_head_tiled.of(model.lm_head) is not None
 
 
 @pytest.mark.gpu
