@@ -673,7 +673,8 @@ int launch(DecodeArgs a, int batch, hipStream_t stream) {
 //        tokens per dim with v_perm: product e takes dims 8c + e as its 16 rows.  P^T needs no lane
 //        movement: its k-slots are taken in the order the S^T accumulators hold the tokens.
 // Tiles and rows past the wave's range lie past the tile's buffer range: they read zeros without a
-// memory access.  Bound by the K/V stream, as the kernel above: a group of 8 over 16 x U[512, 4096] takes 28.8 us
+// memory access, whatever bits an unwritten row of the cache holds.  The row is part of the vector offset, which
+// the range check covers; it does not cover a scalar offset.  Bound by the K/V stream, as the kernel above: a group of 8 over 16 x U[512, 4096] takes 28.8 us
 // (4.4 TB/s) where two launches over 4 heads took 63.5 us, and 100 x U[2048, 4096] 232 us (5.3 TB/s) against
 // 458; what is left over the dot-product kernel's 5.8 TB/s at 2 heads is the records' traffic.
 __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
@@ -910,7 +911,7 @@ __device__ __forceinline__ bool mfma_item(const DecodeArgs &a, const int tid, co
     for (int x = 0; x < 2; ++x)
 #pragma unroll
       for (int k = 0; k < 2; ++k)
-        kt[i][2 * x + k] = __builtin_amdgcn_raw_buffer_load_b128(rk, k_off + 128 * k, 8 * x * row_bytes, kAux);
+        kt[i][2 * x + k] = __builtin_amdgcn_raw_buffer_load_b128(rk, k_off + 8 * x * row_bytes + 128 * k, 0, kAux);
   };
   auto load_v = [&](const int h) {
 #pragma unroll
@@ -919,7 +920,7 @@ __device__ __forceinline__ bool mfma_item(const DecodeArgs &a, const int tid, co
                                                                          kBufferRsrcWord3);
 #pragma unroll
       for (int t = 0; t < 4; ++t)
-        vt[h][4 * (i & 1) + t] = __builtin_amdgcn_raw_buffer_load_b128(rv, v_off, t * row_bytes, kAux);
+        vt[h][4 * (i & 1) + t] = __builtin_amdgcn_raw_buffer_load_b128(rv, v_off + t * row_bytes, 0, kAux);
     }
   };
   auto score = [&](const int i) {

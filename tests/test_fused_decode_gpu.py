@@ -182,3 +182,25 @@ def test_fused_step_mfma_groups(device, heads, bound):
     of its own, and outside the pool's order; bounds that share merges and loop over items."""
     ctx = [1, 64, 65, 129, 200, 256, 257, 300, 777, 1023, 1025, 2100]
     check(Case(device, len(ctx), 0, 0, 128, seed=11, heads=heads, context_lens=ctx), max_ctx=bound or None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,bound", [((3, 1), 0), ((8, 2), 0), ((8, 1), 4096), ((9, 1), 0), ((16, 8), 40960)])
+def test_fused_step_mfma_ignores_stale_rows(device, heads, bound):
+    """Every row but those of earlier positions (the new token's own row too) holds NaN keys and infinite values."""
+    ctx = [*range(1, 34), *range(495, 513)] + ([*range(1007, 1025)] if bound else [])
+    case = Case(device, len(ctx), 0, 0, 16 * len(ctx), seed=5, heads=heads, bs=64, context_lens=ctx)
+    work = case.work
+    written = torch.zeros(work.key_cache.shape[1:3], dtype=torch.bool, device=device)
+    for i, c in enumerate(ctx):
+        pos = torch.arange(c - 1, device=device)
+        written[work.block_tables[i, pos // 64].long(), pos % 64] = True
+    work.key_cache[0, ~written] = float("nan")
+    work.value_cache[0, ~written] = float("inf")
+    max_ctx = bound or max(ctx)
+    out, _, _ = case.fused(max_ctx)
+    ref, _, _ = case.unfused(max_ctx)
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref)
+    err = (out.cpu().float() - case.oracle()).abs().max().item()
+    assert err <= BF16_TOL, err

@@ -315,3 +315,24 @@ def test_decode_refuses_bounds_past_the_largest(device):
     work = W.make_decode(1, 0, 0, 8, seed=1, device=device, num_heads=8, num_kv_heads=1, context_lens=[40])
     with pytest.raises(ValueError, match="unsupported"):
         run_decode(work.q, work.key_cache[0], work.value_cache[0], work.block_tables, work.context_lens, 131073)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,bound", [((3, 1), 0), ((8, 2), 0), ((10, 2), 0), ((8, 1), 0), ((9, 1), 0), ((16, 2), 4096),
+                                         ((16, 8), 40960), ((8, 8), 40960)])
+def test_decode_mfma_ignores_stale_rows(device, heads, bound):
+    """As above for the MFMA variant: contexts that end at every row of a 16-token tile, in the first and a later
+    tile of a wave and in a later partition; whole units (no bound given), split launches and loops over items."""
+    hq, hkv = heads
+    ctx = [*range(1, 34), *range(495, 513)]
+    if bound:
+        ctx += [*range(1007, 1025)]
+    work = W.make_decode(len(ctx), 0, 0, 16 * len(ctx), seed=hq, device=device, block_size=64, num_heads=hq,
+                         num_kv_heads=hkv, context_lens=ctx)
+    written = torch.zeros(work.key_cache.shape[1:3], dtype=torch.bool, device=device)
+    for i, c in enumerate(ctx):
+        pos = torch.arange(c, device=device)
+        written[work.block_tables[i, pos // 64].long(), pos % 64] = True
+    work.key_cache[0, ~written] = float("nan")
+    work.value_cache[0, ~written] = float("inf")
+    check(work, max_ctx=bound or None)
