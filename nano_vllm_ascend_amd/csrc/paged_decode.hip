@@ -949,17 +949,19 @@ __device__ __forceinline__ bool mfma_item(const DecodeArgs &a, const int tid, co
     m = cm;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      // P as a bf16 value and the bf16 of its remainder: a wave's reference is one maximum over 64 tokens, so
+      // P as its bf16 truncation and the bf16 of what that leaves: a wave's reference is one maximum over 64 tokens, so
       // P rounded once would put more error on the large weights than the kernel above does, whose 8
       // references per wave each leave the largest weight of 8 tokens exact (relative error against 64 bits over 4 x
       // U[8192, 40960]: 2.1e-3 rounded once, 1.7e-3 with the remainder, 1.9e-3 there; no difference in time).
-      // An infinity in V gives NaN.
+      // Both parts of a P > 0 are positive (a remainder of 0 becomes 1e-37, or P if that is less), so an infinity
+      // in V makes its dim infinite and not a NaN.
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int i = 2 * h + (e >> 1), x = 2 * (e & 1);
         const float p0 = fast_exp2(s[i][x] - ref), p1 = fast_exp2(s[i][x + 1] - ref);
-        pf[h][e] = pack_bf16x2(p0, p1);
-        pr[h][e] = pack_bf16x2(p0 - bf16_lo(pf[h][e]), p1 - bf16_hi(pf[h][e]));
+        pf[h][e] = pair_hi(__float_as_uint(p0), __float_as_uint(p1));
+        pr[h][e] = pack_bf16x2(__builtin_amdgcn_fmed3f(p0 - bf16_lo(pf[h][e]), 1e-37f, p0),
+                               __builtin_amdgcn_fmed3f(p1 - bf16_hi(pf[h][e]), 1e-37f, p1));
         l += p0 + p1;
       }
     }

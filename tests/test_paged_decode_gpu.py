@@ -336,3 +336,27 @@ def test_decode_mfma_ignores_stale_rows(device, heads, bound):
     work.key_cache[0, ~written] = float("nan")
     work.value_cache[0, ~written] = float("inf")
     check(work, max_ctx=bound or None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,bound", [((3, 1), 0), ((8, 2), 0), ((8, 1), 4096), ((9, 1), 0), ((16, 8), 0),
+                                         ((16, 8), 40960)])
+def test_decode_infinite_values_stay_infinite(device, heads, bound):
+    """An infinite value in a visible row makes its dim infinite (NaN where both signs meet), and no other."""
+    hq, hkv = heads
+    ctx = [1, 2, 16, 17, 64, 100, 300, 511]
+    work = W.make_decode(len(ctx), 0, 0, 64, seed=hq, device=device, num_heads=hq, num_kv_heads=hkv, context_lens=ctx)
+    vc = work.value_cache[0]
+    for i, c in enumerate(ctx):
+        for j, (t, x) in enumerate([(0, "inf"), (c - 1, "-inf"), (c // 2, "inf"), (c // 2, "-inf")]):
+            vc[int(work.block_tables[i, t // 128]), t % 128, (i + j) % hkv, (37 * i + 5 * j) % 128] = float(x)
+    both = vc[int(work.block_tables[6, 0]), :, 0, 3]  # both signs in one dim, in one tile
+    both[20], both[21] = float("inf"), float("-inf")
+    out = run_decode(work.q, work.key_cache[0], vc, work.block_tables, work.context_lens, bound or max(ctx))
+    torch.cuda.synchronize()
+    out = out.float().cpu()
+    ref = paged_decode_ref(work.q, work.key_cache[0], vc, work.block_tables, work.context_lens, SCALE)
+    finite = ref.isfinite()
+    assert bool(ref.isinf().any()) and bool(ref.isnan().any())
+    assert torch.equal(out.isnan(), ref.isnan()) and torch.equal(out[ref.isinf()], ref[ref.isinf()])
+    assert (out[finite] - ref[finite]).abs().max().item() <= TOL
