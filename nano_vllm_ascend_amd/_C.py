@@ -594,8 +594,20 @@ def skinny_linear_workspace_size(n: int, k: int, epilogue: int = EPI_STORE) -> i
     return int(load().nvamd_skinny_linear_workspace_size(n, k, epilogue))
 
 
+_SKINNY_COUNTER_BYTES = 16384  # arrival counters at the front of the workspace: the only part that has to be zero
+
+
+def alloc_skinny_workspace(shapes, device) -> torch.Tensor:
+    """A workspace for skinny projections of the given (n, k, epilogue) shapes, called one after another."""
+    need = max([skinny_linear_workspace_size(*s) for s in shapes] + [16])
+    ws = torch.empty(need, dtype=torch.uint8, device=device)
+    ws[:_SKINNY_COUNTER_BYTES].zero_()
+    return ws
+
+
 GEMM_X_TILED = 1
 GEMM_Y_TILED = 2
+GEMM_W_ROWS = 4
 
 
 def is_tiled(t: torch.Tensor) -> bool:
@@ -630,17 +642,23 @@ def tiled_empty(rows: int, cols: int, device, dtype=torch.bfloat16) -> torch.Ten
 def skinny_linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None, *, epilogue: int = EPI_STORE,
                   x_ssq: torch.Tensor | None = None, norm_weight: torch.Tensor | None = None, eps: float = 1e-6,
                   y_ssq: torch.Tensor | None = None, workspace: torch.Tensor | None = None, m: int | None = None,
-                  y_tiled: bool = False) -> torch.Tensor:
+                  y_tiled: bool = False, w_rows: bool = False) -> torch.Tensor:
     """Decode-batch projection x[M, K] @ W^T (M <= 128) with an optional RMSNorm prologue and a store,
     SiLU*mul or residual-add epilogue (one HIP launch).  Returns the output (the residual for EPI_RESID).
 
-    w is the weight tiled (``tile(W)``; SILU: the fused [2I, K] gate/up weight).  x is row-major
+    w is the weight tiled (``tile(W)``; SILU: the fused [2I, K] gate/up weight), or with ``w_rows`` the
+    contiguous [N, K] weight itself (no norm prologue).  x is row-major
     [M, K] or tiled (then ``m`` gives the valid rows); with ``y_tiled`` the output (the residual
     for EPI_RESID) is tiled with 16 * ceil(M/16) rows."""
     lib = load()
     _bf16_cuda("x", x)
     _bf16_cuda("w", w)
-    _require(is_tiled(w), "w must be tiled: tile(W)")
+    if w_rows:
+        _require(w.dim() == 2 and w.is_contiguous(), "w must be a contiguous [N, K] matrix")
+        wn, wk = w.shape
+    else:
+        _require(is_tiled(w), "w must be tiled: tile(W)")
+        wn, wk = 16 * w.shape[0], 32 * w.shape[1]
     x_tiled = is_tiled(x)
     if x_tiled:
         _require(m is not None and 0 <= m <= 16 * x.shape[0], "a tiled x needs m <= its padded rows")
@@ -648,8 +666,8 @@ def skinny_linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = N
         k = 32 * x.shape[1]
     else:
         m, k = x.shape
-    _require(32 * w.shape[1] == k, "w must be tiled [N/16, K/32, 512]")
-    n = 8 * w.shape[0] if epilogue == EPI_SILU else 16 * w.shape[0]
+    _require(wk == k, "w must be [N, K], tiled [N/16, K/32, 512]")
+    n = wn // 2 if epilogue == EPI_SILU else wn
     if epilogue == EPI_RESID:
         _require(out is not None, "the residual epilogue updates `out` in place")
         _require(y_ssq is not None and y_ssq.dtype == torch.float32 and y_ssq.is_contiguous()
@@ -670,7 +688,7 @@ def skinny_linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = N
     need = skinny_linear_workspace_size(n, k, epilogue) if n % 32 == 0 and k % 256 == 0 else 0
     if need and workspace is None:
         workspace = torch.zeros(need, dtype=torch.uint8, device=x.device)
-    flags = (GEMM_X_TILED if x_tiled else 0) | (GEMM_Y_TILED if y_tiled else 0)
+    flags = (GEMM_X_TILED if x_tiled else 0) | (GEMM_Y_TILED if y_tiled else 0) | (GEMM_W_ROWS if w_rows else 0)
     status = lib.nvamd_skinny_linear(
         x.data_ptr(), 0 if x_tiled else _row_stride(x), _ptr(x_ssq), _ptr(norm_weight), float(eps), w.data_ptr(),
         out.data_ptr(), 0 if y_tiled else out.stride(0), _ptr(y_ssq), int(epilogue), flags, m, n, k,

@@ -14,7 +14,8 @@
 //     instruction reads 1 KB of contiguous memory.  Against row-major operands (16 rows x
 //     64 bytes per instruction) this halves the vector L1 accesses that bound the
 //     M = 32 projections (inside the decode step: qkv 7.0 -> 6.1 us, gate/up 8.3 -> 7.3 us).
-//     Row-major X rows past M repeat row M-1;
+//     W may also stay row-major (W_ROWS: a weight that other code changes, or that is too large to
+//     hold twice): 10-30% slower on the stream.  Row-major X rows past M repeat row M-1;
 //     a tiled X holds 16 * ceil(M/16) rows, and rows past M only reach dropped outputs;
 //   * a workgroup of NW waves owns 16*NT output columns, one of KS slices of K
 //     (split-K across workgroups where the column count alone gives too few
@@ -38,6 +39,8 @@
 // of squares for the next NORM prologue.
 #include "common.h"
 
+#include <algorithm>
+
 namespace nvamd {
 namespace {
 
@@ -57,7 +60,7 @@ struct GemmArgs {
   const float *x_ssq;       // NORM: [m][k / 32]
   const u16 *norm_w;        // NORM: [k]
   float eps;
-  const u16 *w;             // tiled [n (SILU: 2n), k]
+  const u16 *w;             // [n (SILU: 2n), k], tiled or (W_ROWS) row-major
   u16 *y;                   // STORE / SILU output; RESID: the residual, updated in place
   int64_t y_stride;         // row-major Y
   bool x_tiled;
@@ -101,7 +104,7 @@ __device__ __forceinline__ void mfma_step(f32x4 (&acc)[NACC][MT], const u32x4 (&
                                                           __builtin_bit_cast(bf16x8v, wv[t]), acc[t][mt], 0, 0, 0);
 }
 
-template <int NW, int KB, int NT, int MT, int EPI, bool NORM, bool SLABS>
+template <int NW, int KB, int NT, int MT, int EPI, bool NORM, bool SLABS, bool W_ROWS>
 __global__ void __launch_bounds__(NW * 64)
 skinny_gemm_kernel(GemmArgs a) {
   constexpr int kNW = NW;
@@ -156,10 +159,11 @@ skinny_gemm_kernel(GemmArgs a) {
     xp[mt] = a.x_tiled ? a.x + (int64_t)mt_x * (a.k >> 5) * 512 + 8 * lane : a.x + (int64_t)xr[mt] * a.x_stride + 8 * g;
   }
   const u16 *wp[NACC];
+  constexpr int ws = W_ROWS ? 1 : 16;
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    wp[t] = a.w + (int64_t)(group * NT + t) * (a.k >> 5) * 512 + 8 * lane;
-    if (EPI == kEpiSilu) wp[NT + t] = wp[t] + (int64_t)(a.n >> 4) * (a.k >> 5) * 512;
+  for (int t = 0; t < NT; ++t) {  // 16 rows of W are 16 k elements in either layout
+    wp[t] = a.w + (int64_t)(group * NT + t) * 16 * a.k + (W_ROWS ? (int64_t)n * a.k + 8 * g : 8 * lane);
+    if (EPI == kEpiSilu) wp[NT + t] = wp[t] + (int64_t)a.n * a.k;
   }
   const u16 *np = NORM ? a.norm_w + 8 * g : nullptr;
 
@@ -217,7 +221,7 @@ skinny_gemm_kernel(GemmArgs a) {
 #pragma unroll
     for (int b = 0; b < KB; ++b) {
 #pragma unroll
-      for (int t = 0; t < NACC; ++t) wv[b][t] = ld16(wp[t] + (int64_t)(k0 + 32 * b) * 16);
+      for (int t = 0; t < NACC; ++t) wv[b][t] = ld16(wp[t] + (int64_t)(k0 + 32 * b) * ws);
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) xv[b][mt] = ld16(xp[mt] + (int64_t)(k0 + 32 * b) * xs);
       if (NORM) nv[b] = ld16(np + k0 + 32 * b);
@@ -376,8 +380,24 @@ struct Plan {
 //   * otherwise (qkv): 16 columns per 8-wave workgroup, 32 from N = 6,144 on (6,144 x 4,096 at M = 8 / 32: 11.4 / 13.5
 //     against 13.6 / 17.5) and above 64 rows, halving the X reads per weight byte (normed, K = 2,048 at
 //     M = 100: 13.6 against 20.3).
-Plan make_plan(int n, int k, int epi, int m, bool wide) {
+//   * row-major W (W_ROWS; 16 rows x 64 bytes per load instruction), M = 8 / 32: gate_up from N = 8,192 on 16 columns per 4-wave
+//     workgroup, 256 bytes of a row per wave and round (12,288 x 4,096 41.6 / 45.9 against 43.7 / 50.0 with 128 bytes
+//     of 8 waves, 9,728 x 2,560 26.4 / 31.2 against 29.0 / 33.3); residual projections 4 waves, split to >= 512 workgroups of >=
+//     512 K (4,096 x 4,096 12.0 / 12.6 against 13.5 / 15.9 unsplit of 8 waves, 2,560 x 9,728 14.9 / 18.0 against
+//     16.6 / 20.5 at 160 of 8, 5,120 x 17,408 45.8 / 54.5 against 54.4 / 63.9 unsplit); others as tiled.
+Plan make_plan(int n, int k, int epi, int m, bool wide, bool w_rows) {
   Plan p{8, 1, 1, k % 512 == 0 ? 2 : 1};
+  static const int kSlices[] = {1, 2, 3, 4, 6, 8, 12, 16};
+  auto whole = [&](int ks) { return k % ks == 0 && (k / ks) % 64 == 0; };  // 64-wide wave blocks
+  if (w_rows && epi == kEpiResid) {
+    p = Plan{4, 2, 1, 1};
+    for (int ks : kSlices) {
+      if (n / 32 * p.ks >= 512 || k / ks < 512) break;
+      if (whole(ks)) p.ks = ks;
+    }
+    return p;
+  }
+  if (w_rows && epi == kEpiSilu && n >= 8192) return Plan{4, m > 32 ? 2 : 1, 1, 4};
   if (epi == kEpiStore && n % 128 == 0 && n / 128 >= 512) {
     if (wide) return Plan{4, 4, 1, 2};
     return m <= 16 ? Plan{8, 2, 1, 2} : Plan{8, 4, 1, 1};
@@ -385,8 +405,6 @@ Plan make_plan(int n, int k, int epi, int m, bool wide) {
   if (epi == kEpiResid) {
     p = Plan{8, 2, 1, 2};
     const int groups = n / 32;
-    static const int kSlices[] = {1, 2, 3, 4, 6, 8, 12, 16};
-    auto whole = [&](int ks) { return k % ks == 0 && (k / ks) % 64 == 0; };  // 64-wide wave blocks
     for (int ks : kSlices) {
       if (!whole(ks)) continue;
       p.ks = ks;
@@ -431,51 +449,61 @@ bool wide_rows(int m, int k, bool norm, int epi) {
 template <int NW, int NT, int EPI, bool NORM>
 constexpr bool kWideBuilt = (NT <= 2 || NW == 4) && !(NORM && EPI == kEpiResid);
 
-template <int NW, int KB, int NT, int EPI, bool NORM>
+template <int NW, int KB, int NT, int EPI, bool NORM, bool W_ROWS>
 int launch(const GemmArgs &a, int grid, bool wide, hipStream_t stream) {
   if (wide) {
     if constexpr (kWideBuilt<NW, NT, EPI, NORM>) {
       if (a.m <= 64)
-        hipLaunchKernelGGL((skinny_gemm_kernel<NW, KB, NT, 4, EPI, NORM, false>), dim3(grid), dim3(NW * 64), 0,
+        hipLaunchKernelGGL((skinny_gemm_kernel<NW, KB, NT, 4, EPI, NORM, false, W_ROWS>), dim3(grid), dim3(NW * 64), 0,
                            stream, a);
       else
-        hipLaunchKernelGGL((skinny_gemm_kernel<NW, KB, NT, 4, EPI, NORM, true>), dim3(grid), dim3(NW * 64), 0,
+        hipLaunchKernelGGL((skinny_gemm_kernel<NW, KB, NT, 4, EPI, NORM, true, W_ROWS>), dim3(grid), dim3(NW * 64), 0,
                            stream, a);
     } else {
       return NVAMD_EUNSUPPORTED;
     }
   } else if (a.m > 32)
-    hipLaunchKernelGGL((skinny_gemm_kernel<NW, KB, NT, 2, EPI, NORM, true>), dim3(grid), dim3(NW * 64), 0, stream,
+    hipLaunchKernelGGL((skinny_gemm_kernel<NW, KB, NT, 2, EPI, NORM, true, W_ROWS>), dim3(grid), dim3(NW * 64), 0, stream,
                        a);
   else if (a.m > 16)
-    hipLaunchKernelGGL((skinny_gemm_kernel<NW, KB, NT, 2, EPI, NORM, false>), dim3(grid), dim3(NW * 64), 0, stream,
+    hipLaunchKernelGGL((skinny_gemm_kernel<NW, KB, NT, 2, EPI, NORM, false, W_ROWS>), dim3(grid), dim3(NW * 64), 0, stream,
                        a);
   else
-    hipLaunchKernelGGL((skinny_gemm_kernel<NW, KB, NT, 1, EPI, NORM, false>), dim3(grid), dim3(NW * 64), 0, stream,
+    hipLaunchKernelGGL((skinny_gemm_kernel<NW, KB, NT, 1, EPI, NORM, false, W_ROWS>), dim3(grid), dim3(NW * 64), 0, stream,
                        a);
   return launch_status();
 }
 
-template <int NW, int NT, int EPI, bool NORM>
+template <int NW, int NT, int EPI, bool NORM, bool W_ROWS>
 int launch_kb(const GemmArgs &a, const Plan &p, int grid, bool wide, hipStream_t stream) {
-  return p.kb == 2 ? launch<NW, 2, NT, EPI, NORM>(a, grid, wide, stream)
-                   : launch<NW, 1, NT, EPI, NORM>(a, grid, wide, stream);
+  if constexpr (W_ROWS && EPI == kEpiSilu && NW == 4)
+    if (p.kb == 4) return launch<NW, 4, NT, EPI, NORM, W_ROWS>(a, grid, wide, stream);
+  return p.kb == 2 ? launch<NW, 2, NT, EPI, NORM, W_ROWS>(a, grid, wide, stream)
+                   : launch<NW, 1, NT, EPI, NORM, W_ROWS>(a, grid, wide, stream);
 }
 
-template <int EPI, bool NORM>
+template <int EPI, bool NORM, bool W_ROWS>
 int dispatch(const GemmArgs &a, const Plan &p, int grid, bool wide, hipStream_t stream) {
   if constexpr (EPI == kEpiStore) {
-    if (p.nw == 4 && p.nt == 4) return launch_kb<4, 4, EPI, NORM>(a, p, grid, wide, stream);
-    if (p.nw == 8 && p.nt == 4) return launch_kb<8, 4, EPI, NORM>(a, p, grid, wide, stream);
+    if (p.nw == 4 && p.nt == 4) return launch_kb<4, 4, EPI, NORM, W_ROWS>(a, p, grid, wide, stream);
+    if (p.nw == 8 && p.nt == 4) return launch_kb<8, 4, EPI, NORM, W_ROWS>(a, p, grid, wide, stream);
   } else if constexpr (EPI == kEpiSilu) {
-    if (p.nw == 4 && p.nt == 1) return launch_kb<4, 1, EPI, NORM>(a, p, grid, wide, stream);
+    if (p.nw == 4 && p.nt == 1) return launch_kb<4, 1, EPI, NORM, W_ROWS>(a, p, grid, wide, stream);
   }
   if constexpr (EPI != kEpiResid) {
-    if (p.nw == 8 && p.nt == 1) return launch_kb<8, 1, EPI, NORM>(a, p, grid, wide, stream);
+    if (p.nw == 8 && p.nt == 1) return launch_kb<8, 1, EPI, NORM, W_ROWS>(a, p, grid, wide, stream);
   }
-  if (p.nw == 4 && p.nt == 2) return launch_kb<4, 2, EPI, NORM>(a, p, grid, wide, stream);
-  if (p.nw == 8 && p.nt == 2) return launch_kb<8, 2, EPI, NORM>(a, p, grid, wide, stream);
+  if (p.nw == 4 && p.nt == 2) return launch_kb<4, 2, EPI, NORM, W_ROWS>(a, p, grid, wide, stream);
+  if (p.nw == 8 && p.nt == 2) return launch_kb<8, 2, EPI, NORM, W_ROWS>(a, p, grid, wide, stream);
   return NVAMD_EUNSUPPORTED;
+}
+
+template <int EPI>
+int dispatch_layout(const GemmArgs &a, const Plan &p, int grid, bool wide, int flags, hipStream_t stream) {
+  const bool norm = a.x_ssq != nullptr;
+  if (flags & NVAMD_GEMM_W_ROWS)  // no NORM prologue (refused before)
+    return dispatch<EPI, false, true>(a, p, grid, wide, stream);
+  return norm ? dispatch<EPI, true, false>(a, p, grid, wide, stream) : dispatch<EPI, false, false>(a, p, grid, wide, stream);
 }
 
 }  // namespace
@@ -485,10 +513,11 @@ using namespace nvamd;
 
 extern "C" size_t nvamd_skinny_linear_workspace_size(int n, int k, int epilogue) {
   if (n <= 0 || k <= 0 || n % 32 || k % 256 || epilogue < 0 || epilogue > 2) return 0;
-  // the larger of the two plans' needs (the row count is not known here)
-  const size_t slabs = workspace_bytes_for(make_plan(n, k, epilogue, 32, false), n, epilogue);
-  const size_t wide = workspace_bytes_for(make_plan(n, k, epilogue, 128, true), n, epilogue);
-  return slabs > wide ? slabs : wide;
+  // the largest of the plans' needs (the row count and the weight's layout are not known here)
+  const size_t slabs = workspace_bytes_for(make_plan(n, k, epilogue, 32, false, false), n, epilogue);
+  const size_t wide = workspace_bytes_for(make_plan(n, k, epilogue, 128, true, false), n, epilogue);
+  const size_t rows = workspace_bytes_for(make_plan(n, k, epilogue, 32, false, true), n, epilogue);
+  return std::max({slabs, wide, rows});
 }
 
 extern "C" int nvamd_skinny_linear(const void *x, int64_t x_stride, const float *x_ssq, const void *norm_weight,
@@ -497,20 +526,20 @@ extern "C" int nvamd_skinny_linear(const void *x, int64_t x_stride, const float 
                                    size_t workspace_bytes, hipStream_t stream) {
   if (m == 0) return NVAMD_OK;
   if (!x || !w_tiled || !y || m < 0 || n <= 0 || k <= 0 || epilogue < 0 || epilogue > 2 ||
-      (flags & ~(NVAMD_GEMM_X_TILED | NVAMD_GEMM_Y_TILED)))
+      (flags & ~(NVAMD_GEMM_X_TILED | NVAMD_GEMM_Y_TILED | NVAMD_GEMM_W_ROWS)))
     return NVAMD_EINVAL;
   if (m > 32 * kMaxSlabs || n % 32 != 0 || k % 256 != 0) return NVAMD_EUNSUPPORTED;
   const bool x_tiled = flags & NVAMD_GEMM_X_TILED, y_tiled = flags & NVAMD_GEMM_Y_TILED;
   const bool norm = x_ssq != nullptr;
   if (norm && !norm_weight) return NVAMD_EINVAL;
-  if (norm && k > kMaxNormK) return NVAMD_EUNSUPPORTED;
+  if (norm && (k > kMaxNormK || (flags & NVAMD_GEMM_W_ROWS))) return NVAMD_EUNSUPPORTED;
   if (epilogue == kEpiResid && !y_ssq) return NVAMD_EINVAL;
   if (!aligned16(x) || !aligned16(w_tiled) || (reinterpret_cast<uintptr_t>(y) & 7u) ||
       (!x_tiled && (x_stride % 8 || x_stride < k)) || (!y_tiled && (y_stride < n || y_stride % 4)) ||
       (norm && (!aligned16(x_ssq) || !aligned16(norm_weight))))
     return NVAMD_EINVAL;
   const bool wide = wide_rows(m, k, norm, epilogue);
-  const Plan p = make_plan(n, k, epilogue, m, wide);
+  const Plan p = make_plan(n, k, epilogue, m, wide, flags & NVAMD_GEMM_W_ROWS);
   const int groups = n / (16 * p.nt);
   if ((k / p.ks) % (32 * p.kb) != 0) return NVAMD_EUNSUPPORTED;  // whole wave blocks per slice
   const int slabs = wide ? (m + 63) / 64 : (m + 31) / 32;
@@ -540,11 +569,8 @@ extern "C" int nvamd_skinny_linear(const void *x, int64_t x_stride, const float 
   a.partials = workspace ? reinterpret_cast<float *>(static_cast<char *>(workspace) + kCounterBytes) : nullptr;
   const int grid = groups * p.ks * slabs;
   switch (epilogue) {
-    case kEpiSilu:
-      return norm ? dispatch<kEpiSilu, true>(a, p, grid, wide, stream) : dispatch<kEpiSilu, false>(a, p, grid, wide, stream);
-    case kEpiResid:
-      return norm ? dispatch<kEpiResid, true>(a, p, grid, wide, stream) : dispatch<kEpiResid, false>(a, p, grid, wide, stream);
-    default:
-      return norm ? dispatch<kEpiStore, true>(a, p, grid, wide, stream) : dispatch<kEpiStore, false>(a, p, grid, wide, stream);
+    case kEpiSilu: return dispatch_layout<kEpiSilu>(a, p, grid, wide, flags, stream);
+    case kEpiResid: return dispatch_layout<kEpiResid>(a, p, grid, wide, flags, stream);
+    default: return dispatch_layout<kEpiStore>(a, p, grid, wide, flags, stream);
   }
 }

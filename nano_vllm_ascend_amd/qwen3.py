@@ -13,13 +13,13 @@ skinny-M HIP GEMM runs every projection, each RMSNorm in the prologue of the GEM
 that consumes it, and each residual add in the epilogue of the GEMM that produces
 it (with the per-32-column sums of squares the next norm needs), and SiLU*mul in
 the gate/up epilogue -- 5 launches per layer instead of 9, same rounding points.
-Hidden sizes that are no multiple of 1024, or past 2048, keep the norms in launches of
-their own (``forward_decode_wide``): 7 per layer.
 That path reads tiled copies of the projection weights (the GEMM's operand order,
 built once by ``build_decode_weights``) and keeps the residual stream and the SiLU
 output tiled as well; the qkv output, the attention output and the logits stay
-row-major.  Prefill and larger batches run the unfused chain on hipBLASLt +
-add_rms_norm over the row-major weights.
+row-major.  Batches of <= 32 rows at hidden sizes that are no multiple of 1024, or
+past 2048, run the same GEMMs over the weights themselves, with the norms in launches
+of their own (``forward_decode_wide``): 7 per layer.  Prefill and larger batches run
+the unfused chain on hipBLASLt + add_rms_norm over the row-major weights.
 """
 from __future__ import annotations
 
@@ -117,14 +117,15 @@ class Qwen3Attention(nn.Module):
                                            workspace=getattr(attn_metadata, "decode_workspace", None))
 
     def decode_wide(self, x, residual, ssq, t: int, rotary, positions, kv_cache, attn_metadata, workspace):
-        """residual += o_proj(attention(qkv_proj(x))) in place for t rows: x normed and tiled, residual row-major."""
-        qkv = _C.skinny_linear(x, self.qkv_tiled.storage, workspace=workspace, m=t)
+        """residual += o_proj(attention(qkv_proj(x))) in place for t rows: x normed and tiled, residual and weights
+        row-major."""
+        qkv = _C.skinny_linear(x, self.qkv_weight, workspace=workspace, m=t, w_rows=True)
         q = qkv[:, : self.q_size].view(t, self.num_heads, self.head_dim)
         k = qkv[:, self.q_size : self.q_size + self.kv_size].view(t, self.num_kv_heads, self.head_dim)
         v = qkv[:, self.q_size + self.kv_size :].view(t, self.num_kv_heads, self.head_dim)
         attn = self.decode_attention(q, k, v, rotary, positions, kv_cache, attn_metadata)
-        _C.skinny_linear(attn.reshape(t, self.q_size), self.o_tiled.storage, residual, epilogue=_C.EPI_RESID,
-                         y_ssq=ssq, workspace=workspace)
+        _C.skinny_linear(attn.reshape(t, self.q_size), self.o_weight, residual, epilogue=_C.EPI_RESID, y_ssq=ssq,
+                         workspace=workspace, w_rows=True)
 
     def decode_fused(self, residual, ssq, t: int, norm: RMSNorm, rotary, positions, kv_cache, attn_metadata,
                      workspace):
@@ -159,11 +160,11 @@ class Qwen3MLP(nn.Module):
         return linear(act, self.down_weight, skinny=False)
 
     def decode_wide(self, x, residual, ssq, t: int, workspace):
-        """residual += mlp(x) in place for t rows: x normed and tiled, residual row-major."""
-        act = _C.skinny_linear(x, self.gate_up_tiled.storage, epilogue=_C.EPI_SILU, workspace=workspace, m=t,
-                               y_tiled=True)
-        _C.skinny_linear(act, self.down_tiled.storage, residual, epilogue=_C.EPI_RESID, y_ssq=ssq,
-                         workspace=workspace, m=t)
+        """residual += mlp(x) in place for t rows: x normed and tiled, residual and weights row-major."""
+        act = _C.skinny_linear(x, self.gate_up_weight, epilogue=_C.EPI_SILU, workspace=workspace, m=t, y_tiled=True,
+                               w_rows=True)
+        _C.skinny_linear(act, self.down_weight, residual, epilogue=_C.EPI_RESID, y_ssq=ssq, workspace=workspace, m=t,
+                         w_rows=True)
 
     def decode_fused(self, residual, ssq, t: int, norm: RMSNorm, workspace):
         """residual += down(silu(gate(norm(residual))) * up(norm(residual))) in place (t <= 128 rows,
@@ -228,9 +229,9 @@ class Qwen3Model(nn.Module):
         return residual, ssq
 
     def forward_decode_wide(self, input_ids_flat, position_ids_flat, kv_cache, attn_metadata, workspace):
-        """Decode forward for <= 128 rows at the hidden sizes that the projections' norm prologue does not take:
-        as forward_decode_fused, with each RMSNorm in a launch that writes the next projection's tiled
-        operand -- 7 launches per layer.  Returns the final residual stream, row-major."""
+        """Decode forward for <= 32 rows at the hidden sizes that the projections' norm prologue does not take:
+        as forward_decode_fused, over the weights themselves, with each RMSNorm in a launch that writes the next
+        projection's tiled operand -- 7 launches per layer.  Returns the final residual stream, row-major."""
         t = input_ids_flat.shape[0]
         residual = F.embedding(input_ids_flat, self.embed_tokens)
         ssq = torch.empty((t, residual.shape[1] // 32), dtype=torch.float32, device=residual.device)
@@ -295,11 +296,18 @@ class Qwen3ForCausalLM(nn.Module):
         return self._skinny_shapes(rows) and c.hidden_size % 1024 == 0 and c.hidden_size <= 2048
 
     def decode_wide(self, rows: int) -> bool:
-        """Whether a decode batch of `rows` runs on the skinny GEMMs with the norms in launches of their own."""
+        """Whether a decode batch of `rows` runs on the skinny GEMMs with the norms in launches of their own, reading
+        the weights as they are.  Up to 32 rows it leads the library GEMMs and separate SiLU (a layer's projections of
+        hidden 4096, 8 / 32 rows: 92 / 101 against 101 / 108 us; 2560: 63 / 71 against 96 / 76); a row-major weight
+        streams 10-30% slower than a tiled copy, which would double the weights' memory and would have to follow
+        every change of the weights."""
         c = self.config
-        return (self._skinny_shapes(rows) and c.hidden_size % 256 == 0 and c.hidden_size <= 8192
+        return (rows <= 32 and self._skinny_shapes(rows) and c.hidden_size % 256 == 0 and c.hidden_size <= 8192
                 and not (c.hidden_size % 1024 == 0 and c.hidden_size <= 2048)
-                and self.model.embed_tokens.dtype == torch.bfloat16)
+                and all(w.dtype is torch.bfloat16 and w.is_contiguous() and w.data_ptr() % 16 == 0
+                        for layer in self.model.layers
+                        for w in (layer.self_attn.qkv_weight, layer.self_attn.o_weight, layer.mlp.gate_up_weight,
+                                  layer.mlp.down_weight)))
 
     def _skinny_shapes(self, rows: int) -> bool:
         c = self.config
@@ -307,42 +315,24 @@ class Qwen3ForCausalLM(nn.Module):
                 and c.intermediate_size % 256 == 0 and (c.num_attention_heads * c.head_dim) % 256 == 0
                 and c.vocab_size % 32 == 0)
 
-    def _tiled_current(self) -> bool:
-        return self.lm_head_tiled.of(self.lm_head) is not None
-
-    def _wide_weights_ready(self) -> bool:
-        """Build the tiled weights of a wide model if they are missing and can be: not under capture, nor when
-        the copies would leave less than a 32nd of the device's memory free (a KV pool sized to the rest of
-        it).  Without them its decode stays on the library GEMMs."""
-        if self._tiled_current():
-            return True
-        if torch.cuda.is_current_stream_capturing():
-            return False
-        dev = self.lm_head.device
-        need = sum(p.numel() for p in self.parameters()) * 2
-        free, total = torch.cuda.mem_get_info(dev)
-        free += torch.cuda.memory_reserved(dev) - torch.cuda.memory_allocated(dev)
-        if free < need + total // 32:
-            return False
-        self.build_decode_weights()
-        return True
+    def _gemm_shapes(self) -> list[tuple[int, int, int]]:
+        """(N, K, epilogue) of the decode projections that may split K."""
+        c = self.config
+        h, i, q = c.hidden_size, c.intermediate_size, c.num_attention_heads * c.head_dim
+        return [(h, q, _C.EPI_RESID), (h, i, _C.EPI_RESID), (i, h, _C.EPI_SILU),
+                (q + 2 * c.num_key_value_heads * c.head_dim, h, _C.EPI_STORE), (c.vocab_size, h, _C.EPI_STORE)]
 
     def gemm_workspace(self) -> torch.Tensor:
         """Zero-filled workspace shared by the decode projections (calls run in stream order)."""
         if self._gemm_workspace is None:
-            c = self.config
-            h, i, q = c.hidden_size, c.intermediate_size, c.num_attention_heads * c.head_dim
-            shapes = [(h, q, _C.EPI_RESID), (h, i, _C.EPI_RESID), (i, h, _C.EPI_SILU),
-                      (q + 2 * c.num_key_value_heads * c.head_dim, h, _C.EPI_STORE), (c.vocab_size, h, _C.EPI_STORE)]
-            need = max([_C.skinny_linear_workspace_size(n, k, e) for n, k, e in shapes] + [16])
-            self._gemm_workspace = torch.zeros(need, dtype=torch.uint8, device=self.model.embed_tokens.device)
+            self._gemm_workspace = _C.alloc_skinny_workspace(self._gemm_shapes(), self.model.embed_tokens.device)
         return self._gemm_workspace
 
     def forward(self, input_ids_flat, position_ids_flat, kv_cache, attn_metadata, is_prefill: bool,
                 logits_indices=None) -> CausalLMOutput:
         rows = input_ids_flat.shape[0]
         if not is_prefill and logits_indices is None and self.decode_fusable(rows):
-            if not self._tiled_current():
+            if self.lm_head_tiled.of(self.lm_head) is None:
                 self.build_decode_weights()
             ws = self.gemm_workspace()
             residual, ssq = self.model.forward_decode_fused(input_ids_flat, position_ids_flat, kv_cache,
@@ -351,19 +341,16 @@ class Qwen3ForCausalLM(nn.Module):
             return CausalLMOutput(logits=_C.skinny_linear(residual, self.lm_head_tiled.storage, x_ssq=ssq,
                                                           norm_weight=norm.weight, eps=norm.variance_epsilon,
                                                           workspace=ws, m=rows))
-        if not is_prefill and logits_indices is None and self.decode_wide(rows) and self._wide_weights_ready():
-            ws = self.gemm_workspace()
+        if not is_prefill and logits_indices is None and self.decode_wide(rows):
+            # a workspace of the call's own: calls on several streams or threads share none
+            ws = _C.alloc_skinny_workspace(self._gemm_shapes(), input_ids_flat.device)
             residual = self.model.forward_decode_wide(input_ids_flat, position_ids_flat, kv_cache, attn_metadata, ws)
-            norm = self.model.norm
-            if rows > 64:  # two slabs read the head's weight twice: 363 against 282 us at 128 rows x 4096
-                return CausalLMOutput(logits=linear(norm(residual), self.lm_head, skinny=False))
-            x = _C.rms_norm_tiled(residual, norm.weight, norm.variance_epsilon)
-            return CausalLMOutput(logits=_C.skinny_linear(x, self.lm_head_tiled.storage, workspace=ws, m=rows))
-        h = self.model(input_ids_flat, position_ids_flat, kv_cache, attn_metadata, is_prefill)
+            h = self.model.norm(residual)
+        else:
+            h = self.model(input_ids_flat, position_ids_flat, kv_cache, attn_metadata, is_prefill)
         if logits_indices is not None:
             h = h.index_select(0, logits_indices)
-        skinny = h.shape[0] <= 64 or not self.decode_wide(h.shape[0])
-        return CausalLMOutput(logits=linear(h, self.lm_head, skinny, tiled=self.lm_head_tiled.of(self.lm_head)))
+        return CausalLMOutput(logits=linear(h, self.lm_head, tiled=self.lm_head_tiled.of(self.lm_head)))
 
     # ---------------------------------------------------------------- weights
     @torch.no_grad()

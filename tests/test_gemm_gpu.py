@@ -415,3 +415,50 @@ def test_residual_long_k_plans(device, m, nk):
     _C.skinny_linear(x, wt, again, epilogue=_C.EPI_RESID, y_ssq=ssq, workspace=ws)
     torch.cuda.synchronize()
     assert torch.equal(again, r)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 16, 17, 32, 33, 64, 65, 128])
+@pytest.mark.parametrize("n,k,epi", [(6144, 2560, "store"), (96, 512, "store"), (4096, 768, "silu"), (8192, 1280, "silu"),
+                                     (160, 256, "silu"), (4096, 4096, "resid"), (2560, 9728, "resid"), (96, 256, "resid")])
+def test_row_major_weight(device, m, n, k, epi):
+    """The weight itself instead of its tiled copy, under each of its plans, against the fp32 product."""
+    x, w = _operands(m, 2 * n if epi == "silu" else n, k, device, seed=m + n)
+    full = x.float() @ w.float().t()
+    if epi == "store":
+        y = _C.skinny_linear(x, w, w_rows=True)
+        torch.cuda.synchronize()
+        assert torch.equal(y, _C.skinny_linear(x, _C.tile(w)))  # the same plan in either layout
+        _assert_close_bf16(y, full)
+    elif epi == "silu":
+        y = _C.skinny_linear(x, w, epilogue=_C.EPI_SILU, w_rows=True).float()
+        full = full.to(torch.bfloat16)
+        ref = _C.silu_mul(full).float()
+        torch.cuda.synchronize()
+        # as in test_silu_column_plans
+        bound = 2.0 ** -6 * ref.abs() + 2.0 ** -7 * 1.1 * full[:, :n].abs().float() * full[:, n:].abs().float() + 3e-5
+        assert ((y - ref).abs() <= bound).all()
+    else:
+        gen = torch.Generator(device=device).manual_seed(6)
+        r0 = torch.randn((m, n), generator=gen, device=device).to(torch.bfloat16)
+        ssq = torch.full((m, n // 32), -1.0, device=device)
+        ws = _C.alloc_skinny_workspace([(n, k, _C.EPI_RESID)], device)
+        d = full.to(torch.bfloat16).float()
+        ref = r0.float() + d
+        for _ in range(2):  # the workspace is ready for the next call
+            r = r0.clone()
+            _C.skinny_linear(x, w, r, epilogue=_C.EPI_RESID, y_ssq=ssq, workspace=ws, w_rows=True)
+            torch.cuda.synchronize()
+            assert ((r.float() - ref).abs() <= 2 * ULP * (d.abs() + ref.abs()) + 1e-5).all()
+            assert torch.allclose(ssq, _tile_ssq(r), rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.gpu
+def test_row_major_weight_refusals(device):
+    x, w = _operands(4, 64, 1024, device, seed=1)
+    with pytest.raises(ValueError, match="tiled"):
+        _C.skinny_linear(x, w)
+    with pytest.raises(ValueError, match="contiguous"):
+        _C.skinny_linear(x, w.t().contiguous().t(), w_rows=True)
+    with pytest.raises(ValueError, match="unsupported"):
+        _C.skinny_linear(x, w, x_ssq=torch.ones(4, 32, device=device), norm_weight=w[0].contiguous(), w_rows=True)

@@ -55,8 +55,8 @@ def _model(device, hidden, inter, heads, batch):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("hidden,inter,heads,batch", [(2560, 3072, 32, 7), (4096, 8192, 32, 33), (5120, 2560, 40, 16),
-                                                      (4096, 4096, 64, 70), (256, 512, 8, 1)])
+@pytest.mark.parametrize("hidden,inter,heads,batch", [(2560, 3072, 32, 7), (4096, 8192, 32, 32), (5120, 2560, 40, 17),
+                                                      (4096, 4096, 64, 16), (256, 512, 8, 1), (2560, 9728, 32, 20)])
 @torch.inference_mode()
 def test_wide_decode_matches_the_library_path(device, hidden, inter, heads, batch):
     model, cache, md, ids = _model(device, hidden, inter, heads, batch)
@@ -65,11 +65,14 @@ def test_wide_decode_matches_the_library_path(device, hidden, inter, heads, batc
         return model(input_ids_flat=ids, position_ids_flat=md.positions, kv_cache=cache, attn_metadata=md,
                      is_prefill=False).logits.float()
 
-    assert model.decode_wide(batch) and not model.decode_fusable(batch)
+    assert model.decode_wide(batch) and not model.decode_fusable(batch) and not model.decode_wide(33)
+    with pytest.MonkeyPatch.context() as m:
+        m.setattr(model, "decode_wide", lambda rows: False)
+        plain = step()
+    before = torch.cuda.memory_allocated()
     wide = step()
-    assert model.lm_head_tiled.of(model.lm_head) is not None
-    model.decode_wide = lambda rows: False
-    plain = step()
+    torch.cuda.synchronize()
+    assert torch.cuda.memory_allocated() - before == -(-wide.nbytes // 512) * 512  # nothing but the logits stays
     torch.cuda.synchronize()
     # each of the 2 layers rounds its projections to bf16 six times (1.7e-3 rms each) on either path
     assert ((wide - plain).norm() / plain.norm()).item() < 2e-2
@@ -77,51 +80,104 @@ def test_wide_decode_matches_the_library_path(device, hidden, inter, heads, batc
 
 @pytest.mark.gpu
 @torch.inference_mode()
-def test_wide_decode_keeps_the_library_path_under_a_first_capture_and_without_room(device, monkeypatch):
-    """A capture cannot build the tiled weights, and neither can a device whose memory the KV pool fills."""
+def test_wide_decode_takes_the_library_path_for_weights_the_kernels_cannot_read(device):
     model, cache, md, ids = _model(device, 2560, 3072, 32, 4)
 
     def step():
         return model(input_ids_flat=ids, position_ids_flat=md.positions, kv_cache=cache, attn_metadata=md,
-                     is_prefill=False).logits
+                     is_prefill=False).logits.float()
 
-    with monkeypatch.context() as m:
-        m.setattr(torch.cuda, "mem_get_info", lambda d=None: (0, 1 << 40))
-        eager = step().float()
-        assert model.lm_head_tiled.of(model.lm_head) is None
-        torch.cuda.synchronize()
+    wide = step()
+    down = model.model.layers[1].mlp.down_weight
+    down.data = down.data.t().contiguous().t()  # the same values, column by column
+    assert not model.decode_wide(4)
+    plain = step()
+    torch.cuda.synchronize()
+    assert ((wide - plain).norm() / plain.norm()).item() < 2e-2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("change", ["data", "in_place", "state_dict", "load"])
+@torch.no_grad()
+def test_new_weights_reach_eager_steps_and_captured_graphs(device, change):
+    """A wide model reads its weights as they are: after any change of them an eager step and a graph captured before
+    give the bits of a model that held the new weights from the start."""
+    model, cache, md, ids = _model(device, 2560, 3072, 32, 4)
+    other, cache2, md2, _ = _model(device, 2560, 3072, 32, 4)
+    other.init_random(4)
+
+    def step(m, kv, meta):
+        return m(input_ids_flat=ids, position_ids_flat=meta.positions, kv_cache=kv, attn_metadata=meta,
+                 is_prefill=False).logits
+
+    first = step(model, cache, md).float()
+    torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
-        out = step()
-    assert model.lm_head_tiled.of(model.lm_head) is None
+        out = step(model, cache, md)
+    if change == "load":
+        model.init_random(4)
+    elif change == "state_dict":
+        model.load_state_dict(other.state_dict())
+    else:
+        for p, q in zip(model.parameters(), other.parameters()):
+            (p.data if change == "data" else p).copy_(q)
+    ref = step(other, cache2, md2).float()
+    eager = step(model, cache, md).float()
+    torch.cuda.synchronize()
+    assert torch.equal(eager, ref) and not torch.equal(ref, first)
     for _ in range(2):
         graph.replay()
         torch.cuda.synchronize()
-        assert torch.equal(out.float(), eager)
-    step()
-    assert model.lm_head_tiled.of(model.lm_head) is not None
+        assert torch.equal(out.float(), ref)
 
 
 @pytest.mark.gpu
 @torch.inference_mode()
-def test_new_weights_reach_captured_graphs(device):
-    """Loading weights rewrites the tiled copies in place: a graph captured before replays with the new ones."""
-    model, cache, md, ids = _model(device, 2560, 3072, 32, 4)
+def test_wide_decode_captured_first_equals_eager(device):
+    """A capture before any eager step: the replays, with eager steps between them, give the eager bits."""
+    model, cache, md, ids = _model(device, 2560, 9728, 32, 4)
 
     def step():
         return model(input_ids_flat=ids, position_ids_flat=md.positions, kv_cache=cache, attn_metadata=md,
                      is_prefill=False).logits
 
-    first = step().float()
+    torch.mm(torch.ones(8, 8, device=device).bfloat16(), torch.ones(8, 8, device=device).bfloat16())  # library handle
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         out = step()
-    model.init_random(4)
-    for _ in range(2):
+    for _ in range(3):
         graph.replay()
         torch.cuda.synchronize()
         got = out.float()
         eager = step().float()
         torch.cuda.synchronize()
-        assert torch.equal(got, eager) and not torch.equal(got, first)
+        assert torch.equal(got, eager)
+
+
+@pytest.mark.gpu
+@torch.inference_mode()
+def test_wide_decode_on_two_streams_at_once(device):
+    """Steps of one model queued on two streams share no workspace: each repeats the bits of a step alone."""
+    model, cache, md, ids = _model(device, 2560, 9728, 32, 4)
+    cache2 = PagedKVCache(2, 16, 16, 8, 128, torch.bfloat16, device)
+    cache2.key_cache.copy_(cache.key_cache)
+    cache2.value_cache.copy_(cache.value_cache)
+    md2 = PagedKVCacheMetadata(**{**md.__dict__, "decode_workspace": _C.alloc_paged_decode_workspace(4, 32, 8, 512,
+                                                                                                     device)})
+
+    def step(kv, meta):
+        return model(input_ids_flat=ids, position_ids_flat=meta.positions, kv_cache=kv, attn_metadata=meta,
+                     is_prefill=False).logits
+
+    alone = step(cache, md).float()
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    outs = []
+    for _ in range(6):
+        for s, kv, meta in zip(streams, (cache, cache2), (md, md2)):
+            with torch.cuda.stream(s):
+                outs.append(step(kv, meta))
+    torch.cuda.synchronize()
+    assert all(torch.equal(o.float(), alone) for o in outs)
