@@ -357,77 +357,61 @@ skinny_gemm_kernel(GemmArgs a) {
     __hip_atomic_store(a.counters + group, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Waves, 16-column tiles per wave, K slices over workgroups, 32-wide K steps per wave and round.  nw, ks and kb order a
+// row's sums.  They follow from the weight's shape, the epilogue and W's layout alone, so a row's result does not depend on
+// the rows beside it; only nt follows the row count.
 struct Plan {
   int nw, nt, ks, kb;
 };
 
 // Measured on MI355X with weights streamed from HBM (rotating copies, one graph), us per launch:
-//   * vocabulary-sized N (LM head), no split: 32 columns per 8-wave workgroup up to 16 rows (N = 151,936, K = 1,024 / 4,096 at M = 4:
-//     51.8 / 211 against 56.3 / 226 for 128 columns of 4 waves), 64 up to 32 rows (58.5 / 236.7 against
-//     61.6 / 242), where X is read again per column group; 64 of 4 waves for 64-row slabs (128
-//     would need 128 accumulator registers at 4 M tiles);
+//   * vocabulary-sized N (LM head), no split, 4 waves: 32 columns per workgroup up to 16 rows (151,936 x 1,024 at M = 4 51.3 against
+//     56.3 for 128 columns; 8 waves 51.7), then 64, which keep X's repeated reads down (M = 32 / 64 / 100 59.3 /
+//     72.5 / 114.6; 8 waves 58.4 / 93.5 / 157);
 //   * residual epilogue (N = hidden: o_proj, down_proj): 32 columns (the epilogue's sums of
 //     squares cover whole 32-column groups) per 8-wave workgroup, K split over >= 128
 //     workgroups (at N = 1,024, K = 2,048 / 3,072 o 6.5, down 6.6; unsplit 16-wave workgroups 8.2).  A long K
-//     (down_proj, K >= 1.5 N) is split further, to >= 512 workgroups of >= 1,152 K each, where a workgroup's
-//     stream would otherwise last many rounds of 128 workgroups: at M = 32, N x K = 4,096 x 12,288 22.6 against 32.7,
-//     5,120 x 17,408 37.4 against 47.2, 2,560 x 9,728 14.6 against 16.7, 2,048 x 6,144 9.3 against 11.6; where that gives 512
-//     workgroups four waves lead eight (37.4 / 42, 14.6 / 15.9).  Above 64 rows the merges of two slabs cost what the split gains
-//     (4,096 x 12,288 at M = 100: 39.4 unsplit, 42.4 in two);
-//   * gate_up: 16 columns per 8-wave workgroup; from N = 4,096 on 32, from N = 8,192 on and up to 32 rows 16 per 4-wave workgroup (M = 32:
-//     6,144 x 2,048 normed 14.1 against 17.3, 12,288 x 4,096 37.3 against 39.6, 9,728 x 2,560 21.2 against 23.5; above 64 rows
-//     32 per 4-wave workgroup, 62.3 against 67.2);
+//     (down_proj, K >= 1.5 N) is split over >= 256, in slices of >= 1,152, where a workgroup's
+//     stream would otherwise last many rounds: at M = 32, N x K = 4,096 x 12,288 22.7 against 34.8, 2,048 x 6,144
+//     9.3 against 11.5.  Above 64 rows the merges of two slabs cost about what the split gains (M = 100: 41.6 against 40.1,
+//     15.0 against 14.2; 2,560 x 9,728 26.8 against 31.7);
+//   * gate_up: 16 columns per 8-wave workgroup, 32 above 64 rows; 32 from N = 4,096 on (6,144 x 2,048 normed at M = 32: 13.8 against
+//     17.3); from N = 8,192 on 4 waves, 16 columns up to 32 rows and 32 above (12,288 x 4,096 at M = 32 / 100: 40.4 /
+//     61.7 against 42.3 / 67.0 of 8 waves);
 //   * otherwise (qkv): 16 columns per 8-wave workgroup, 32 from N = 6,144 on (6,144 x 4,096 at M = 8 / 32: 11.4 / 13.5
-//     against 13.6 / 17.5) and above 64 rows, halving the X reads per weight byte (normed, K = 2,048 at
-//     M = 100: 13.6 against 20.3).
-//   * row-major W (W_ROWS; 16 rows x 64 bytes per load instruction), M = 8 / 32: gate_up from N = 8,192 on 16 columns per 4-wave
-//     workgroup, 256 bytes of a row per wave and round (12,288 x 4,096 41.6 / 45.9 against 43.7 / 50.0 with 128 bytes
-//     of 8 waves, 9,728 x 2,560 26.4 / 31.2 against 29.0 / 33.3); residual projections 4 waves, split to >= 512 workgroups of >=
-//     512 K (4,096 x 4,096 12.0 / 12.6 against 13.5 / 15.9 unsplit of 8 waves, 2,560 x 9,728 14.9 / 18.0 against
-//     16.6 / 20.5 at 160 of 8, 5,120 x 17,408 45.8 / 54.5 against 54.4 / 63.9 unsplit); others as tiled.
-Plan make_plan(int n, int k, int epi, int m, bool wide, bool w_rows) {
-  Plan p{8, 1, 1, k % 512 == 0 ? 2 : 1};
-  static const int kSlices[] = {1, 2, 3, 4, 6, 8, 12, 16};
-  auto whole = [&](int ks) { return k % ks == 0 && (k / ks) % 64 == 0; };  // 64-wide wave blocks
-  if (w_rows && epi == kEpiResid) {
-    p = Plan{4, 2, 1, 1};
-    for (int ks : kSlices) {
-      if (n / 32 * p.ks >= 512 || k / ks < 512) break;
-      if (whole(ks)) p.ks = ks;
-    }
-    return p;
-  }
-  if (w_rows && epi == kEpiSilu && n >= 8192) return Plan{4, m > 32 ? 2 : 1, 1, 4};
-  if (epi == kEpiStore && n % 128 == 0 && n / 128 >= 512) {
-    if (wide) return Plan{4, 4, 1, 2};
-    return m <= 16 ? Plan{8, 2, 1, 2} : Plan{8, 4, 1, 1};
-  }
+//     against 13.6 / 17.5) and above 64 rows, halving the X reads per weight byte (4,096 x 2,048 normed at
+//     M = 100: 14.8 against 20.3);
+//   * row-major W (W_ROWS; 16 rows x 64 bytes per load instruction), M = 8 / 32: gate_up from N = 8,192 on 256 bytes of a row per wave
+//     and round (12,288 x 4,096 41.6 / 45.9 against 44.5 / 48.1 with 128 bytes, 9,728 x 2,560 26.4 / 31.2 against
+//     28.1 / 31.7); residual projections 4 waves, split to >= 512 workgroups of >= 512 K (4,096 x 4,096 12.0 / 12.6 against
+//     13.5 / 15.9 unsplit of 8 waves, 2,560 x 9,728 14.9 / 18.0 against 16.6 / 20.5 at 160 of 8, 5,120 x 17,408 45.8 / 54.5
+//     against 54.4 / 63.9 unsplit); others as tiled.
+Plan make_plan(int n, int k, int epi, int m, bool w_rows) {
+  const int kb = k % 512 == 0 ? 2 : 1;
   if (epi == kEpiResid) {
-    p = Plan{8, 2, 1, 2};
+    static const int kSlices[] = {1, 2, 3, 4, 6, 8, 12, 16};
     const int groups = n / 32;
-    for (int ks : kSlices) {
-      if (!whole(ks)) continue;
-      p.ks = ks;
-      if (groups * ks >= 128) break;
+    int slices = 1;
+    auto split = [&](int workgroups, int min_k) {
+      for (int ks : kSlices) {
+        if (groups * slices >= workgroups || k / ks < min_k) break;
+        if (ks > slices && k % ks == 0 && (k / ks) % 64 == 0) slices = ks;  // whole 64-wide wave blocks
+      }
+    };
+    if (w_rows) {
+      split(512, 512);
+      return {4, 2, slices, 1};
     }
-    if (m > 64 || 2 * k < 3 * n) return p;
-    for (int ks : kSlices) {
-      if (groups * p.ks >= 512 || k / ks < 1152) break;
-      if (ks > p.ks && whole(ks)) p.ks = ks;
-    }
-    if (groups * p.ks >= 512) p = Plan{4, 2, p.ks, 1};
-    return p;
+    split(128, 1);
+    if (2 * k >= 3 * n) split(256, 1152);
+    return {8, 2, slices, 2};
   }
-  if (m > 64) {
-    p.nt = 2;
-    if (epi == kEpiSilu ? n >= 4096 : !wide && n < 6144) p.nw = 4;
-  } else if (epi == kEpiSilu) {
-    if (n >= 8192 && m <= 32) return Plan{4, 1, 1, k <= 4096 ? 1 : 2};
-    if (n >= 4096 && n < 8192) return Plan{8, 2, 1, 1};
-  } else if (n >= 6144) {
-    p.nt = 2;
+  if (epi == kEpiSilu) {
+    if (n >= 8192) return {4, m > 32 ? 2 : 1, 1, w_rows ? 4 : 2};
+    return {8, m > 64 || n >= 4096 ? 2 : 1, 1, kb};
   }
-  return p;
+  if (n % 128 == 0 && n / 128 >= 512) return {4, m <= 16 ? 2 : 4, 1, 2};
+  return {8, m > 64 || n >= 6144 ? 2 : 1, 1, kb};
 }
 
 constexpr int kMaxSlabs = 4;  // M <= 128
@@ -445,14 +429,14 @@ size_t workspace_bytes_for(const Plan &p, int n, int epi) {
 bool wide_rows(int m, int k, bool norm, int epi) {
   return m > 32 && (!norm || (k <= kMaxWideNormK && epi != kEpiResid));
 }
-// Configurations 64-row slabs are built for (at most 64 columns per workgroup).
-template <int NW, int NT, int EPI, bool NORM>
-constexpr bool kWideBuilt = (NT <= 2 || NW == 4) && !(NORM && EPI == kEpiResid);
+// Configurations 64-row slabs are built for.
+template <int EPI, bool NORM>
+constexpr bool kWideBuilt = !(NORM && EPI == kEpiResid);
 
 template <int NW, int KB, int NT, int EPI, bool NORM, bool W_ROWS>
 int launch(const GemmArgs &a, int grid, bool wide, hipStream_t stream) {
   if (wide) {
-    if constexpr (kWideBuilt<NW, NT, EPI, NORM>) {
+    if constexpr (kWideBuilt<EPI, NORM>) {
       if (a.m <= 64)
         hipLaunchKernelGGL((skinny_gemm_kernel<NW, KB, NT, 4, EPI, NORM, false, W_ROWS>), dim3(grid), dim3(NW * 64), 0,
                            stream, a);
@@ -474,27 +458,21 @@ int launch(const GemmArgs &a, int grid, bool wide, hipStream_t stream) {
   return launch_status();
 }
 
-template <int NW, int NT, int EPI, bool NORM, bool W_ROWS>
-int launch_kb(const GemmArgs &a, const Plan &p, int grid, bool wide, hipStream_t stream) {
-  if constexpr (W_ROWS && EPI == kEpiSilu && NW == 4)
-    if (p.kb == 4) return launch<NW, 4, NT, EPI, NORM, W_ROWS>(a, grid, wide, stream);
-  return p.kb == 2 ? launch<NW, 2, NT, EPI, NORM, W_ROWS>(a, grid, wide, stream)
-                   : launch<NW, 1, NT, EPI, NORM, W_ROWS>(a, grid, wide, stream);
-}
-
 template <int EPI, bool NORM, bool W_ROWS>
 int dispatch(const GemmArgs &a, const Plan &p, int grid, bool wide, hipStream_t stream) {
-  if constexpr (EPI == kEpiStore) {
-    if (p.nw == 4 && p.nt == 4) return launch_kb<4, 4, EPI, NORM, W_ROWS>(a, p, grid, wide, stream);
-    if (p.nw == 8 && p.nt == 4) return launch_kb<8, 4, EPI, NORM, W_ROWS>(a, p, grid, wide, stream);
-  } else if constexpr (EPI == kEpiSilu) {
-    if (p.nw == 4 && p.nt == 1) return launch_kb<4, 1, EPI, NORM, W_ROWS>(a, p, grid, wide, stream);
+  auto is = [&](int nw, int nt, int kb) { return p.nw == nw && p.nt == nt && p.kb == kb; };
+  if constexpr (EPI == kEpiResid) {
+    constexpr int NW = W_ROWS ? 4 : 8, KB = W_ROWS ? 1 : 2;
+    if (is(NW, 2, KB)) return launch<NW, KB, 2, EPI, NORM, W_ROWS>(a, grid, wide, stream);
+  } else {
+    if (is(8, 1, 1)) return launch<8, 1, 1, EPI, NORM, W_ROWS>(a, grid, wide, stream);
+    if (is(8, 1, 2)) return launch<8, 2, 1, EPI, NORM, W_ROWS>(a, grid, wide, stream);
+    if (is(8, 2, 1)) return launch<8, 1, 2, EPI, NORM, W_ROWS>(a, grid, wide, stream);
+    if (is(8, 2, 2)) return launch<8, 2, 2, EPI, NORM, W_ROWS>(a, grid, wide, stream);
+    constexpr int KB = EPI == kEpiSilu && W_ROWS ? 4 : 2, NT = EPI == kEpiSilu ? 1 : 4;
+    if (is(4, NT, KB)) return launch<4, KB, NT, EPI, NORM, W_ROWS>(a, grid, wide, stream);
+    if (is(4, 2, KB)) return launch<4, KB, 2, EPI, NORM, W_ROWS>(a, grid, wide, stream);
   }
-  if constexpr (EPI != kEpiResid) {
-    if (p.nw == 8 && p.nt == 1) return launch_kb<8, 1, EPI, NORM, W_ROWS>(a, p, grid, wide, stream);
-  }
-  if (p.nw == 4 && p.nt == 2) return launch_kb<4, 2, EPI, NORM, W_ROWS>(a, p, grid, wide, stream);
-  if (p.nw == 8 && p.nt == 2) return launch_kb<8, 2, EPI, NORM, W_ROWS>(a, p, grid, wide, stream);
   return NVAMD_EUNSUPPORTED;
 }
 
@@ -513,11 +491,9 @@ using namespace nvamd;
 
 extern "C" size_t nvamd_skinny_linear_workspace_size(int n, int k, int epilogue) {
   if (n <= 0 || k <= 0 || n % 32 || k % 256 || epilogue < 0 || epilogue > 2) return 0;
-  // the largest of the plans' needs (the row count and the weight's layout are not known here)
-  const size_t slabs = workspace_bytes_for(make_plan(n, k, epilogue, 32, false, false), n, epilogue);
-  const size_t wide = workspace_bytes_for(make_plan(n, k, epilogue, 128, true, false), n, epilogue);
-  const size_t rows = workspace_bytes_for(make_plan(n, k, epilogue, 32, false, true), n, epilogue);
-  return std::max({slabs, wide, rows});
+  // the larger of the two layouts' needs (what a plan needs does not depend on the row count)
+  return std::max(workspace_bytes_for(make_plan(n, k, epilogue, 1, false), n, epilogue),
+                  workspace_bytes_for(make_plan(n, k, epilogue, 1, true), n, epilogue));
 }
 
 extern "C" int nvamd_skinny_linear(const void *x, int64_t x_stride, const float *x_ssq, const void *norm_weight,
@@ -539,7 +515,7 @@ extern "C" int nvamd_skinny_linear(const void *x, int64_t x_stride, const float 
       (norm && (!aligned16(x_ssq) || !aligned16(norm_weight))))
     return NVAMD_EINVAL;
   const bool wide = wide_rows(m, k, norm, epilogue);
-  const Plan p = make_plan(n, k, epilogue, m, wide, flags & NVAMD_GEMM_W_ROWS);
+  const Plan p = make_plan(n, k, epilogue, m, flags & NVAMD_GEMM_W_ROWS);
   const int groups = n / (16 * p.nt);
   if ((k / p.ks) % (32 * p.kb) != 0) return NVAMD_EUNSUPPORTED;  // whole wave blocks per slice
   const int slabs = wide ? (m + 63) / 64 : (m + 31) / 32;

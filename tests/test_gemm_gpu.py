@@ -462,3 +462,52 @@ def test_row_major_weight_refusals(device):
         _C.skinny_linear(x, w.t().contiguous().t(), w_rows=True)
     with pytest.raises(ValueError, match="unsupported"):
         _C.skinny_linear(x, w, x_ssq=torch.ones(4, 32, device=device), norm_weight=w[0].contiguous(), w_rows=True)
+
+
+ROW_SHAPES = [(151936, 1024, "store", True), (65536, 2048, "store", True), (4096, 2048, "store", True),
+              (6144, 2560, "store", False), (6144, 2048, "silu", True), (3072, 1024, "silu", True),
+              (8192, 1024, "silu", True), (9728, 2560, "silu", False), (2048, 6144, "resid", False),
+              (2560, 9728, "resid", False), (4096, 12288, "resid", False), (1024, 3072, "resid", False)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,k,epi,norm", ROW_SHAPES)
+def test_rows_do_not_depend_on_the_batch(device, n, k, epi, norm):
+    """Every row, at row counts on either side of each switch of slabs and columns, equals the same projection of that
+    row alone, bit for bit, in both layouts of the weight; the one-row call against the fp32 product."""
+    x, w = _operands(128, 2 * n if epi == "silu" else n, k, device, seed=k)
+    nw = (1.0 + 0.1 * torch.randn(k, generator=torch.Generator().manual_seed(2))).to(torch.bfloat16).to(device)
+    code = {"store": _C.EPI_STORE, "silu": _C.EPI_SILU, "resid": _C.EPI_RESID}[epi]
+    ws = _C.alloc_skinny_workspace([(n, k, code)], device)
+    r0 = torch.randn((128, n), generator=torch.Generator(device=device).manual_seed(3), device=device).bfloat16()
+
+    def run(weight, rows, **kw):
+        xs, y = x[rows], r0[rows].clone()
+        if norm and not kw:
+            kw = dict(x_ssq=_tile_ssq(xs).contiguous(), norm_weight=nw)
+        return _C.skinny_linear(xs, weight, y, epilogue=code, workspace=ws,
+                                y_ssq=torch.empty((len(y), n // 32), device=device) if epi == "resid" else None, **kw)
+
+    for weight, kw in ((_C.tile(w), {}), (w, {"w_rows": True})):
+        one = {}
+        for m in (16, 17, 32, 33, 64, 65, 128):
+            y = run(weight, slice(0, m), **kw)
+            for r in (0, m // 2, m - 1):
+                if r not in one:
+                    one[r] = run(weight, slice(r, r + 1), **kw)
+                torch.cuda.synchronize()
+                assert torch.equal(y[r], one[r][0]), (m, r, (y[r].float() - one[r][0].float()).abs().max().item())
+        f = x[:1].float()
+        if norm and not kw:
+            f = (f * torch.rsqrt(f.pow(2).mean(-1, keepdim=True) + 1e-6) * nw.float()).bfloat16().float()
+        full = (f @ w.float().t()).bfloat16().float()
+        got = one[0].float()
+        if epi == "store":
+            # a sum in another order, and a normed operand that may round to its neighbour (2^-9 of it, at random)
+            assert ((got - full).abs() <= 2 * ULP * full.abs() + 4e-3).all()
+        elif epi == "resid":
+            assert ((got - r0[:1].float() - full).abs() <= 2 * ULP * (full.abs() + r0[:1].float().abs()) + 4e-3).all()
+        else:
+            gate, up = full[:, :n], full[:, n:]
+            ref = torch.nn.functional.silu(gate) * up
+            assert ((got - ref).abs() <= 2.0 ** -6 * ref.abs() + 2.0 ** -6 * gate.abs() * up.abs() + 4e-3).all()
