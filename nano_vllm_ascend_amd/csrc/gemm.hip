@@ -371,10 +371,11 @@ struct Plan {
 //   * residual epilogue (N = hidden: o_proj, down_proj): 32 columns (the epilogue's sums of
 //     squares cover whole 32-column groups) per 8-wave workgroup, K split over >= 128
 //     workgroups (at N = 1,024, K = 2,048 / 3,072 o 6.5, down 6.6; unsplit 16-wave workgroups 8.2).  A long K
-//     (down_proj, K >= 1.5 N) is split over >= 256, in slices of >= 1,152, where a workgroup's
-//     stream would otherwise last many rounds: at M = 32, N x K = 4,096 x 12,288 22.7 against 34.8, 2,048 x 6,144
-//     9.3 against 11.5.  Above 64 rows the merges of two slabs cost about what the split gains (M = 100: 41.6 against 40.1,
-//     15.0 against 14.2; 2,560 x 9,728 26.8 against 31.7);
+//     (down_proj, K >= 1.5 N) is split over up to 512, in slices of >= 1,152, where a workgroup's stream would otherwise
+//     last many rounds, and four waves lead eight where that gives 512 (N x K at M = 4 / 32 / 64 / 100, against 128:
+//     2,048 x 6,144 9.0 / 9.5 / 12.1 / 15.4 against 11.7 / 12.9 / 15.0 / 14.7, 2,560 x 9,728 14.0 / 15.0 / 21.6 / 30.2
+//     against 15.7 / 18.8 / 21.9 / 32.4, 4,096 x 12,288 22.6 / 23.8 / 30.7 / 47.4 against 30.3 / 35.2 / 43.8 / 40.9,
+//     5,120 x 17,408 35.8 / 39.0 / 56.9 / 82.6 against 41.8 / 51.3 / 62.4 / 95.8);
 //   * gate_up: 16 columns per 8-wave workgroup, 32 above 64 rows; 32 from N = 4,096 on (6,144 x 2,048 normed at M = 32: 13.8 against
 //     17.3); from N = 8,192 on 4 waves, 16 columns up to 32 rows and 32 above (12,288 x 4,096 at M = 32 / 100: 40.4 /
 //     61.7 against 42.3 / 67.0 of 8 waves);
@@ -403,7 +404,10 @@ Plan make_plan(int n, int k, int epi, int m, bool w_rows) {
       return {4, 2, slices, 1};
     }
     split(128, 1);
-    if (2 * k >= 3 * n) split(256, 1152);
+    if (2 * k >= 3 * n) {
+      split(512, 1152);
+      if (groups * slices >= 512) return {4, 2, slices, 1};
+    }
     return {8, 2, slices, 2};
   }
   if (epi == kEpiSilu) {
@@ -462,8 +466,9 @@ template <int EPI, bool NORM, bool W_ROWS>
 int dispatch(const GemmArgs &a, const Plan &p, int grid, bool wide, hipStream_t stream) {
   auto is = [&](int nw, int nt, int kb) { return p.nw == nw && p.nt == nt && p.kb == kb; };
   if constexpr (EPI == kEpiResid) {
-    constexpr int NW = W_ROWS ? 4 : 8, KB = W_ROWS ? 1 : 2;
-    if (is(NW, 2, KB)) return launch<NW, KB, 2, EPI, NORM, W_ROWS>(a, grid, wide, stream);
+    if (is(4, 2, 1)) return launch<4, 1, 2, EPI, NORM, W_ROWS>(a, grid, wide, stream);
+    if constexpr (!W_ROWS)
+      if (is(8, 2, 2)) return launch<8, 2, 2, EPI, NORM, W_ROWS>(a, grid, wide, stream);
   } else {
     if (is(8, 1, 1)) return launch<8, 1, 1, EPI, NORM, W_ROWS>(a, grid, wide, stream);
     if (is(8, 1, 2)) return launch<8, 2, 1, EPI, NORM, W_ROWS>(a, grid, wide, stream);
