@@ -656,10 +656,11 @@ int launch(DecodeArgs a, int batch, hipStream_t stream) {
 }
 
 // ------------------------------------------------------------------------------------------
-// MFMA variant, for groups of 3 to 16 query heads.
+// MFMA variant, for up to 8 query heads of a group: groups of 3 and more, and those of 1 and 2 under bounds past 16,384
+// tokens.
 //
 // The same split-KV items, scan, records and arrival counting as above, for up to GP query heads of
-// a kv head in one launch, so K and V are read once whatever the ratio.  A wave's 64 tokens:
+// a kv head in one launch, so K and V are read once up to a ratio of 8.  A chunk of 64 tokens, of which a wave takes CPW:
 //   S^T = K . Q^T by v_mfma_f32_16x16x32_bf16 with A = rows of K as read from the cache.  The operand's
 //        16 rows x 32 dims give a load only 64 consecutive bytes of a cache row, and K read that way
 //        took 1.07-1.15x the launch's time.  So 8 row slots take dims 0..31 of a 64-dim half and the other 8 (z = 1)
@@ -702,11 +703,11 @@ __device__ __forceinline__ float half_max(float v) {
 __device__ __forceinline__ float half_sum(float v) { return sum_xor16(sum16(v)); }
 
 constexpr int kCachePolicyStream = 2;  // nt
-template <int GP, int NW, bool WHOLE, bool FUSED, bool MANY>
+template <int GP, int NW, int CPW, bool WHOLE, bool FUSED, bool MANY>
 __device__ __forceinline__ bool mfma_item(const DecodeArgs &a, const int tid, const int item, float (&s_o)[NW][GP * kPartFloats],
                                           float (&s_m)[NW][GP], float (&s_l)[NW][GP], int &s_last) {
   constexpr int D = kHeadDim;
-  constexpr int PART = NW * 64;
+  constexpr int PART = NW * CPW * 64;
   constexpr int HS = kPartFloats;   // floats per head in LDS (4 of padding: rows spread over the banks)
   const int hkv = a.num_kv_heads;
   const int G = a.q_sub;
@@ -784,17 +785,23 @@ __device__ __forceinline__ bool mfma_item(const DecodeArgs &a, const int tid, co
   const int gq = lane >> 4;
 
   const_i32 *bt_row = (const_i32 *)(a.block_tables + (int64_t)b * a.bt_stride);
-  const int t_begin = p * PART + 64 * w;
-  const int t_end = min(t_begin + 64, ctx);
+  // The wave's chunks are the w-th, w + NW-th ... 64 tokens of the partition.
+  int t_begin = p * PART + 64 * w;
+  int t_end = min(t_begin + 64, ctx);
   const int bs_mask = (1 << a.bs_log2) - 1;
   const int64_t row_elems = (int64_t)hkv * D;
   const int head0 = g * a.q_group + a.q_head0;
 
-  int blk_t[4] = {};
+  int blk_t[4] = {}, blk_n[4] = {};  // this chunk's and the next one's blocks
   if (t_begin < t_end) {
     const int last = (t_end - 1) & ~15;
 #pragma unroll
     for (int i = 0; i < 4; ++i) blk_t[i] = bt_row[min(t_begin + 16 * i, last) >> a.bs_log2];
+    if constexpr (CPW > 1) {
+      const int next = t_begin + 64 * NW, last_n = (min(next + 64, ctx) - 1) & ~15;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) blk_n[i] = bt_row[min(next + 16 * i, last_n) >> a.bs_log2];
+    }
   }
 
   // Query operand: lane (z, h, gq) holds dims 64k + 32z + 8gq .. +7 of head h (lanes past the group's
@@ -819,7 +826,7 @@ __device__ __forceinline__ bool mfma_item(const DecodeArgs &a, const int tid, co
       }
     };
     const bool nr_in = nr >= 0 && nr < ctx;
-    const bool owner = a.store_new && (nr_in ? (nr >= t_begin && nr < t_end) : (p == n_parts - 1 && w == 0));
+    const bool owner = a.store_new && (nr_in ? (nr >= p * PART && nr < (p + 1) * PART && (int)(nr >> 6) % NW == w) : (p == n_parts - 1 && w == 0));
     const u16 *qp = a.q + (int64_t)b * a.q_stride + (int64_t)(head0 + min(r, G - 1)) * D + 8 * c;
     qr[0] = ld16(qp);
     qr[1] = ld16(qp + 64);
@@ -934,6 +941,7 @@ __device__ __forceinline__ bool mfma_item(const DecodeArgs &a, const int tid, co
     }
   };
   u32x4 pf[2], pr[2];
+  float alpha = 1.f;
   auto softmax = [&]() {
     float cm = -INFINITY;
 #pragma unroll
@@ -945,7 +953,12 @@ __device__ __forceinline__ bool mfma_item(const DecodeArgs &a, const int tid, co
         cm = fmaxf(cm, s[i][e]);
       }
     cm = max_xor32(max_xor16(cm));
+    if (CPW > 1) cm = fmaxf(cm, m);
     const float ref = cm == -INFINITY ? 0.f : cm;  // no visible score yet
+    if (CPW > 1) {
+      alpha = fast_exp2(m - ref);
+      l *= alpha;
+    }
     m = cm;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -982,13 +995,15 @@ __device__ __forceinline__ bool mfma_item(const DecodeArgs &a, const int tid, co
       }
     }
   };
-  // K first, V in halves as the scores free K's registers: 128 VGPRs (four waves per SIMD) hold no more.
-  // Every load up front at 147-183 VGPRs measured the same or slower, at small batches too.
-  if (t_begin < t_end) {
+  // K first, V in halves as the scores free K's registers: 128 VGPRs (four waves per SIMD) hold no more, and with a
+  // running O none of it (CPW 2: three waves).  Every load up front at 147-183 VGPRs measured the same or slower, at
+  // small batches too.
+  auto chunk = [&](const bool first) {
     tiles();
 #pragma unroll
     for (int i = 0; i < 4; ++i) load_k(i);
-    if constexpr (FUSED) norm_queries();  // while K is in flight
+    if constexpr (FUSED)
+      if (first) norm_queries();  // while K is in flight
     __builtin_amdgcn_sched_barrier(0);
     score(0);
     score(1);
@@ -999,8 +1014,25 @@ __device__ __forceinline__ bool mfma_item(const DecodeArgs &a, const int tid, co
     softmax();
     __builtin_amdgcn_sched_barrier(0);
     load_v(1);
+    if (!first) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] *= alpha;
+    }
     __builtin_amdgcn_sched_barrier(0);
     pv();
+  };
+  if (t_begin < t_end) {
+    chunk(true);
+    static_assert(CPW <= 2, "one further chunk");
+    if constexpr (CPW > 1) {
+      t_begin += 64 * NW;
+      t_end = min(t_begin + 64, ctx);
+      if (t_begin < t_end) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) blk_t[i] = blk_n[i];
+        chunk(false);
+      }
+    }
   }
 
   err_bits = __builtin_amdgcn_readfirstlane(err_bits);
@@ -1176,16 +1208,16 @@ __device__ __forceinline__ bool mfma_item(const DecodeArgs &a, const int tid, co
 // workgroups: 4-8 us).  Each
 // item reads its arguments and thread index anew: values kept over the loop would not fit the
 // registers.
-template <int GP, int NW, bool WHOLE, bool FUSED, bool MANY>
+template <int GP, int NW, int CPW, bool WHOLE, bool FUSED, bool MANY>
 __global__ void __launch_bounds__(NW * 64)
-__attribute__((amdgpu_waves_per_eu(4)))
+__attribute__((amdgpu_waves_per_eu(CPW > 1 ? 3 : 4)))
 paged_decode_mfma_kernel(DecodeArgs a) {
   __shared__ __attribute__((aligned(16))) float s_o[NW][GP * kPartFloats];
   __shared__ float s_m[NW][GP];
   __shared__ float s_l[NW][GP];
   __shared__ int s_last;
   if constexpr (!MANY) {
-    mfma_item<GP, NW, WHOLE, FUSED, MANY>(a, threadIdx.x, blockIdx.x, s_o, s_m, s_l, s_last);
+    mfma_item<GP, NW, CPW, WHOLE, FUSED, MANY>(a, threadIdx.x, blockIdx.x, s_o, s_m, s_l, s_last);
   } else {
     const int items = a.max_items;
 #pragma unroll 1
@@ -1195,7 +1227,7 @@ paged_decode_mfma_kernel(DecodeArgs a) {
       int tid = threadIdx.x;
       asm volatile("" : "+s"(p), "+v"(tid));
       const DecodeArgs args = *(const DecodeArgs *)p;
-      if (!mfma_item<GP, NW, WHOLE, FUSED, MANY>(args, tid, item, s_o, s_m, s_l, s_last)) break;
+      if (!mfma_item<GP, NW, CPW, WHOLE, FUSED, MANY>(args, tid, item, s_o, s_m, s_l, s_last)) break;
       item += gridDim.x;
       if (item >= items) break;
       __syncthreads();  // every wave has read this item's LDS
@@ -1203,21 +1235,21 @@ paged_decode_mfma_kernel(DecodeArgs a) {
   }
 }
 
-template <int GP, int NW, bool WHOLE, bool FUSED>
+template <int GP, int NW, int CPW, bool WHOLE, bool FUSED>
 int launch_mfma(DecodeArgs a, int batch, hipStream_t stream) {
-  a.max_parts = ceil_div(a.max_ctx, NW * 64);
+  a.max_parts = ceil_div(a.max_ctx, NW * CPW * 64);
   if (WHOLE && a.max_parts != 1) return NVAMD_EINVAL;
   a.batch = batch;
   const int64_t items = (int64_t)batch * a.num_kv_heads * a.max_parts;
   a.max_items = (int)items;  // <= kCounterSlots units of <= 512 partitions
   if constexpr (!WHOLE) {
     if (items > kMaxGroups) {
-      hipLaunchKernelGGL((paged_decode_mfma_kernel<GP, NW, WHOLE, FUSED, true>), dim3(kMaxGroups), dim3(NW * 64),
+      hipLaunchKernelGGL((paged_decode_mfma_kernel<GP, NW, CPW, WHOLE, FUSED, true>), dim3(kMaxGroups), dim3(NW * 64),
                          0, stream, a);
       return launch_status();
     }
   }
-  hipLaunchKernelGGL((paged_decode_mfma_kernel<GP, NW, WHOLE, FUSED, false>), dim3((unsigned)items),
+  hipLaunchKernelGGL((paged_decode_mfma_kernel<GP, NW, CPW, WHOLE, FUSED, false>), dim3((unsigned)items),
                      dim3(NW * 64), 0, stream, a);
   return launch_status();
 }
@@ -1261,27 +1293,34 @@ int dispatch(const DecodeArgs &a, int batch, hipStream_t stream) {
   }
 }
 
-// Partitions of the MFMA variant: 256 tokens, or 512 tokens of 8 waves (half the partial records) in two cases.
+// Partitions of the MFMA variant: 256 tokens, or 512 (half the partial records) in two cases.
 // Groups of 5 to 8 heads publish 4 KB per partition, 3% of what a 256-token partition reads: launches of
-// more than 8,192 items, which are bandwidth-bound over many rounds, take 512 (100 x U[2048, 4096] at 8
-// heads: 235 against 245 us; fewer items prefer 256: 28.7 against 30.5 us at 16 x U[512, 4096]).  Bounds past
-// 16,384 tokens over fewer than 64 (sequence, kv head) units take 512 for the sake of the last merges,
-// 80 records instead of 160 at 40,960 tokens (4 x U[8192, 40960]: 59.2 / 55.2 / 53.1 against 67.2 / 59.4 / 54.6 us at 8 /
-// 4 / 2 heads); over more units contexts tend to be far shorter than such a bound: 256 (32 x U[256, 2304]
-// at a bound of 40,960: 36.7 against 38.9 us at 2 heads, 40.5 against 42.5 us at 8).
+// more than 8,192 items, which are bandwidth-bound over many rounds, take 512 tokens of 8 waves (100 x U[2048, 4096] at 8
+// heads: 235 against 245 us; fewer items prefer 256: 28.7 against 30.5 us at 16 x U[512, 4096]), and so do bounds past
+// 16,384 tokens over fewer than 64 (sequence, kv head) units, for the sake of the last merges (4 x U[8192, 40960]: 59.2
+// against 67.2 us; over more units contexts tend to be far shorter than such a bound: 32 x U[256, 2304] 40.5 against
+// 42.5 us).  Groups of up to 4 heads under bounds past 16,384 tokens take 512 tokens of 4 waves, two 64-token chunks
+// each: where contexts are that long, a workgroup's scan, publishing and merge weigh half (us at a bound of 40,960, against
+// 256 tokens of one chunk: 64 x U[8000, 16000] at 16 / 4 heads 271 / 308, 32 x U[20000, 40000] at 8 / 2 179 / 199, 32 x
+// U[8000, 16000] at 32 / 8 268 / 294; short contexts lose up to 10%: 16 x U[1250, 2500] at 16 / 8 29.6 / 27.0, 100 x
+// U[300, 600] 45.9 / 42.4).
 template <int GP, bool FUSED>
 int dispatch_mfma(const DecodeArgs &a, int batch, hipStream_t stream) {
   if (a.max_ctx > kMaxContext) return NVAMD_EUNSUPPORTED;
   const int64_t units = (int64_t)batch * a.num_kv_heads;
   switch (whole_waves(a, batch)) {
-    case 2: return launch_mfma<GP, 2, true, FUSED>(a, batch, stream);
-    case 4: return launch_mfma<GP, 4, true, FUSED>(a, batch, stream);
-    case 8: return launch_mfma<GP, 8, true, FUSED>(a, batch, stream);
+    case 2: return launch_mfma<GP, 2, 1, true, FUSED>(a, batch, stream);
+    case 4: return launch_mfma<GP, 4, 1, true, FUSED>(a, batch, stream);
+    case 8: return launch_mfma<GP, 8, 1, true, FUSED>(a, batch, stream);
     default: break;
   }
-  if ((GP == 8 && units * ceil_div(a.max_ctx, 256) > 8192) || (a.max_ctx > 16384 && units < 64))
-    return launch_mfma<GP, 8, false, FUSED>(a, batch, stream);
-  return launch_mfma<GP, 4, false, FUSED>(a, batch, stream);
+  if constexpr (GP == 8) {
+    if (units * ceil_div(a.max_ctx, 256) > 8192 || (a.max_ctx > 16384 && units < 64))
+      return launch_mfma<GP, 8, 1, false, FUSED>(a, batch, stream);
+  } else if (a.max_ctx > 16384) {
+    return launch_mfma<GP, 4, 2, false, FUSED>(a, batch, stream);
+  }
+  return launch_mfma<GP, 4, 1, false, FUSED>(a, batch, stream);
 }
 
 }  // namespace
