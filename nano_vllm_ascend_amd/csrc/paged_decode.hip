@@ -3,10 +3,10 @@
 //
 // Work decomposition (split-KV, one kernel):
 //   a workgroup of NW waves owns one (sequence b, kv head g, partition p) of
-//   PART = NW * 64 consecutive context tokens, for all GQA query heads
+//   PART = NW * CPW * 64 consecutive context tokens, for all GQA query heads
 //   that read kv head g, so every K/V byte is read from HBM once.  Each wave
-//   owns 64 tokens.  Groups of 1 or 2 query heads run on v_dot2 (this kernel), larger ones on
-//   MFMA (the variant below).  The grid is 1-D over the items in b, g, p
+//   owns CPW chunks of 64 tokens.  Groups of 1 or 2 query heads run on v_dot2 (this kernel) up to
+//   bounds of kMaxDots tokens, everything else on MFMA (the variant below).  The grid is 1-D over the items in b, g, p
 //   order with p fastest, counted over the partitions that exist for the
 //   device-side context lengths: a unit's partitions run side by side, so its
 //   merge overlaps other units' loads, and the slack a loose context bound adds
@@ -59,6 +59,7 @@ constexpr int kPartFloats = 132;  // max, sum, 128 accumulators, 2 pad (16-byte 
 constexpr int kCounterSlots = 16384;
 constexpr size_t kCounterBytes = kCounterSlots * sizeof(int);
 constexpr int kMaxGroups = 4096;  // workgroups of an MFMA launch; each takes every kMaxGroups-th item
+constexpr int kMaxDots = 32768;  // largest context bound of the dot-product kernel: 64 partitions of 512 tokens
 constexpr int kMaxContext = 131072;  // largest context bound of a call
 constexpr int kMinPart = 256;  // smallest partition of a split launch (sizes the workspace)
 
@@ -159,14 +160,16 @@ __device__ __forceinline__ void load_block(__amdgpu_buffer_rsrc_t rsrc, int byte
   }
 }
 
-// GQA 1 and 2 fit 128 VGPRs without spills: four waves per SIMD.
-template <int GQA, int NW, bool WHOLE, bool FUSED>
+// GQA 1, and GQA 2 with one chunk per wave, fit 128 VGPRs without spills: four waves per SIMD.
+template <int GQA, int NW, int CPW, bool WHOLE, bool FUSED>
 __global__ void __launch_bounds__(NW * 64)
-__attribute__((amdgpu_waves_per_eu(4)))
+__attribute__((amdgpu_waves_per_eu(GQA == 1 || CPW == 1 ? 4 : 1)))
 paged_decode_kernel(DecodeArgs a) {
   constexpr int D = kHeadDim;
-  constexpr int TILES = 4;        // tiles of 16 rows per wave
-  constexpr int WT = 16 * TILES;  // tokens per wave
+  static_assert(GQA <= 2, "larger groups run on MFMA");
+  constexpr int TILES = 4;        // tiles of 16 rows per chunk
+  constexpr int CT = 16 * TILES;  // tokens per chunk
+  constexpr int WT = CPW * CT;    // tokens per wave
   constexpr int PART = NW * WT;
 
   const int hkv = a.num_kv_heads;
@@ -350,120 +353,126 @@ paged_decode_kernel(DecodeArgs a) {
       }
       __builtin_amdgcn_s_waitcnt(0);  // vmcnt counts stores on gfx9: they are acknowledged
     }
+    if constexpr (CPW > 1) {  // several chunks per wave: normalise once, before the loop
+      if (t_begin < t_end) norm_queries();
+    }
   }
 
   if (t_begin < t_end) {
     const int last_tile = (t_end - 1) & ~15;
-    KVTile T[TILES];
-    // the chunk's block-table entries first, so their scalar loads share one wait
-    int blk_t[TILES];
+#pragma unroll 1
+    for (int tc = t_begin; tc < t_end; tc += CT) {
+      KVTile T[TILES];
+      // the chunk's block-table entries first, so their scalar loads share one wait
+      int blk_t[TILES];
 #pragma unroll
-    for (int i = 0; i < TILES; ++i)
-      blk_t[i] = FUSED ? first_blk[i] : bt_row[min(t_begin + 16 * i, last_tile) >> a.bs_log2];
-#pragma unroll
-    for (int i = 0; i < TILES; ++i) {
-      const int t0 = min(t_begin + 16 * i, last_tile);
-      int blk = blk_t[i];
-      if ((unsigned)blk >= (unsigned)a.num_blocks) err_bits |= NVAMD_ERR_BLOCK;
-      blk = min(max(blk, 0), a.num_blocks - 1);               // never leave the pool
-      const int64_t slot = ((int64_t)blk << a.bs_log2) + (t0 & bs_mask) + r;
-      const int64_t off = slot * row_elems + (int64_t)g * D + 8 * c;
-      const u16 *kp = a.k_cache + off;
-      const u16 *vp = a.v_cache + off;
-      // K/V are read once per step.  Bandwidth-bound (split) launches use nontemporal loads,
-      // which keep them from displacing other lines in the L2 (1.08x faster over a
-      // 32 x U[256, 2304] step); latency-bound whole-unit launches use plain loads, whose
-      // round trip is shorter (1.16x faster over a 4 x U[1, 512] step).
-      auto ld = [](const u16 *ptr) { return WHOLE ? ld16(ptr) : ld16_stream(ptr); };
-      T[i].ka0 = ld(kp);
-      T[i].ka1 = ld(kp + 64);
-      T[i].kb0 = ld(kp + step8);
-      T[i].kb1 = ld(kp + step8 + 64);
-      T[i].va0 = ld(vp);
-      T[i].va1 = ld(vp + 64);
-      T[i].vb0 = ld(vp + step8);
-      T[i].vb1 = ld(vp + step8 + 64);
-    }
-    if constexpr (FUSED) norm_queries();
-    // QK for the chunk: s[tile][row a/b][head]
-    float s[TILES][2][GQA];
-#pragma unroll
-    for (int i = 0; i < TILES; ++i) {
-#pragma unroll
-      for (int j = 0; j < GQA; ++j) {
-        float sa = 0.f, sb = 0.f;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          sa = dot2_bf16(qr[j][0][e], T[i].ka0[e], sa);
-          sb = dot2_bf16(qr[j][0][e], T[i].kb0[e], sb);
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          sa = dot2_bf16(qr[j][1][e], T[i].ka1[e], sa);
-          sb = dot2_bf16(qr[j][1][e], T[i].kb1[e], sb);
-        }
-        s[i][0][j] = sa;
-        s[i][1][j] = sb;
-      }
-    }
-    bool ok[TILES][2];
-#pragma unroll
-    for (int i = 0; i < TILES; ++i) {
-      ok[i][0] = (t_begin + 16 * i + r) < t_end;
-      ok[i][1] = (t_begin + 16 * i + 8 + r) < t_end;
-#pragma unroll
-      for (int j = 0; j < GQA; ++j) {
-        const float sa = sum8(s[i][0][j]) * a.scale_log2e;
-        const float sb = sum8(s[i][1][j]) * a.scale_log2e;
-        s[i][0][j] = ok[i][0] ? sa : -INFINITY;
-        s[i][1][j] = ok[i][1] ? sb : -INFINITY;
-      }
-    }
-
-    // Online softmax, one step per chunk, per 8-lane row group.
-    u32 pp[TILES][GQA];
-#pragma unroll
-    for (int j = 0; j < GQA; ++j) {
-      float cm = m[j];
-#pragma unroll
-      for (int i = 0; i < TILES; ++i) cm = fmaxf(cm, fmaxf(s[i][0][j], s[i][1][j]));
-      const float ref = cm == -INFINITY ? 0.f : cm;  // a group with no valid row yet
-      const float alpha = fast_exp2(m[j] - ref);
-      m[j] = cm;
-      float add = 0.f;
+      for (int i = 0; i < TILES; ++i)
+        blk_t[i] = FUSED && CPW == 1 ? first_blk[i] : bt_row[min(tc + 16 * i, last_tile) >> a.bs_log2];
 #pragma unroll
       for (int i = 0; i < TILES; ++i) {
-        pp[i][j] = pack_bf16x2(fast_exp2(s[i][0][j] - ref), fast_exp2(s[i][1][j] - ref));
-        add += bf16_lo(pp[i][j]) + bf16_hi(pp[i][j]);
+        const int t0 = min(tc + 16 * i, last_tile);
+        int blk = blk_t[i];
+        if ((unsigned)blk >= (unsigned)a.num_blocks) err_bits |= NVAMD_ERR_BLOCK;
+        blk = min(max(blk, 0), a.num_blocks - 1);               // never leave the pool
+        const int64_t slot = ((int64_t)blk << a.bs_log2) + (t0 & bs_mask) + r;
+        const int64_t off = slot * row_elems + (int64_t)g * D + 8 * c;
+        const u16 *kp = a.k_cache + off;
+        const u16 *vp = a.v_cache + off;
+        // K/V are read once per step.  Bandwidth-bound (split) launches use nontemporal loads,
+        // which keep them from displacing other lines in the L2 (1.08x faster over a
+        // 32 x U[256, 2304] step); latency-bound whole-unit launches use plain loads, whose
+        // round trip is shorter (1.16x faster over a 4 x U[1, 512] step).
+        auto ld = [](const u16 *ptr) { return WHOLE ? ld16(ptr) : ld16_stream(ptr); };
+        T[i].ka0 = ld(kp);
+        T[i].ka1 = ld(kp + 64);
+        T[i].kb0 = ld(kp + step8);
+        T[i].kb1 = ld(kp + step8 + 64);
+        T[i].va0 = ld(vp);
+        T[i].va1 = ld(vp + 64);
+        T[i].vb0 = ld(vp + step8);
+        T[i].vb1 = ld(vp + step8 + 64);
       }
-      l[j] = l[j] * alpha + add;
-#pragma unroll
-      for (int e = 0; e < 16; ++e) o[j][e] *= alpha;
-    }
-
-    // Rows past the context may hold stale bits (NaN * 0 = NaN): zero their V.
-    if (t_begin + WT > t_end) {
-      const u32x4 z = {0u, 0u, 0u, 0u};
+      if constexpr (FUSED && CPW == 1) norm_queries();  // the wave's only chunk
+      // QK for the chunk: s[tile][row a/b][head]
+      float s[TILES][2][GQA];
 #pragma unroll
       for (int i = 0; i < TILES; ++i) {
-        if (!ok[i][0]) { T[i].va0 = z; T[i].va1 = z; }
-        if (!ok[i][1]) { T[i].vb0 = z; T[i].vb1 = z; }
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < TILES; ++i) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const u32 lo0 = pair_lo(T[i].va0[e], T[i].vb0[e]);
-        const u32 hi0 = pair_hi(T[i].va0[e], T[i].vb0[e]);
-        const u32 lo1 = pair_lo(T[i].va1[e], T[i].vb1[e]);
-        const u32 hi1 = pair_hi(T[i].va1[e], T[i].vb1[e]);
 #pragma unroll
         for (int j = 0; j < GQA; ++j) {
-          o[j][2 * e] = dot2_bf16(pp[i][j], lo0, o[j][2 * e]);
-          o[j][2 * e + 1] = dot2_bf16(pp[i][j], hi0, o[j][2 * e + 1]);
-          o[j][8 + 2 * e] = dot2_bf16(pp[i][j], lo1, o[j][8 + 2 * e]);
-          o[j][8 + 2 * e + 1] = dot2_bf16(pp[i][j], hi1, o[j][8 + 2 * e + 1]);
+          float sa = 0.f, sb = 0.f;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            sa = dot2_bf16(qr[j][0][e], T[i].ka0[e], sa);
+            sb = dot2_bf16(qr[j][0][e], T[i].kb0[e], sb);
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            sa = dot2_bf16(qr[j][1][e], T[i].ka1[e], sa);
+            sb = dot2_bf16(qr[j][1][e], T[i].kb1[e], sb);
+          }
+          s[i][0][j] = sa;
+          s[i][1][j] = sb;
+        }
+      }
+      bool ok[TILES][2];
+#pragma unroll
+      for (int i = 0; i < TILES; ++i) {
+        ok[i][0] = (tc + 16 * i + r) < t_end;
+        ok[i][1] = (tc + 16 * i + 8 + r) < t_end;
+#pragma unroll
+        for (int j = 0; j < GQA; ++j) {
+          const float sa = sum8(s[i][0][j]) * a.scale_log2e;
+          const float sb = sum8(s[i][1][j]) * a.scale_log2e;
+          s[i][0][j] = ok[i][0] ? sa : -INFINITY;
+          s[i][1][j] = ok[i][1] ? sb : -INFINITY;
+        }
+      }
+
+      // Online softmax, one step per chunk, per 8-lane row group.
+      u32 pp[TILES][GQA];
+#pragma unroll
+      for (int j = 0; j < GQA; ++j) {
+        float cm = m[j];
+#pragma unroll
+        for (int i = 0; i < TILES; ++i) cm = fmaxf(cm, fmaxf(s[i][0][j], s[i][1][j]));
+        const float ref = cm == -INFINITY ? 0.f : cm;  // a group with no valid row yet
+        const float alpha = fast_exp2(m[j] - ref);
+        m[j] = cm;
+        float add = 0.f;
+#pragma unroll
+        for (int i = 0; i < TILES; ++i) {
+          pp[i][j] = pack_bf16x2(fast_exp2(s[i][0][j] - ref), fast_exp2(s[i][1][j] - ref));
+          add += bf16_lo(pp[i][j]) + bf16_hi(pp[i][j]);
+        }
+        l[j] = l[j] * alpha + add;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[j][e] *= alpha;
+      }
+
+      // Rows past the context may hold stale bits (NaN * 0 = NaN): zero their V.
+      if (tc + CT > t_end) {
+        const u32x4 z = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int i = 0; i < TILES; ++i) {
+          if (!ok[i][0]) { T[i].va0 = z; T[i].va1 = z; }
+          if (!ok[i][1]) { T[i].vb0 = z; T[i].vb1 = z; }
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < TILES; ++i) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const u32 lo0 = pair_lo(T[i].va0[e], T[i].vb0[e]);
+          const u32 hi0 = pair_hi(T[i].va0[e], T[i].vb0[e]);
+          const u32 lo1 = pair_lo(T[i].va1[e], T[i].vb1[e]);
+          const u32 hi1 = pair_hi(T[i].va1[e], T[i].vb1[e]);
+#pragma unroll
+          for (int j = 0; j < GQA; ++j) {
+            o[j][2 * e] = dot2_bf16(pp[i][j], lo0, o[j][2 * e]);
+            o[j][2 * e + 1] = dot2_bf16(pp[i][j], hi0, o[j][2 * e + 1]);
+            o[j][8 + 2 * e] = dot2_bf16(pp[i][j], lo1, o[j][8 + 2 * e]);
+            o[j][8 + 2 * e + 1] = dot2_bf16(pp[i][j], hi1, o[j][8 + 2 * e + 1]);
+          }
         }
       }
     }
@@ -642,16 +651,16 @@ paged_decode_kernel(DecodeArgs a) {
   }
 }
 
-template <int GQA, int NW, bool WHOLE, bool FUSED>
+template <int GQA, int NW, int CPW, bool WHOLE, bool FUSED>
 int launch(DecodeArgs a, int batch, hipStream_t stream) {
-  constexpr int PART = NW * 64;
+  constexpr int PART = NW * CPW * 64;
   a.max_parts = ceil_div(a.max_ctx, PART);
   if (a.max_parts > 64) return NVAMD_EUNSUPPORTED;  // merge stage holds <= 64 partitions
   if (WHOLE && a.max_parts != 1) return NVAMD_EINVAL;
   a.batch = batch;
   // One workgroup per possible (b, g, p); the ones past the last existing item exit at once.
   dim3 grid((unsigned)((int64_t)batch * a.num_kv_heads * a.max_parts));
-  hipLaunchKernelGGL((paged_decode_kernel<GQA, NW, WHOLE, FUSED>), grid, dim3(NW * 64), 0, stream, a);
+  hipLaunchKernelGGL((paged_decode_kernel<GQA, NW, CPW, WHOLE, FUSED>), grid, dim3(NW * 64), 0, stream, a);
   return launch_status();
 }
 
@@ -1286,11 +1295,13 @@ int whole_waves(const DecodeArgs &a, int batch) {
 template <int GQA, bool FUSED>
 int dispatch(const DecodeArgs &a, int batch, hipStream_t stream) {
   switch (whole_waves(a, batch)) {
-    case 2: return launch<GQA, 2, true, FUSED>(a, batch, stream);
-    case 4: return launch<GQA, 4, true, FUSED>(a, batch, stream);
-    case 8: return launch<GQA, 8, true, FUSED>(a, batch, stream);
-    default: return launch<GQA, 4, false, FUSED>(a, batch, stream);
+    case 2: return launch<GQA, 2, 1, true, FUSED>(a, batch, stream);
+    case 4: return launch<GQA, 4, 1, true, FUSED>(a, batch, stream);
+    case 8: return launch<GQA, 8, 1, true, FUSED>(a, batch, stream);
+    default: break;
   }
+  return a.max_ctx <= kMaxDots / 2 ? launch<GQA, 4, 1, false, FUSED>(a, batch, stream)
+                                   : launch<GQA, 4, 2, false, FUSED>(a, batch, stream);
 }
 
 // Partitions of the MFMA variant: 256 tokens, or 512 (half the partial records) in two cases.
@@ -1388,16 +1399,24 @@ int fill_decode_args(DecodeArgs &a, void *out, int64_t out_stride, const void *q
 // the rest; each launch re-reads the group's K/V, and only the first stores the fused step's new k / v.
 // Groups of 1 and 2 heads keep the dot-product kernel, which is as fast over large batches and faster
 // where latency counts (at 2 heads 33.6 against 33.9 us over 32 x U[256, 2304], 6.6 against 7.1 us over 4 x U[1, 512]; at 4
-// heads the MFMA variant leads: 35.7 against 36.5 us and 7.2 against 9.6 us), up to the 64 partitions of 256
-// tokens that its merge holds.
+// heads the MFMA variant leads: 35.7 against 36.5 us and 7.2 against 9.6 us), up to the 64 partitions that its merge
+// holds: 256 tokens each, and 512 of two chunks per wave under bounds past 16,384, there up to 8,192 workgroups (at 20,480,
+// dot product / MFMA: 16 / 8 heads 28.0 / 29.6 us over 16 x U[1250, 2500], 8.9 / 9.9 over 4 x U[1, 512]; 8 / 8 8.6 / 10.2 over the
+// latter; 2 / 1 10.4 / 12.1 over 16 x U[1250, 2500]).  More of them are mostly empty ones, which the MFMA variant's item
+// loop saves (16 / 8 heads over 100 x U[300, 600] at 20,480 60 / 44 us, 100 x U[1250, 2500] at 32,768 167 / 138).  Past
+// 32,768 tokens the dot-product kernel would need 1,024-token partitions, whose few workgroups lose to the MFMA variant where
+// contexts are short for the bound (at 40,960: 2 x U[1250, 2500] at 16 / 8 16.8 / 12.4, 100 x U[300, 600] 58.2 / 45.9, 100 x
+// U[1250, 2500] 150 / 133) and lead it where they are long for the batch (2 x U[8000, 16000] at 16 / 8 20.2 / 21.9, 8 x the
+// same at 8 / 8 78.3 / 81.4, 100 x U[1250, 2500] at 2 / 1 19.6 / 22.1); the host cannot tell these apart.
 template <bool FUSED>
 int dispatch_gqa(DecodeArgs a, int gqa, int batch, hipStream_t stream) {
   a.q_group = gqa;
+  const int64_t items = (int64_t)batch * a.num_kv_heads * ceil_div(a.max_ctx, 512);
   for (int head0 = 0; head0 < gqa;) {
     a.q_head0 = head0;
     a.q_sub = min(gqa - head0, 8);
     a.store_new = head0 == 0;
-    const bool dots = a.q_sub <= 2 && a.max_ctx <= 16384;
+    const bool dots = a.q_sub <= 2 && (a.max_ctx <= kMaxDots / 2 || (a.max_ctx <= kMaxDots && items <= 8192));
     const int st = dots ? (a.q_sub == 2 ? dispatch<2, FUSED>(a, batch, stream) : dispatch<1, FUSED>(a, batch, stream))
                  : a.q_sub <= 4 ? dispatch_mfma<4, FUSED>(a, batch, stream)
                                 : dispatch_mfma<8, FUSED>(a, batch, stream);

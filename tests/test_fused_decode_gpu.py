@@ -204,3 +204,11 @@ def test_fused_step_mfma_ignores_stale_rows(device, heads, bound):
     assert torch.equal(out, ref)
     err = (out.cpu().float() - case.oracle()).abs().max().item()
     assert err <= BF16_TOL, err
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,bound", [((16, 8), 20480), ((8, 8), 20480), ((16, 8), 40960), ((3, 1), 20480)])
+def test_fused_step_two_chunks_per_wave(device, heads, bound):
+    """The new token in a wave's first and second chunk, at its edges, and first of a partition of its own."""
+    ctx = [1, 64, 65, 128, 129, 255, 256, 257, 320, 321, 512, 513, 577, 769, 1024, 1025, 2100]
+    check(Case(device, len(ctx), 0, 0, 100, seed=13, heads=heads, context_lens=ctx), max_ctx=bound)

@@ -67,12 +67,12 @@ def test_decode_long_contexts_many_partitions(device):
 @pytest.mark.gpu
 @pytest.mark.parametrize("lo,hi,seed", [(16400, 32000, 23), (33000, 40960, 29)])
 def test_decode_very_long_contexts_several_chunks_per_wave(device, lo, hi, seed):
-    """Bounds past 64 partitions of 256 tokens (16,384 tokens) give each wave two 64-token chunks,
-    bounds past 32,768 tokens four; the second case reaches Qwen3's 40,960 positions."""
+    """Bounds past 64 partitions of 256 tokens (16,384 tokens) give each wave two 64-token chunks, in the
+    dot-product kernel up to 32,768 tokens and on MFMA past them; the second case reaches Qwen3's 40,960 positions."""
     work = W.make_decode(2, lo, hi, 2 * (hi // 128 + 1), seed=seed, device=device)
     assert max(work.context_lens_list) > 16384
     check(work)
-    check(work, max_ctx=40960)  # the four-chunk launch over shorter contexts
+    check(work, max_ctx=40960)  # the MFMA launch over shorter contexts
 
 
 @pytest.mark.gpu
@@ -360,3 +360,19 @@ def test_decode_infinite_values_stay_infinite(device, heads, bound):
     assert bool(ref.isinf().any()) and bool(ref.isnan().any())
     assert torch.equal(out.isnan(), ref.isnan()) and torch.equal(out[ref.isinf()], ref[ref.isinf()])
     assert (out[finite] - ref[finite]).abs().max().item() <= TOL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,bound", [((16, 8), 16384), ((16, 8), 16385), ((8, 8), 32768), ((16, 8), 32768),
+                                         ((16, 8), 32769), ((8, 8), 32769), ((3, 1), 16385), ((8, 2), 16385)])
+def test_decode_two_chunks_per_wave(device, heads, bound):
+    """Both kernels' two-chunk partitions (consecutive chunks of a wave in the dot-product kernel, chunks 256 tokens apart on
+    MFMA) and the bounds on either side of each: contexts at the edges of a chunk, of the waves' second chunks and of a
+    partition, few enough launches for the dot-product kernel and, at 34 sequences, too many."""
+    hq, hkv = heads
+    ctx = [1, 63, 64, 65, 127, 128, 129, 255, 256, 257, 319, 320, 321, 511, 512, 513, 700, 768, 769, 1025, 0, 1537, 5000]
+    for extra in (0, 34 - len(ctx)):
+        lens = ctx + [40 + 77 * i for i in range(extra)]
+        work = W.make_decode(len(lens), 0, 0, 260, seed=hq + extra, device=device, num_heads=hq, num_kv_heads=hkv,
+                             context_lens=lens)
+        check(work, max_ctx=bound)
