@@ -128,20 +128,16 @@ __device__ __forceinline__ int wave_incl_scan(int v, int lane) {
 }
 
 // 2 * GQA consecutive floats of a partial record through an agent-coherent buffer range
-// (write-through stores, loads that bypass the non-coherent caches): 8 bytes for one head,
-// 16-byte pieces for two or four.
+// (write-through stores, loads that bypass the non-coherent caches): 8 bytes for one head, 16 for two.
 template <int GQA>
 __device__ __forceinline__ void store_block(__amdgpu_buffer_rsrc_t rsrc, int byte_off, const float (&v)[2 * GQA]) {
   if constexpr (GQA == 1) {
     __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(v[0]), __float_as_uint(v[1])}, rsrc, byte_off, 0,
                                           kCachePolicyAgent);
   } else {
-#pragma unroll
-    for (int h = 0; h < GQA / 2; ++h)
-      __builtin_amdgcn_raw_buffer_store_b128(
-          u32x4{__float_as_uint(v[4 * h]), __float_as_uint(v[4 * h + 1]), __float_as_uint(v[4 * h + 2]),
-                __float_as_uint(v[4 * h + 3])},
-          rsrc, byte_off + 16 * h, 0, kCachePolicyAgent);
+    __builtin_amdgcn_raw_buffer_store_b128(
+        u32x4{__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3])}, rsrc,
+        byte_off, 0, kCachePolicyAgent);
   }
 }
 template <int GQA>
@@ -151,12 +147,9 @@ __device__ __forceinline__ void load_block(__amdgpu_buffer_rsrc_t rsrc, int byte
     v[0] = __uint_as_float(x[0]);
     v[1] = __uint_as_float(x[1]);
   } else {
+    const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(rsrc, byte_off, 0, kCachePolicyAgent);
 #pragma unroll
-    for (int h = 0; h < GQA / 2; ++h) {
-      const u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(rsrc, byte_off + 16 * h, 0, kCachePolicyAgent);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[4 * h + e] = __uint_as_float(x[e]);
-    }
+    for (int e = 0; e < 4; ++e) v[e] = __uint_as_float(x[e]);
   }
 }
 
@@ -547,9 +540,9 @@ paged_decode_kernel(DecodeArgs a) {
 
   // A partition's record (GQA * kPartFloats floats): the heads' (max, sum) pairs, then lane l's
   // accumulators of every head (dims 2l, 2l+1 of head j at 2j, 2j+1), 2 * GQA floats at
-  // kHdr + 2 * GQA * l, so a lane publishes and reads its share of a partition in 16-byte pieces.
+  // kHdr + 2 * GQA * l, so a lane publishes and reads its share of a partition in one piece.
   constexpr int kRec = GQA * kPartFloats;
-  constexpr int kHdr = GQA <= 2 ? 4 : 2 * GQA;
+  constexpr int kHdr = 4;
   static_assert(kHdr + 2 * GQA * 64 <= kRec, "partial record");
   float *part_base = a.partials + (((int64_t)b * hkv + g) * a.max_parts) * kRec;
   // Buffer range over exactly the n_parts partitions: reads past them return zeros without a
@@ -585,7 +578,7 @@ paged_decode_kernel(DecodeArgs a) {
   // Merge.  Lane x holds partition x's (max, sum) of every head; the accumulators of the
   // first MP partitions are loaded in the same round (every load issued before the first
   // use, so the merge waits for one memory round trip), later ones 8 partitions per round.
-  constexpr int MP = GQA <= 2 ? 16 : 8;
+  constexpr int MP = 16;
   float pm[GQA], pl[GQA], v0f[GQA][MP], v1f[GQA][MP];
   {
     float hx[2 * GQA];
