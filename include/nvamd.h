@@ -305,9 +305,7 @@ int nvamd_argmax_rows(const void *logits, int64_t row_stride, int rows,
 /*   stride.  flags: NVAMD_GEMM_X_TILED -- x is tiled with 16 * ceil(m/16)    */
 /*   rows (x_stride unused; rows past m only reach dropped outputs);          */
 /*   NVAMD_GEMM_Y_TILED -- y is tiled [16 * ceil(m/16), n] (y_stride unused;  */
-/*   rows past m are neither read as inputs nor written);                     */
-/*   NVAMD_GEMM_W_ROWS -- w_tiled is the row-major weight itself, rows of k   */
-/*   elements one after another (with x_ssq: NVAMD_EUNSUPPORTED).             */
+/*   rows past m are neither read as inputs nor written).                     */
 /* Prologue: with x_ssq == NULL, a = x.  Otherwise x is the residual stream,  */
 /*   x_ssq[r * (k/32) + t] holds the sum of squares of x[r, 32t..32t+31], and */
 /*   a = bf16((x * rsqrt(sum_t x_ssq / k + eps)) * norm_weight); k <= 2048   */
@@ -333,7 +331,6 @@ size_t nvamd_skinny_linear_workspace_size(int n, int k, int epilogue);
 
 #define NVAMD_GEMM_X_TILED 1
 #define NVAMD_GEMM_Y_TILED 2
-#define NVAMD_GEMM_W_ROWS 4
 
 int nvamd_skinny_linear(const void *x, int64_t x_stride, const float *x_ssq,
                         const void *norm_weight, float eps,
@@ -341,6 +338,15 @@ int nvamd_skinny_linear(const void *x, int64_t x_stride, const float *x_ssq,
                         float *y_ssq, int epilogue, int flags, int m, int n,
                         int k, void *workspace, size_t workspace_bytes,
                         hipStream_t stream);
+
+/* skinny_linear_rows: the same without the prologue, over the row-major      */
+/*   weight itself (rows of k elements one after another, 16-byte aligned):   */
+/*   for weights that other code changes or that are too large to hold twice. */
+int nvamd_skinny_linear_rows(const void *x, int64_t x_stride, const void *w,
+                             void *y, int64_t y_stride, float *y_ssq,
+                             int epilogue, int flags, int m, int n, int k,
+                             void *workspace, size_t workspace_bytes,
+                             hipStream_t stream);
 
 int nvamd_embed_rows(const int64_t *ids, const void *table,
                      int64_t table_stride, int vocab, void *out,

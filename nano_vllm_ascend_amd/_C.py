@@ -79,6 +79,10 @@ _SIGNATURES = {
         _c_int,
         [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_float, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_int, _c_int, _c_int, _c_int,
          _c_int, _c_ptr, _c_size, _c_ptr]),
+    "nvamd_skinny_linear_rows": (
+        _c_int,
+        [_c_ptr, _c_i64, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr, _c_size,
+         _c_ptr]),
     "nvamd_embed_rows": (
         _c_int, [_c_ptr, _c_ptr, _c_i64, _c_int, _c_ptr, _c_i64, _c_int, _c_ptr, _c_int, _c_int, _c_ptr]),
     "nvamd_qk_norm_rope": (
@@ -607,7 +611,6 @@ def alloc_skinny_workspace(shapes, device) -> torch.Tensor:
 
 GEMM_X_TILED = 1
 GEMM_Y_TILED = 2
-GEMM_W_ROWS = 4
 
 
 def is_tiled(t: torch.Tensor) -> bool:
@@ -655,6 +658,7 @@ def skinny_linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = N
     _bf16_cuda("w", w)
     if w_rows:
         _require(w.dim() == 2 and w.is_contiguous(), "w must be a contiguous [N, K] matrix")
+        _require(x_ssq is None, "a row-major weight takes no norm prologue")
         wn, wk = w.shape
     else:
         _require(is_tiled(w), "w must be tiled: tile(W)")
@@ -688,11 +692,14 @@ def skinny_linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = N
     need = skinny_linear_workspace_size(n, k, epilogue) if n % 32 == 0 and k % 256 == 0 else 0
     if need and workspace is None:
         workspace = torch.zeros(need, dtype=torch.uint8, device=x.device)
-    flags = (GEMM_X_TILED if x_tiled else 0) | (GEMM_Y_TILED if y_tiled else 0) | (GEMM_W_ROWS if w_rows else 0)
-    status = lib.nvamd_skinny_linear(
-        x.data_ptr(), 0 if x_tiled else _row_stride(x), _ptr(x_ssq), _ptr(norm_weight), float(eps), w.data_ptr(),
-        out.data_ptr(), 0 if y_tiled else out.stride(0), _ptr(y_ssq), int(epilogue), flags, m, n, k,
-        _ptr(workspace), workspace.numel() if workspace is not None else 0, _stream())
+    flags = (GEMM_X_TILED if x_tiled else 0) | (GEMM_Y_TILED if y_tiled else 0)
+    tail = (out.data_ptr(), 0 if y_tiled else out.stride(0), _ptr(y_ssq), int(epilogue), flags, m, n, k, _ptr(workspace),
+            workspace.numel() if workspace is not None else 0, _stream())
+    x_args = (x.data_ptr(), 0 if x_tiled else _row_stride(x))
+    if w_rows:
+        status = lib.nvamd_skinny_linear_rows(*x_args, w.data_ptr(), *tail)
+    else:
+        status = lib.nvamd_skinny_linear(*x_args, _ptr(x_ssq), _ptr(norm_weight), float(eps), w.data_ptr(), *tail)
     _check(status, "nvamd_skinny_linear")
     return out
 

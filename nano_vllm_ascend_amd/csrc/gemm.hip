@@ -482,11 +482,64 @@ int dispatch(const GemmArgs &a, const Plan &p, int grid, bool wide, hipStream_t 
 }
 
 template <int EPI>
-int dispatch_layout(const GemmArgs &a, const Plan &p, int grid, bool wide, int flags, hipStream_t stream) {
-  const bool norm = a.x_ssq != nullptr;
-  if (flags & NVAMD_GEMM_W_ROWS)  // no NORM prologue (refused before)
-    return dispatch<EPI, false, true>(a, p, grid, wide, stream);
+int dispatch_layout(const GemmArgs &a, const Plan &p, int grid, bool wide, bool w_rows, hipStream_t stream) {
+  const bool norm = a.x_ssq != nullptr;  // never with w_rows
+  if (w_rows) return dispatch<EPI, false, true>(a, p, grid, wide, stream);
   return norm ? dispatch<EPI, true, false>(a, p, grid, wide, stream) : dispatch<EPI, false, false>(a, p, grid, wide, stream);
+}
+
+int skinny_linear(const void *x, int64_t x_stride, const float *x_ssq, const void *norm_weight, float eps, const void *w,
+                  bool w_rows, void *y, int64_t y_stride, float *y_ssq, int epilogue, int flags, int m, int n, int k,
+                  void *workspace, size_t workspace_bytes, hipStream_t stream) {
+  if (m == 0) return NVAMD_OK;
+  if (!x || !w || !y || m < 0 || n <= 0 || k <= 0 || epilogue < 0 || epilogue > 2 ||
+      (flags & ~(NVAMD_GEMM_X_TILED | NVAMD_GEMM_Y_TILED)))
+    return NVAMD_EINVAL;
+  if (m > 32 * kMaxSlabs || n % 32 != 0 || k % 256 != 0) return NVAMD_EUNSUPPORTED;
+  const bool x_tiled = flags & NVAMD_GEMM_X_TILED, y_tiled = flags & NVAMD_GEMM_Y_TILED;
+  const bool norm = x_ssq != nullptr;
+  if (norm && !norm_weight) return NVAMD_EINVAL;
+  if (norm && k > kMaxNormK) return NVAMD_EUNSUPPORTED;
+  if (epilogue == kEpiResid && !y_ssq) return NVAMD_EINVAL;
+  if (!aligned16(x) || !aligned16(w) || (reinterpret_cast<uintptr_t>(y) & 7u) ||
+      (!x_tiled && (x_stride % 8 || x_stride < k)) || (!y_tiled && (y_stride < n || y_stride % 4)) ||
+      (norm && (!aligned16(x_ssq) || !aligned16(norm_weight))))
+    return NVAMD_EINVAL;
+  const bool wide = wide_rows(m, k, norm, epilogue);
+  const Plan p = make_plan(n, k, epilogue, m, w_rows);
+  const int groups = n / (16 * p.nt);
+  if ((k / p.ks) % (32 * p.kb) != 0) return NVAMD_EUNSUPPORTED;  // whole wave blocks per slice
+  const int slabs = wide ? (m + 63) / 64 : (m + 31) / 32;
+  if (p.ks > 1) {
+    if (groups * slabs > kCounterSlots) return NVAMD_EUNSUPPORTED;
+    if (!workspace || !aligned16(workspace) || workspace_bytes < workspace_bytes_for(p, n, epilogue))
+      return NVAMD_EWORKSPACE;
+  }
+  GemmArgs a;
+  a.x = static_cast<const u16 *>(x);
+  a.x_stride = x_stride;
+  a.x_ssq = x_ssq;
+  a.norm_w = static_cast<const u16 *>(norm_weight);
+  a.eps = eps;
+  a.w = static_cast<const u16 *>(w);
+  a.y = static_cast<u16 *>(y);
+  a.y_stride = y_stride;
+  a.x_tiled = x_tiled;
+  a.y_tiled = y_tiled;
+  a.y_ssq = y_ssq;
+  a.m = m;
+  a.n = n;
+  a.k = k;
+  a.ks = p.ks;
+  a.k_slice = k / p.ks;
+  a.counters = static_cast<int *>(workspace);
+  a.partials = workspace ? reinterpret_cast<float *>(static_cast<char *>(workspace) + kCounterBytes) : nullptr;
+  const int grid = groups * p.ks * slabs;
+  switch (epilogue) {
+    case kEpiSilu: return dispatch_layout<kEpiSilu>(a, p, grid, wide, w_rows, stream);
+    case kEpiResid: return dispatch_layout<kEpiResid>(a, p, grid, wide, w_rows, stream);
+    default: return dispatch_layout<kEpiStore>(a, p, grid, wide, w_rows, stream);
+  }
 }
 
 }  // namespace
@@ -505,53 +558,13 @@ extern "C" int nvamd_skinny_linear(const void *x, int64_t x_stride, const float 
                                    float eps, const void *w_tiled, void *y, int64_t y_stride, float *y_ssq,
                                    int epilogue, int flags, int m, int n, int k, void *workspace,
                                    size_t workspace_bytes, hipStream_t stream) {
-  if (m == 0) return NVAMD_OK;
-  if (!x || !w_tiled || !y || m < 0 || n <= 0 || k <= 0 || epilogue < 0 || epilogue > 2 ||
-      (flags & ~(NVAMD_GEMM_X_TILED | NVAMD_GEMM_Y_TILED | NVAMD_GEMM_W_ROWS)))
-    return NVAMD_EINVAL;
-  if (m > 32 * kMaxSlabs || n % 32 != 0 || k % 256 != 0) return NVAMD_EUNSUPPORTED;
-  const bool x_tiled = flags & NVAMD_GEMM_X_TILED, y_tiled = flags & NVAMD_GEMM_Y_TILED;
-  const bool norm = x_ssq != nullptr;
-  if (norm && !norm_weight) return NVAMD_EINVAL;
-  if (norm && (k > kMaxNormK || (flags & NVAMD_GEMM_W_ROWS))) return NVAMD_EUNSUPPORTED;
-  if (epilogue == kEpiResid && !y_ssq) return NVAMD_EINVAL;
-  if (!aligned16(x) || !aligned16(w_tiled) || (reinterpret_cast<uintptr_t>(y) & 7u) ||
-      (!x_tiled && (x_stride % 8 || x_stride < k)) || (!y_tiled && (y_stride < n || y_stride % 4)) ||
-      (norm && (!aligned16(x_ssq) || !aligned16(norm_weight))))
-    return NVAMD_EINVAL;
-  const bool wide = wide_rows(m, k, norm, epilogue);
-  const Plan p = make_plan(n, k, epilogue, m, flags & NVAMD_GEMM_W_ROWS);
-  const int groups = n / (16 * p.nt);
-  if ((k / p.ks) % (32 * p.kb) != 0) return NVAMD_EUNSUPPORTED;  // whole wave blocks per slice
-  const int slabs = wide ? (m + 63) / 64 : (m + 31) / 32;
-  if (p.ks > 1) {
-    if (groups * slabs > kCounterSlots) return NVAMD_EUNSUPPORTED;
-    if (!workspace || !aligned16(workspace) || workspace_bytes < workspace_bytes_for(p, n, epilogue))
-      return NVAMD_EWORKSPACE;
-  }
-  GemmArgs a;
-  a.x = static_cast<const u16 *>(x);
-  a.x_stride = x_stride;
-  a.x_ssq = x_ssq;
-  a.norm_w = static_cast<const u16 *>(norm_weight);
-  a.eps = eps;
-  a.w = static_cast<const u16 *>(w_tiled);
-  a.y = static_cast<u16 *>(y);
-  a.y_stride = y_stride;
-  a.x_tiled = x_tiled;
-  a.y_tiled = y_tiled;
-  a.y_ssq = y_ssq;
-  a.m = m;
-  a.n = n;
-  a.k = k;
-  a.ks = p.ks;
-  a.k_slice = k / p.ks;
-  a.counters = static_cast<int *>(workspace);
-  a.partials = workspace ? reinterpret_cast<float *>(static_cast<char *>(workspace) + kCounterBytes) : nullptr;
-  const int grid = groups * p.ks * slabs;
-  switch (epilogue) {
-    case kEpiSilu: return dispatch_layout<kEpiSilu>(a, p, grid, wide, flags, stream);
-    case kEpiResid: return dispatch_layout<kEpiResid>(a, p, grid, wide, flags, stream);
-    default: return dispatch_layout<kEpiStore>(a, p, grid, wide, flags, stream);
-  }
+  return skinny_linear(x, x_stride, x_ssq, norm_weight, eps, w_tiled, false, y, y_stride, y_ssq, epilogue, flags, m, n, k,
+                       workspace, workspace_bytes, stream);
+}
+
+extern "C" int nvamd_skinny_linear_rows(const void *x, int64_t x_stride, const void *w, void *y, int64_t y_stride,
+                                        float *y_ssq, int epilogue, int flags, int m, int n, int k, void *workspace,
+                                        size_t workspace_bytes, hipStream_t stream) {
+  return skinny_linear(x, x_stride, nullptr, nullptr, 0.f, w, true, y, y_stride, y_ssq, epilogue, flags, m, n, k,
+                       workspace, workspace_bytes, stream);
 }

@@ -97,6 +97,24 @@ def test_skinny_linear_argument_errors():
     assert call(epi=2, y_ssq=None) == EINVAL               # the residual epilogue writes sums of squares
 
 
+def test_skinny_linear_rows_argument_errors():
+    lib = _C.load()
+
+    def call(**over):
+        args = dict(x=A, x_stride=4096, w=A, y=A, y_stride=4096, y_ssq=None, epi=0, flags=0, m=32, n=4096, k=4096, ws=None,
+                    ws_bytes=0, stream=None)
+        args.update(over)
+        return lib.nvamd_skinny_linear_rows(*args.values())
+
+    assert call(m=0) == 0
+    assert call(w=None) == EINVAL and call(w=A + 8) == EINVAL and call(x_stride=4088) == EINVAL
+    assert call(flags=4) == EINVAL
+    assert call(m=129) == EUNSUPPORTED and call(k=4000) == EUNSUPPORTED
+    assert call(epi=2) == EINVAL                            # no sums of squares
+    assert call(epi=2, y_ssq=A) == EWORKSPACE               # K split over workgroups
+
+
+
 def test_paged_prefill_rejects_small_blocks():
     lib = _C.load()
     common = dict(out=A, out_stride=2048, q=A, q_stride=2048, k_cache=A, v_cache=A, num_blocks=64)
