@@ -693,8 +693,8 @@ def skinny_linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = N
     if need and workspace is None:
         workspace = torch.zeros(need, dtype=torch.uint8, device=x.device)
     flags = (GEMM_X_TILED if x_tiled else 0) | (GEMM_Y_TILED if y_tiled else 0)
-    tail = (out.data_ptr(), 0 if y_tiled else out.stride(0), _ptr(y_ssq), int(epilogue), flags, m, n, k, _ptr(workspace),
-            workspace.numel() if workspace is not None else 0, _stream())
+    tail = (out.data_ptr(), 0 if y_tiled else out.stride(0), _ptr(y_ssq), int(epilogue), flags, m, n, k,
+            _ptr(workspace), workspace.numel() if workspace is not None else 0, _stream())
     x_args = (x.data_ptr(), 0 if x_tiled else _row_stride(x))
     if w_rows:
         status = lib.nvamd_skinny_linear_rows(*x_args, w.data_ptr(), *tail)

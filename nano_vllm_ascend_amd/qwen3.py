@@ -68,6 +68,11 @@ class _TiledCopy:
                 self.storage = new
         self.current = True
 
+    def operand(self, weight: torch.Tensor) -> dict:
+        """The weight as ``skinny_linear`` takes it: the copy where one was built, else row-major as it is."""
+        copy = self.of(weight)
+        return {"w": weight, "w_rows": True} if copy is None else {"w": copy}
+
 
 class Qwen3Attention(nn.Module):
     def __init__(self, config: Qwen3Config, layer_idx: int, block_size: int, max_model_len: int):
@@ -117,15 +122,14 @@ class Qwen3Attention(nn.Module):
                                            workspace=getattr(attn_metadata, "decode_workspace", None))
 
     def decode_wide(self, x, residual, ssq, t: int, rotary, positions, kv_cache, attn_metadata, workspace):
-        """residual += o_proj(attention(qkv_proj(x))) in place for t rows: x normed and tiled, residual and weights
-        row-major."""
-        qkv = _C.skinny_linear(x, self.qkv_weight, workspace=workspace, m=t, w_rows=True)
+        """residual += o_proj(attention(qkv_proj(x))) in place for t rows: x normed and tiled, residual row-major."""
+        qkv = _C.skinny_linear(x, **self.qkv_tiled.operand(self.qkv_weight), workspace=workspace, m=t)
         q = qkv[:, : self.q_size].view(t, self.num_heads, self.head_dim)
         k = qkv[:, self.q_size : self.q_size + self.kv_size].view(t, self.num_kv_heads, self.head_dim)
         v = qkv[:, self.q_size + self.kv_size :].view(t, self.num_kv_heads, self.head_dim)
         attn = self.decode_attention(q, k, v, rotary, positions, kv_cache, attn_metadata)
-        _C.skinny_linear(attn.reshape(t, self.q_size), self.o_weight, residual, epilogue=_C.EPI_RESID, y_ssq=ssq,
-                         workspace=workspace, w_rows=True)
+        _C.skinny_linear(attn.reshape(t, self.q_size), **self.o_tiled.operand(self.o_weight), out=residual,
+                         epilogue=_C.EPI_RESID, y_ssq=ssq, workspace=workspace)
 
     def decode_fused(self, residual, ssq, t: int, norm: RMSNorm, rotary, positions, kv_cache, attn_metadata,
                      workspace):
@@ -160,11 +164,11 @@ class Qwen3MLP(nn.Module):
         return linear(act, self.down_weight, skinny=False)
 
     def decode_wide(self, x, residual, ssq, t: int, workspace):
-        """residual += mlp(x) in place for t rows: x normed and tiled, residual and weights row-major."""
-        act = _C.skinny_linear(x, self.gate_up_weight, epilogue=_C.EPI_SILU, workspace=workspace, m=t, y_tiled=True,
-                               w_rows=True)
-        _C.skinny_linear(act, self.down_weight, residual, epilogue=_C.EPI_RESID, y_ssq=ssq, workspace=workspace, m=t,
-                         w_rows=True)
+        """residual += mlp(x) in place for t rows: x normed and tiled, residual row-major."""
+        act = _C.skinny_linear(x, **self.gate_up_tiled.operand(self.gate_up_weight), epilogue=_C.EPI_SILU,
+                               workspace=workspace, m=t, y_tiled=True)
+        _C.skinny_linear(act, **self.down_tiled.operand(self.down_weight), out=residual, epilogue=_C.EPI_RESID,
+                         y_ssq=ssq, workspace=workspace, m=t)
 
     def decode_fused(self, residual, ssq, t: int, norm: RMSNorm, workspace):
         """residual += down(silu(gate(norm(residual))) * up(norm(residual))) in place (t <= 128 rows,
@@ -230,8 +234,9 @@ class Qwen3Model(nn.Module):
 
     def forward_decode_wide(self, input_ids_flat, position_ids_flat, kv_cache, attn_metadata, workspace):
         """Decode forward for <= 32 rows at the hidden sizes that the projections' norm prologue does not take:
-        as forward_decode_fused, over the weights themselves, with each RMSNorm in a launch that writes the next
-        projection's tiled operand -- 7 launches per layer.  Returns the final residual stream, row-major."""
+        as forward_decode_fused, over the weights themselves (or the tiled copies that the caller had built), with
+        each RMSNorm in a launch that writes the next projection's tiled operand -- 7 launches per layer.  Returns the
+        final residual stream, row-major."""
         t = input_ids_flat.shape[0]
         residual = F.embedding(input_ids_flat, self.embed_tokens)
         ssq = torch.empty((t, residual.shape[1] // 32), dtype=torch.float32, device=residual.device)
@@ -267,8 +272,8 @@ class Qwen3ForCausalLM(nn.Module):
 
     def build_decode_weights(self) -> None:
         """Tiled copies of the projection and LM head weights for the fused decode path (about the
-        size of the weights again).  Built on the first fused decode; call it again after changing
-        weights in place."""
+        size of the weights again).  Built on the first fused decode, which is that of hidden 1024 and 2048; at
+        other sizes only this call builds them.  Call it again after changing weights in place."""
         if self.lm_head.is_cuda and torch.cuda.is_current_stream_capturing():
             raise RuntimeError("the tiled decode weights must be built before graph capture")
         self._drop_decode_weights()
@@ -297,10 +302,10 @@ class Qwen3ForCausalLM(nn.Module):
 
     def decode_wide(self, rows: int) -> bool:
         """Whether a decode batch of `rows` runs on the skinny GEMMs with the norms in launches of their own, reading
-        the weights as they are.  Up to 32 rows it leads the library GEMMs and separate SiLU (a layer's projections of
-        hidden 4096, 8 / 32 rows: 92 / 101 against 101 / 108 us; 2560: 63 / 71 against 96 / 76); a row-major weight
-        streams 10-30% slower than a tiled copy, which would double the weights' memory and would have to follow
-        every change of the weights."""
+        the weights as they are.  Up to 32 rows it leads the library GEMMs and separate SiLU (a layer's projections at
+        8 / 32 rows, us: hidden 2560 65 / 75 against 95 / 76, 4096 97 / 109 against 102 / 108, 5120 183 / 213 against
+        238 / 258; the norms' launches save another 2); a row-major weight streams 10-30% slower than a tiled copy, which
+        would double the weights' memory and would have to follow every change of the weights."""
         c = self.config
         return (rows <= 32 and self._skinny_shapes(rows) and c.hidden_size % 256 == 0 and c.hidden_size <= 8192
                 and not (c.hidden_size % 1024 == 0 and c.hidden_size <= 2048)

@@ -136,8 +136,8 @@ def test_prefill_and_captured_decode_after_a_failed_and_a_corrected_load(device)
         from nano_vllm_ascend_amd.block_manager import PagedKVCacheMetadata
 
         n = torch.tensor([lens], device=device)
-        md = PagedKVCacheMetadata(block_tables=kwargs["attn_metadata"].block_tables, slot_mapping=n - 1, positions=n - 1,
-                                  context_lens=n.int(), max_context_bound=128,
+        md = PagedKVCacheMetadata(block_tables=kwargs["attn_metadata"].block_tables, slot_mapping=n - 1,
+                                  positions=n - 1, context_lens=n.int(), max_context_bound=128,
                                   decode_workspace=_C.alloc_paged_decode_workspace(1, 4, 2, 128, device))
         return dict(input_ids_flat=n % 64, position_ids_flat=n - 1, kv_cache=kwargs["kv_cache"], attn_metadata=md,
                     is_prefill=False)

@@ -127,8 +127,7 @@ def test_decode_large_ragged_batch_with_empty_sequences(device):
     assert (out_tight.float().cpu() - ref).abs().max().item() <= TOL
 
 
-# (24, 8), (40, 8) and (32, 4): ratios 3, 5 and 8 (Qwen3-14B and -32B have 5 and 8) run as several
-# launches over 4, 2 and 1 query heads of every kv head.
+# Ratios 1 and 2 run on the dot-product kernel, 3, 4, 5 and 8 (Qwen3-14B and -32B have 5 and 8) in one launch on MFMA.
 GQA_HEADS = [(8, 8), (16, 8), (16, 4), (24, 8), (40, 8), (32, 4)]
 
 
@@ -292,8 +291,9 @@ def test_decode_mfma_groups(device, heads):
 @pytest.mark.gpu
 @pytest.mark.parametrize("heads,batch", [((1, 1), 3), ((2, 1), 70), ((8, 2), 5), ((8, 1), 70), ((40, 8), 9)])
 def test_decode_mfma_shared_merges_and_item_loops(device, heads, batch):
-    """Bounds past 16,384 tokens: merges of many partitions shared by the half-waves (512-token partitions below
-    64 units, 256-token ones above), and workgroups that take several items (more than 4,096 of them)."""
+    """Bounds past 16,384 tokens: merges of many partitions shared by the half-waves (512 tokens each, of two chunks
+    per wave up to 4 heads and of 8 waves past them below 64 units, else 256), and workgroups that take several items
+    (more than 4,096 of them)."""
     hq, hkv = heads
     ctx = [20000, 1, 4200] + [(37 * i) % 900 for i in range(batch - 3)]
     work = W.make_decode(batch, 0, 0, 600, seed=batch, device=device, num_heads=hq, num_kv_heads=hkv, context_lens=ctx)

@@ -181,3 +181,38 @@ def test_wide_decode_on_two_streams_at_once(device):
                 outs.append(step(kv, meta))
     torch.cuda.synchronize()
     assert all(torch.equal(o.float(), alone) for o in outs)
+
+
+@pytest.mark.gpu
+@torch.inference_mode()
+def test_wide_decode_uses_copies_that_were_built(device, monkeypatch):
+    """After build_decode_weights the wide path reads the copies, which a load rewrites."""
+    model, cache, md, ids = _model(device, 2560, 9728, 32, 4)
+
+    def step():
+        return model(input_ids_flat=ids, position_ids_flat=md.positions, kv_cache=cache, attn_metadata=md,
+                     is_prefill=False).logits.float()
+
+    rows = step()
+    model.build_decode_weights()
+    layouts = []
+    inner = _C.skinny_linear
+
+    def spy(*args, **kwargs):
+        layouts.append(kwargs.get("w_rows", False))
+        return inner(*args, **kwargs)
+
+    monkeypatch.setattr(_C, "skinny_linear", spy)
+    tiled = step()
+    torch.cuda.synchronize()
+    assert layouts and not any(layouts)
+    assert ((tiled - rows).norm() / rows.norm()).item() < 2e-2  # other K splits
+    model.init_random(4)
+    again = step()
+    other, cache2, md2, _ = _model(device, 2560, 9728, 32, 4)
+    other.init_random(4)
+    other.build_decode_weights()
+    ref = other(input_ids_flat=ids, position_ids_flat=md2.positions, kv_cache=cache2, attn_metadata=md2,
+                is_prefill=False).logits.float()
+    torch.cuda.synchronize()
+    assert torch.equal(again, ref) and not torch.equal(again, tiled)
