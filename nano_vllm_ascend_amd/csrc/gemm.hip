@@ -357,17 +357,17 @@ skinny_gemm_kernel(GemmArgs a) {
     __hip_atomic_store(a.counters + group, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Waves, 16-column tiles per wave, K slices over workgroups, 32-wide K steps per wave and round.  nw, ks and kb order a
-// row's sums.  They follow from the weight's shape, the epilogue and W's layout alone, so a row's result does not depend on
-// the rows beside it; only nt follows the row count.
+// Waves, 16-column tiles per wave, K slices over workgroups, 32-wide K steps per wave and round.  nw, ks and kb order
+// a row's sums.  They follow from the weight's shape, the epilogue and W's layout alone, so a row's result does not
+// depend on the rows beside it; only nt follows the row count.
 struct Plan {
   int nw, nt, ks, kb;
 };
 
 // Measured on MI355X with weights streamed from HBM (rotating copies, one graph), us per launch:
-//   * vocabulary-sized N (LM head), no split, 4 waves: 32 columns per workgroup up to 16 rows (151,936 x 1,024 at M = 4 51.3 against
-//     56.3 for 128 columns; 8 waves 51.7), then 64, which keep X's repeated reads down (M = 32 / 64 / 100 59.3 /
-//     72.5 / 114.6; 8 waves 58.4 / 93.5 / 157);
+//   * vocabulary-sized N (LM head), no split, 4 waves: 32 columns per workgroup up to 16 rows (151,936 x 1,024 at
+//     M = 4 51.3 against 56.3 for 128 columns; 8 waves 51.7), then 64, which keep X's repeated reads down (M = 32 /
+//     64 / 100 59.3 / 72.5 / 114.6; 8 waves 58.4 / 93.5 / 157);
 //   * residual epilogue (N = hidden: o_proj, down_proj): 32 columns (the epilogue's sums of
 //     squares cover whole 32-column groups) per 8-wave workgroup, K split over >= 128
 //     workgroups (at N = 1,024, K = 2,048 / 3,072 o 6.5, down 6.6; unsplit 16-wave workgroups 8.2).  A long K
@@ -376,17 +376,17 @@ struct Plan {
 //     2,048 x 6,144 9.0 / 9.5 / 12.1 / 15.4 against 11.7 / 12.9 / 15.0 / 14.7, 2,560 x 9,728 14.0 / 15.0 / 21.6 / 30.2
 //     against 15.7 / 18.8 / 21.9 / 32.4, 4,096 x 12,288 22.6 / 23.8 / 30.7 / 47.4 against 30.3 / 35.2 / 43.8 / 40.9,
 //     5,120 x 17,408 35.8 / 39.0 / 56.9 / 82.6 against 41.8 / 51.3 / 62.4 / 95.8);
-//   * gate_up: 16 columns per 8-wave workgroup, 32 above 64 rows; 32 from N = 4,096 on (6,144 x 2,048 normed at M = 32: 13.8 against
-//     17.3); from N = 8,192 on 4 waves, 16 columns up to 32 rows and 32 above (12,288 x 4,096 at M = 32 / 100: 40.4 /
-//     61.7 against 42.3 / 67.0 of 8 waves);
+//   * gate_up: 16 columns per 8-wave workgroup, 32 above 64 rows; 32 from N = 4,096 on (6,144 x 2,048 normed at
+//     M = 32: 13.8 against 17.3); from N = 8,192 on 4 waves, 16 columns up to 32 rows and 32 above (12,288 x 4,096 at
+//     M = 32 / 100: 40.4 / 61.7 against 42.3 / 67.0 of 8 waves);
 //   * otherwise (qkv): 16 columns per 8-wave workgroup, 32 from N = 6,144 on (6,144 x 4,096 at M = 8 / 32: 11.4 / 13.5
 //     against 13.6 / 17.5) and above 64 rows, halving the X reads per weight byte (4,096 x 2,048 normed at
 //     M = 100: 14.8 against 20.3);
-//   * row-major W (W_ROWS; 16 rows x 64 bytes per load instruction), M = 8 / 32: gate_up from N = 8,192 on 256 bytes of a row per wave
-//     and round (12,288 x 4,096 41.6 / 45.9 against 44.5 / 48.1 with 128 bytes, 9,728 x 2,560 26.4 / 31.2 against
-//     28.1 / 31.7); residual projections 4 waves, split to >= 512 workgroups of >= 512 K (4,096 x 4,096 12.0 / 12.6 against
-//     13.5 / 15.9 unsplit of 8 waves, 2,560 x 9,728 14.9 / 18.0 against 16.6 / 20.5 at 160 of 8, 5,120 x 17,408 45.8 / 54.5
-//     against 54.4 / 63.9 unsplit); others as tiled.
+//   * row-major W (W_ROWS; 16 rows x 64 bytes per load instruction), M = 8 / 32: gate_up from N = 8,192 on 256 bytes
+//     of a row per wave and round (12,288 x 4,096 41.6 / 45.9 against 44.5 / 48.1 with 128 bytes, 9,728 x 2,560 26.4 /
+//     31.2 against 28.1 / 31.7); residual projections 4 waves, split to >= 512 workgroups of >= 512 K (4,096 x 4,096
+//     12.0 / 12.6 against 13.5 / 15.9 unsplit of 8 waves, 2,560 x 9,728 14.9 / 18.0 against 16.6 / 20.5 at 160 of 8,
+//     5,120 x 17,408 45.8 / 54.5 against 54.4 / 63.9 unsplit); others as tiled.
 Plan make_plan(int n, int k, int epi, int m, bool w_rows) {
   const int kb = k % 512 == 0 ? 2 : 1;
   if (epi == kEpiResid) {

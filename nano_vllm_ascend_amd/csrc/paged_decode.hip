@@ -658,11 +658,12 @@ int launch(DecodeArgs a, int batch, hipStream_t stream) {
 }
 
 // ------------------------------------------------------------------------------------------
-// MFMA variant, for up to 8 query heads of a group: groups of 3 and more, and those of 1 and 2 under bounds past 16,384
-// tokens.
+// MFMA variant, for up to 8 query heads of a group: groups of 3 and more, and those of 1 and 2 under bounds that the
+// dot-product kernel does not take (dispatch_gqa).
 //
 // The same split-KV items, scan, records and arrival counting as above, for up to GP query heads of
-// a kv head in one launch, so K and V are read once up to a ratio of 8.  A chunk of 64 tokens, of which a wave takes CPW:
+// a kv head in one launch, so K and V are read once up to a ratio of 8.  A chunk of 64 tokens, of which a wave
+// takes CPW:
 //   S^T = K . Q^T by v_mfma_f32_16x16x32_bf16 with A = rows of K as read from the cache.  The operand's
 //        16 rows x 32 dims give a load only 64 consecutive bytes of a cache row, and K read that way
 //        took 1.07-1.15x the launch's time.  So 8 row slots take dims 0..31 of a 64-dim half and the other 8 (z = 1)
@@ -677,9 +678,10 @@ int launch(DecodeArgs a, int batch, hipStream_t stream) {
 //        movement: its k-slots are taken in the order the S^T accumulators hold the tokens.
 // Tiles and rows past the wave's range lie past the tile's buffer range: they read zeros without a
 // memory access, whatever bits an unwritten row of the cache holds.  The row is part of the vector offset, which
-// the range check covers; it does not cover a scalar offset.  Bound by the K/V stream, as the kernel above: a group of 8 over 16 x U[512, 4096] takes 28.8 us
-// (4.4 TB/s) where two launches over 4 heads took 63.5 us, and 100 x U[2048, 4096] 232 us (5.3 TB/s) against
-// 458; what is left over the dot-product kernel's 5.8 TB/s at 2 heads is the records' traffic.
+// the range check covers; it does not cover a scalar offset.  Bound by the K/V stream, as the kernel above: a group of
+// 8 over 16 x U[512, 4096] takes 28.3 us (4.5 TB/s) where two launches over 4 heads took 63.3 us, and 100 x U[2048,
+// 4096] 232 us (5.3 TB/s) against 459; what is left over the dot-product kernel's 5.8 TB/s at 2 heads is mostly the
+// records' traffic (8% of the bytes).
 __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8v, a), __builtin_bit_cast(bf16x8v, b), c, 0,
                                                  0, 0);
@@ -828,7 +830,8 @@ __device__ __forceinline__ bool mfma_item(const DecodeArgs &a, const int tid, co
       }
     };
     const bool nr_in = nr >= 0 && nr < ctx;
-    const bool owner = a.store_new && (nr_in ? (nr >= p * PART && nr < (p + 1) * PART && (int)(nr >> 6) % NW == w) : (p == n_parts - 1 && w == 0));
+    const bool in_chunk = nr >= p * PART && nr < (p + 1) * PART && (int)(nr >> 6) % NW == w;
+    const bool owner = a.store_new && (nr_in ? in_chunk : (p == n_parts - 1 && w == 0));
     const u16 *qp = a.q + (int64_t)b * a.q_stride + (int64_t)(head0 + min(r, G - 1)) * D + 8 * c;
     qr[0] = ld16(qp);
     qr[1] = ld16(qp + 64);
@@ -1393,14 +1396,15 @@ int fill_decode_args(DecodeArgs &a, void *out, int64_t out_stride, const void *q
 // Groups of 1 and 2 heads keep the dot-product kernel, which is as fast over large batches and faster
 // where latency counts (at 2 heads 33.6 against 33.9 us over 32 x U[256, 2304], 6.6 against 7.1 us over 4 x U[1, 512]; at 4
 // heads the MFMA variant leads: 35.7 against 36.5 us and 7.2 against 9.6 us), up to the 64 partitions that its merge
-// holds: 256 tokens each, and 512 of two chunks per wave under bounds past 16,384, there up to 8,192 workgroups (at 20,480,
-// dot product / MFMA: 16 / 8 heads 28.0 / 29.6 us over 16 x U[1250, 2500], 8.9 / 9.9 over 4 x U[1, 512]; 8 / 8 8.6 / 10.2 over the
-// latter; 2 / 1 10.4 / 12.1 over 16 x U[1250, 2500]).  More of them are mostly empty ones, which the MFMA variant's item
-// loop saves (16 / 8 heads over 100 x U[300, 600] at 20,480 60 / 44 us, 100 x U[1250, 2500] at 32,768 167 / 138).  Past
-// 32,768 tokens the dot-product kernel would need 1,024-token partitions, whose few workgroups lose to the MFMA variant where
-// contexts are short for the bound (at 40,960: 2 x U[1250, 2500] at 16 / 8 16.8 / 12.4, 100 x U[300, 600] 58.2 / 45.9, 100 x
-// U[1250, 2500] 150 / 133) and lead it where they are long for the batch (2 x U[8000, 16000] at 16 / 8 20.2 / 21.9, 8 x the
-// same at 8 / 8 78.3 / 81.4, 100 x U[1250, 2500] at 2 / 1 19.6 / 22.1); the host cannot tell these apart.
+// holds: 256 tokens each, and 512 of two chunks per wave under bounds past 16,384, there up to 8,192 workgroups (at
+// 20,480, dot product / MFMA: 16 / 8 heads 28.0 / 29.6 us over 16 x U[1250, 2500], 8.9 / 9.9 over 4 x U[1, 512]; 8 / 8
+// 8.6 / 10.2 over the latter; 2 / 1 10.4 / 12.1 over 16 x U[1250, 2500]).  More of them are mostly empty ones, which the
+// MFMA variant's item loop saves (16 / 8 heads over 100 x U[300, 600] at 20,480 60 / 46 us, 100 x U[1250, 2500] at
+// 32,768 167 / 133).  Past 32,768 tokens the dot-product kernel would need 1,024-token partitions, whose few workgroups
+// lose to the MFMA variant where contexts are short for the bound (at 40,960: 2 x U[1250, 2500] at 16 / 8 16.8 / 12.4,
+// 100 x U[300, 600] 58.2 / 45.9, 100 x U[1250, 2500] 150 / 133) and lead it where they are long for the batch (2 x
+// U[8000, 16000] at 16 / 8 20.2 / 21.9, 8 x the same at 8 / 8 78.3 / 81.4, 100 x U[1250, 2500] at 2 / 1 19.6 / 22.1);
+// the host cannot tell these apart.
 template <bool FUSED>
 int dispatch_gqa(DecodeArgs a, int gqa, int batch, hipStream_t stream) {
   a.q_group = gqa;
