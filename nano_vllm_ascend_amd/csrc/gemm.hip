@@ -376,8 +376,9 @@ struct Plan {
 //     2,048 x 6,144 9.0 / 9.5 / 12.1 / 15.4 against 11.7 / 12.9 / 15.0 / 14.7, 2,560 x 9,728 14.0 / 15.0 / 21.6 / 30.2
 //     against 15.7 / 18.8 / 21.9 / 32.4, 4,096 x 12,288 22.6 / 23.8 / 30.7 / 47.4 against 30.3 / 35.2 / 43.8 / 40.9,
 //     5,120 x 17,408 35.8 / 39.0 / 56.9 / 82.6 against 41.8 / 51.3 / 62.4 / 95.8);
-//   * gate_up: 16 columns per 8-wave workgroup, 32 above 64 rows; 32 from N = 4,096 on (6,144 x 2,048 normed at
-//     M = 32: 13.8 against 17.3); from N = 8,192 on 4 waves, 16 columns up to 32 rows and 32 above (12,288 x 4,096 at
+//   * gate_up: 16 columns per 8-wave workgroup, 32 above 64 rows, and 32 where 16 would give more than one workgroup
+//     per CU (N > 4,096; at M = 32 6,144 x 2,048 normed 13.8 against 17.3, 4,352 x 4,096 22.8 against 24.1, but 4,096 x
+//     512 5.1 against 4.5 and 4,096 x 2,048 13.1 against 11.3); from N = 8,192 on 4 waves, 16 columns up to 32 rows and 32 above (12,288 x 4,096 at
 //     M = 32 / 100: 40.4 / 61.7 against 42.3 / 67.0 of 8 waves);
 //   * otherwise (qkv): 16 columns per 8-wave workgroup, 32 from N = 6,144 on (6,144 x 4,096 at M = 8 / 32: 11.4 / 13.5
 //     against 13.6 / 17.5) and above 64 rows, halving the X reads per weight byte (4,096 x 2,048 normed at
@@ -412,7 +413,7 @@ Plan make_plan(int n, int k, int epi, int m, bool w_rows) {
   }
   if (epi == kEpiSilu) {
     if (n >= 8192) return {4, m > 32 ? 2 : 1, 1, w_rows ? 4 : 2};
-    return {8, m > 64 || n >= 4096 ? 2 : 1, 1, kb};
+    return {8, m > 64 || n > 4096 ? 2 : 1, 1, kb};
   }
   if (n % 128 == 0 && n / 128 >= 512) return {4, m <= 16 ? 2 : 4, 1, 2};
   return {8, m > 64 || n >= 6144 ? 2 : 1, 1, kb};
